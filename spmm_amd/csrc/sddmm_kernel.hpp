@@ -14,45 +14,188 @@
 
 namespace tca {
 
-constexpr int kSddmmRowsPerBlock = 4;  // one wavefront per row
-constexpr int kSddmmCols = 8;          // columns per lane per chunk (chunk = 512 columns)
+constexpr int kSddmmWaves = 4;          // wavefronts per workgroup (independent spans)
+constexpr uint32_t kSddmmFill = 16384;  // wavefronts a launch is split into before spans grow
+constexpr uint32_t kSddmmMaxBatches = 16;
 
-// out[j] = sum_n G[r, n] * B[colidx[j], n] for the nonzeros j of row r.  The
-// row of G is held in registers chunk by chunk; each nonzero's partial sums
-// are reduced across the wavefront with xor shuffles in a fixed order and
-// chunks are added in column order, so the result does not depend on the
-// schedule.
-template <typename T>
-__global__ __launch_bounds__(64 * kSddmmRowsPerBlock) void sddmm_kernel(const int* __restrict__ rowptr,
-                                                                        const int* __restrict__ colidx, int M, int N,
-                                                                        const float* __restrict__ G,
-                                                                        const T* __restrict__ B,
-                                                                        float* __restrict__ out) {
+struct SddmmArgs {
+    const int* rowptr;
+    const int* colidx;
+    const float* G;
+    const void* B;
+    float* out;
+    int M, N;
+    uint32_t nnz;
+    uint32_t batches;  // 64-nonzero batches per wavefront
+};
+
+// E elements of T at element alignment (one load; rows of any width and bases
+// at any element stay on the vector path).
+template <typename T, int E>
+__device__ __forceinline__ Pack<T, E> load_elems(const T* p) {
+    struct __attribute__((packed, aligned(sizeof(T)))) U {
+        T v[E];
+    };
+    return __builtin_bit_cast(Pack<T, E>, *reinterpret_cast<const U*>(p));
+}
+
+// Partner's value within 8 lanes: 7 - lane, lane ^ 2, lane ^ 1.
+template <int kCtrl>
+__device__ __forceinline__ float dpp_swap(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), kCtrl, 0xf, 0xf, true));
+}
+
+// The row of nonzero j: the last r in [lo, hi] with rowptr[r] <= j.
+__device__ __forceinline__ int row_of(const int* __restrict__ rowptr, uint32_t j, int lo, int hi) {
+    while (lo < hi) {
+        const int mid = lo + (hi - lo + 1) / 2;
+        if (static_cast<uint32_t>(rowptr[mid]) <= j) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// The same for one j per wavefront, 64 probes a step (M = 2^18: three dependent loads).
+__device__ __forceinline__ int wave_row_of(const int* __restrict__ rowptr, uint32_t j, int M, int lane) {
+    int lo = 0, n = M;  // the row is in [lo, lo + n)
+    while (n > 1) {
+        const int step = (n + 63) / 64;
+        const int r = lo + lane * step;
+        const bool le = lane * step < n && static_cast<uint32_t>(rowptr[r]) <= j;
+        const int c = __popcll(__ballot(le));  // >= 1: rowptr[lo] <= j
+        const int at = (c - 1) * step;
+        n = min(step, n - at);
+        lo += at;
+    }
+    return lo;
+}
+
+// out[j] = sum_n G[row(j), n] * B[colidx[j], n] for every nonzero j.
+//
+// Bound: gathering a row of B per nonzero (L2 -> CU).  The nonzeros are split
+// evenly whatever their rows (a wavefront owns `batches` runs of 64; the rows
+// at the ends of its span are searched in rowptr), so a power-law graph's
+// longest row is spread over the chip.  A batch goes to 64 / L slots of L
+// lanes, L nonzeros each; lane l of a slot reads 16-byte pieces l, l + L, ...
+// of the L rows of B, L loads in flight per piece column, and the L partial
+// sums per lane are exchanged and added in log2 L DPP steps (a reduce-scatter:
+// L - 1 adds for L nonzeros) that leave lane i of the wavefront with nonzero
+// i's sum, stored coalesced.  A slot whose nonzeros share a row reads that row
+// of G once per piece (the wavefront takes this path when all its slots do),
+// otherwise once per nonzero, mostly from the L1.  Sums run in a fixed order:
+// a piece in fp32 (chains of four), a lane's pieces in fp64 (a lane adds up
+// to N / 8 products, which in fp32 would round more often than the 64-lane
+// tree that this replaced), the lanes of a slot in fp32.
+//
+// One wavefront per row with one nonzero at a time and a six-step shuffle sum
+// per nonzero (the previous kernel): 25.2 ms on 11.4M nonzeros of an R-MAT
+// graph of 131,072 nodes at N = 128 fp32, 650 us on a 2048 x 2048 layer of
+// 10 % at N = 1024 bf16; now 0.60 ms and 63 us (9.7 and 13.6 TB/s of gathered
+// rows of B).
+template <typename T, int E, int L>
+__global__ __launch_bounds__(64 * kSddmmWaves, 4) void sddmm_kernel(SddmmArgs a) {
     const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * kSddmmRowsPerBlock + (threadIdx.x >> 6);
-    if (r >= M) return;
-    const int j0 = rowptr[r], j1 = rowptr[r + 1];
-    if (j0 == j1) return;
-    const float* g_row = G + static_cast<size_t>(r) * N;
-    for (int n0 = 0; n0 < N; n0 += 64 * kSddmmCols) {
-        float g[kSddmmCols];
+    const uint32_t wave = blockIdx.x * kSddmmWaves + (threadIdx.x >> 6);
+    const uint32_t span = 64 * a.batches;
+    const uint32_t j0 = wave * span;
+    if (j0 >= a.nnz) return;
+    const uint32_t j1 = min(j0 + span, a.nnz);
+    const int r0 = wave_row_of(a.rowptr, j0, a.M, lane);
+    const int r1 = wave_row_of(a.rowptr, j1 - 1, a.M, lane);
+    const size_t N = static_cast<size_t>(a.N);
+    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
+    const int l = lane & (L - 1), first = lane - l;
+    const int V = (a.N + E - 1) / E;      // pieces of a row
+    const int full = a.N / (E * L) * L;   // pieces of whole piece columns
+    int lo = r0;
+    for (uint32_t jb = j0; jb < j1; jb += 64) {
+        const uint32_t j = min(jb + lane, j1 - 1);
+        const int mycol = a.colidx[j];
+        const int myrow = row_of(a.rowptr, j, lo, r1);
+        lo = __builtin_amdgcn_readlane(myrow, 63);
+        uint32_t brow[L];  // byte offsets of the rows of B (a plan's B is below 4 GiB)
+        int grow[L];
 #pragma unroll
-        for (int q = 0; q < kSddmmCols; q++) {
-            const int c = n0 + 64 * q + lane;
-            g[q] = c < N ? g_row[c] : 0.f;
+        for (int u = 0; u < L; u++) {
+            brow[u] = static_cast<uint32_t>(__shfl(mycol, first + u)) * rowbytes;
+            grow[u] = __shfl(myrow, first + u);
         }
-        for (int j = j0; j < j1; j++) {
-            const T* b_row = B + static_cast<size_t>(colidx[j]) * N;
-            float s = 0.f;
+        const bool one_row = __ballot(grow[0] != grow[L - 1]) == 0;  // rows ascend within a slot
+        double acc[L];
 #pragma unroll
-            for (int q = 0; q < kSddmmCols; q++) {
-                const int c = n0 + 64 * q + lane;
-                if (c < N) s += g[q] * to_f32(b_row[c]);
+        for (int u = 0; u < L; u++) acc[u] = 0.;
+        auto add = [&](int u, const Pack<float, E>& g, const Pack<T, E>& b, int skip) {
+            float t[(E + 3) / 4];
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                float s = e % 4 == 0 ? g.v[e] * to_f32(b.v[e]) : __builtin_fmaf(g.v[e], to_f32(b.v[e]), t[e / 4]);
+                if (skip > e) s = 0.f;
+                t[e / 4] = s;
             }
+            acc[u] += static_cast<double>(E == 8 ? t[0] + t[E / 8] : t[0]);
+        };
+        auto load_b = [&](int u, int at) {
+            return load_elems<T, E>(reinterpret_cast<const T*>(static_cast<const char*>(a.B) +
+                                                               (brow[u] + static_cast<uint32_t>(at) * sizeof(T))));
+        };
+        auto load_g = [&](int u, int at) { return load_elems<float, E>(a.G + static_cast<size_t>(grow[u]) * N + at); };
+        auto piece = [&](int at, int skip) {  // columns [at, at + E), the first `skip` of them not counted
+            Pack<T, E> b[L];
+            const Pack<float, E> g = load_g(0, at);
 #pragma unroll
-            for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d, 64);
-            if (lane == 0) out[j] = n0 == 0 ? s : out[j] + s;
+            for (int u = 0; u < L; u++) b[u] = load_b(u, at);
+#pragma unroll
+            for (int u = 0; u < L; u++) add(u, g, b[u], skip);
+        };
+        auto piece_rows = [&](int at, int skip) {  // the same, every nonzero with its own row of G
+            constexpr int H = L > 4 ? 4 : L;       // nonzeros loaded at a time (registers)
+#pragma unroll
+            for (int h = 0; h < L; h += H) {
+                Pack<T, E> b[H];
+                Pack<float, E> g[H];
+#pragma unroll
+                for (int u = 0; u < H; u++) {
+                    g[u] = load_g(h + u, at);
+                    b[u] = load_b(h + u, at);
+                }
+#pragma unroll
+                for (int u = 0; u < H; u++) add(h + u, g[u], b[u], skip);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        const int tail = full + l;  // the last piece of a row that is no whole number of them ends at the row's end
+        const int at = min(tail * E, a.N - E);
+        if (one_row) {
+#pragma unroll(E == 8 ? 1 : 2)
+            for (int p = 0; p < full; p += L) piece((p + l) * E, 0);
+            if (tail < V) piece(at, tail * E - at);
+        } else {
+#pragma unroll 1
+            for (int p = 0; p < full; p += L) piece_rows((p + l) * E, 0);
+            if (tail < V) piece_rows(at, tail * E - at);
         }
+        float sum[L];
+#pragma unroll
+        for (int u = 0; u < L; u++) sum[u] = static_cast<float>(acc[u]);
+        if constexpr (L == 8) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const float give = l & 4 ? sum[u] : sum[u + 4], keep = l & 4 ? sum[u + 4] : sum[u];
+                sum[u] = keep + dpp_swap<0x141>(give);  // row_half_mirror
+            }
+        }
+        if constexpr (L >= 4) {
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const float give = l & 2 ? sum[u] : sum[u + 2], keep = l & 2 ? sum[u + 2] : sum[u];
+                sum[u] = keep + dpp_swap<0x4e>(give);  // quad_perm [2, 3, 0, 1]
+            }
+        }
+        if constexpr (L >= 2) {
+            const float give = l & 1 ? sum[0] : sum[1], keep = l & 1 ? sum[1] : sum[0];
+            sum[0] = keep + dpp_swap<0xb1>(give);  // quad_perm [1, 0, 3, 2]
+        }
+        if (jb + lane < j1) a.out[jb + lane] = sum[0];
     }
 }
 

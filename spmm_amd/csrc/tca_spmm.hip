@@ -458,6 +458,25 @@ int launch_panels(const tca_spmm_plan* p, const void* val, const void* B, float*
     }
 }
 
+// Pieces of 16 bytes (single columns when a row holds less), L lanes per nonzero: as many as a row has pieces, up to 8.
+template <typename T, int E>
+void launch_sddmm_e(const SddmmArgs& a, hipStream_t s) {
+    const uint64_t span = 64ull * a.batches * kSddmmWaves;
+    const dim3 grid(static_cast<unsigned>((a.nnz + span - 1) / span)), block(64 * kSddmmWaves);
+    const int V = (a.N + E - 1) / E;
+    if (V > 4) hipLaunchKernelGGL((sddmm_kernel<T, E, 8>), grid, block, 0, s, a);
+    else if (V > 2) hipLaunchKernelGGL((sddmm_kernel<T, E, 4>), grid, block, 0, s, a);
+    else if (V > 1) hipLaunchKernelGGL((sddmm_kernel<T, E, 2>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((sddmm_kernel<T, E, 1>), grid, block, 0, s, a);
+}
+
+template <typename T>
+void launch_sddmm(const SddmmArgs& a, hipStream_t s) {
+    constexpr int E = 16 / sizeof(T);
+    if (a.N >= E) launch_sddmm_e<T, E>(a, s);
+    else launch_sddmm_e<T, 1>(a, s);
+}
+
 // Bit 1 << TCA_PHASE_* for each phase in which the plan launches a kernel.
 uint32_t phases_used(const tca_spmm_plan* p) {
     uint32_t m = 0;
@@ -1899,19 +1918,20 @@ int tca_sddmm(const tca_spmm_plan* p, const float* d_G, const void* d_B, float* 
     if (p->M == 0 || p->nnz == 0) return TCA_OK;
     if (!d_G || !d_B || !d_out) return fail(TCA_ERR_INVALID, "NULL device pointer");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid((p->M + kSddmmRowsPerBlock - 1) / kSddmmRowsPerBlock), block(64 * kSddmmRowsPerBlock);
+    SddmmArgs a;
+    a.rowptr = p->d_rowptr;
+    a.colidx = p->d_colidx;
+    a.G = d_G;
+    a.B = d_B;
+    a.out = d_out;
+    a.M = p->M;
+    a.N = p->N;
+    a.nnz = static_cast<uint32_t>(p->nnz);
+    a.batches = std::min(std::max(a.nnz / (64 * kSddmmFill), 1u), kSddmmMaxBatches);
     switch (p->dtype) {
-        case TCA_F16:
-            hipLaunchKernelGGL(sddmm_kernel<_Float16>, grid, block, 0, s, p->d_rowptr, p->d_colidx, p->M, p->N, d_G,
-                               static_cast<const _Float16*>(d_B), d_out);
-            break;
-        case TCA_BF16:
-            hipLaunchKernelGGL(sddmm_kernel<bf16_t>, grid, block, 0, s, p->d_rowptr, p->d_colidx, p->M, p->N, d_G,
-                               static_cast<const bf16_t*>(d_B), d_out);
-            break;
-        default:
-            hipLaunchKernelGGL(sddmm_kernel<float>, grid, block, 0, s, p->d_rowptr, p->d_colidx, p->M, p->N, d_G,
-                               static_cast<const float*>(d_B), d_out);
+        case TCA_F16: launch_sddmm<_Float16>(a, s); break;
+        case TCA_BF16: launch_sddmm<bf16_t>(a, s); break;
+        default: launch_sddmm<float>(a, s);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(TCA_ERR_HIP, "kernel launch: %s", hipGetErrorString(e));
