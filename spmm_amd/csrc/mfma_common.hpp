@@ -109,10 +109,110 @@ __host__ __device__ constexpr int bswz64(int r) { return 2 * (((r >> 1) & 1) | (
 __device__ __forceinline__ void dma_x4(const void* g, uint32_t m0) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "{m0}"(m0) : "memory");
 }
+// The same with a wavefront-uniform base and a 32-bit offset per lane; and 4
+// bytes per lane (to m0 + 4 * lane).
+__device__ __forceinline__ void dma_x4(const void* base, uint32_t off, uint32_t m0) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "{m0}"(m0) : "memory");
+}
+__device__ __forceinline__ void dma_x1(const void* g, uint32_t m0) {
+    asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "{m0}"(m0) : "memory");
+}
+// A wavefront's LDS reads have returned: their slot may be written again.
+__device__ __forceinline__ void wait_lds_reads() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     static_assert(N >= 0 && N <= 63, "vmcnt range");
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Source of the B rows past K and columns past N of a transfer.
+static __device__ const int4 kZeroPiece = {0, 0, 0, 0};
+
+// Issues the transfers of 32 * H rows x 64 columns of B (row-major, N columns,
+// rows r0 .., columns c0 ..) into LDS byte address `lds`: H tiles of 32 rows of
+// 128 bytes, 16-byte pieces permuted by bswz64.  4 H transfers of 8 rows.
+template <int H>
+struct BTile {
+    const char* base;     // B + c0
+    uint32_t rowbytes;
+    uint32_t off[2];      // lane's offset within 8 rows, even and odd transfers
+    bool ok[2];           // lane's piece lies within the columns of B
+    bool all;             // every piece does
+    int K, row;           // rows of B; lane's row within 8
+
+    __device__ __forceinline__ void init(const void* B, int K_, int N, int c0, int lane) {
+        rowbytes = static_cast<uint32_t>(N) * 2u;
+        base = static_cast<const char*>(B) + static_cast<size_t>(c0) * 2;
+        K = K_;
+        row = lane >> 3;
+        all = c0 + 64 <= N;
+#pragma unroll
+        for (int odd = 0; odd < 2; odd++) {
+            const int piece = (lane & 7) ^ bswz64(8 * odd + row);
+            off[odd] = static_cast<uint32_t>(row) * rowbytes + 16u * piece;
+            ok[odd] = c0 + 8 * piece < N;
+        }
+    }
+    __device__ __forceinline__ void issue(int r0, uint32_t lds) const {
+        if (all && r0 + 32 * H <= K) {  // wavefront-uniform
+            const char* src = base + static_cast<size_t>(r0) * rowbytes;
+#pragma unroll
+            for (int t = 0; t < 4 * H; t++) {
+                dma_x4(src, off[t & 1], lds + 1024u * t);
+                src += 8 * static_cast<size_t>(rowbytes);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4 * H; t++) {
+                const int r = r0 + 8 * t;
+                const bool in = ok[t & 1] && r + row < K;
+                const char* src = base + static_cast<size_t>(r) * rowbytes + off[t & 1];
+                dma_x4(in ? static_cast<const void*>(src) : static_cast<const void*>(&kZeroPiece), lds + 1024u * t);
+            }
+        }
+    }
+};
+
+// The B operand of column block c (16 columns) of one 32 x 64 tile in that layout.
+__device__ __forceinline__ i32x4v b_fragment(const uint16_t* tile, int c, int lane) {
+    const int li = lane & 15, lh = lane >> 4;
+    const int br = 8 * lh + (li >> 2);
+    const uint16_t* p = tile + br * kDmaBRow + 4 * (li & 1) + 8 * ((2 * c + ((li & 3) >> 1)) ^ bswz64(br));
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p));
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p + 4 * kDmaBRow));
+    return i32x4v{__builtin_bit_cast(int, __builtin_shufflevector(lo, lo, 0, 1)),
+                  __builtin_bit_cast(int, __builtin_shufflevector(lo, lo, 2, 3)),
+                  __builtin_bit_cast(int, __builtin_shufflevector(hi, hi, 0, 1)),
+                  __builtin_bit_cast(int, __builtin_shufflevector(hi, hi, 2, 3))};
+}
+
+// The W wavefronts of a workgroup hold partial sums of the same RB x CB blocks
+// of 16 x 16 (W split the contraction): they meet in LDS (1 KiB per block and
+// wavefront, reusing the rings), each wavefront adds its share of the blocks
+// in wavefront order and stores them.  Every wavefront of the workgroup calls it.
+template <int RB, int CB, int W>
+__device__ __forceinline__ void reduce_store(const f32x4 (&acc)[RB][CB], void* lds, int wave, int lane, int row0, int c0,
+                                             int M, int N, float* C) {
+    f32x4* const part = static_cast<f32x4*>(lds);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RB; r++)
+#pragma unroll
+        for (int c = 0; c < CB; c++) part[(wave * RB * CB + r * CB + c) * 64 + lane] = acc[r][c];
+    __syncthreads();
+    for (int b = wave; b < RB * CB; b += W) {
+        f32x4 s = part[b * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < W; w++) s += part[(w * RB * CB + b) * 64 + lane];
+        const int col = c0 + 16 * (b % CB) + (lane & 15);
+        const int row = row0 + 16 * (b / CB) + 4 * (lane >> 4);
+        if (col < N) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (row + i < M) __builtin_nontemporal_store(s[i], C + static_cast<size_t>(row + i) * N + col);
+        }
+    }
 }
 
 template <typename P>

@@ -16,14 +16,26 @@
 //     rows 32 + 8 g .. + 7 in halves 8..15: two fragments of the dense
 //     v_mfma_f32_16x16x32 B operand, one per 32-row half of the 64-row step;
 //   * D: as the dense 16x16 MFMA (lane l: column l % 16, rows 4 (l / 16) + r).
-// A workgroup owns 64 rows and 256 columns of C; wavefront w owns columns
-// 64 w .. 64 w + 63 (4 row blocks x 4 column blocks).  Per K step of 64:
-// B rows (64 x 256) are staged in LDS, double-buffered, in the layout of the
-// Blocked-ELL kernel (two 32-row halves, bswz64-permuted 128-byte rows, read
-// with ds_read_b64_tr_b16); A's compressed fragment (16 bytes per lane) and
-// meta word come straight from global memory one step ahead.  Steps are
-// added in order (deterministic).  B rows past K load as zeros; rows past M
-// read row M - 1 and are not stored.
+//
+// A workgroup owns 16 RB rows and 64 columns of C.  Its W wavefronts split K,
+// each a contiguous range of it, and meet once at the end (reduce_store), so
+// the loop has no barrier: a wavefront fills LDS of its own with global -> LDS
+// transfers of the next two 64-deep steps (128 rows of B, the compressed A
+// pieces, every fourth time a window of index words) as soon as it has read
+// the last two into registers, and multiplies those meanwhile.
+//
+// What bounds it is lines from the L2 to the CU, about 4 cycles per 128-byte
+// line and CU however much of the line is used.  Hence two steps at a time (a
+// row of A is then one whole line; one step at a time reads half lines) and
+// index words by windows of 64 bytes per row (one step's are 8 bytes): with
+// one step and its index words at a time, rings up to three slots deep, a
+// 4096 x 4096 bf16 product took 40 us at N = 512 whatever the depth, now 22.1
+// (97.7 with 64 x 256 tiles of four wavefronts staging B through registers,
+// one step ahead, on 128 of the 256 CUs).
+//
+// B rows past K, columns past N and A past Kp come from a zero piece; rows
+// past M read row M - 1 and are not stored.  Index words lie at any 2-byte
+// address: the window starts at the aligned dword at or before its first.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -36,148 +48,151 @@ namespace tca {
 typedef _Float16 f16x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kS24Threads = 256;  // 4 wavefronts
-constexpr int kS24Cols = 256;     // columns of C per workgroup
-constexpr int kS24Rows = 64;      // rows of C per workgroup
+constexpr int kS24Cols = 64;  // columns of C per workgroup
 
 struct S24Args {
     const void* vals;       // [M][Kp / 2]
     const uint16_t* meta;   // [M][Kp / 16]
     const void* B;          // K x N row-major
     float* C;               // M x N row-major
-    int M, N, Kp;
-    int col_groups;         // blockIdx.x = row group * col_groups + column group
-    uint32_t B_bytes;       // K * N * 2
+    int M, N, K, Kp;
+    int row_groups, col_groups;
 };
 
-template <bool kBf16>
-__global__ __launch_bounds__(kS24Threads) void sparse24_kernel(S24Args a) {
-    constexpr int KROWS = 64;                 // B rows per step
-    constexpr int PIECES = KROWS / 8;         // 16-byte B pieces per thread and step
-    constexpr int kTile = KROWS * kS24Cols;   // halves of one staged B tile
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][kTile];
+// Workgroup -> tile: workgroup b runs on XCD b % 8; the column groups of one
+// row group follow each other on one XCD, whose L2 then fetches the row
+// group's A once.
+__device__ __forceinline__ void s24_tile(int b, int row_groups, int col_groups, int& rg, int& cg) {
+    const int q = row_groups / 8 * 8 * col_groups;  // workgroups of whole eights of row groups
+    if (b < q) {
+        rg = b / (8 * col_groups) * 8 + b % 8;
+        cg = b / 8 % col_groups;
+    } else {
+        rg = row_groups / 8 * 8 + (b - q) / col_groups;
+        cg = (b - q) % col_groups;
+    }
+}
 
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int row0 = (blockIdx.x / a.col_groups) * kS24Rows;
-    const int c0 = (blockIdx.x % a.col_groups) * kS24Cols;
+// LDS of a wavefront: two steps' B tiles (16 KiB), A pieces (2 KiB per row
+// block) and a window of index words (1 KiB per row block).
+template <int RB>
+constexpr int s24_wave_bytes() {
+    return 16384 + RB * 3072;
+}
+template <int RB, int W>
+constexpr int s24_lds_bytes() {
+    return W * s24_wave_bytes<RB>() > W * RB * 4096 ? W * s24_wave_bytes<RB>() : W * RB * 4096;
+}
+
+template <bool kBf16, int RB, int W>
+__global__ __launch_bounds__(64 * W) void sparse24_kernel(S24Args a) {
+    __shared__ __attribute__((aligned(16))) char lds[s24_lds_bytes<RB, W>()];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int rg, cg;
+    s24_tile(blockIdx.x, a.row_groups, a.col_groups, rg, cg);
+    const int row0 = rg * 16 * RB, c0 = cg * kS24Cols;
     const int steps = a.Kp / 64;
-    const int vcols = a.Kp / 2, mcols = a.Kp / 16;
-    const __amdgpu_buffer_rsrc_t rB = make_rsrc(a.B, a.B_bytes);
-    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * 2u;
-    const uint16_t* const V = static_cast<const uint16_t*>(a.vals);
+    const int pairs = (steps + 1) / 2;  // the second step of the last pair may be missing
+    const int p0 = static_cast<int>(static_cast<int64_t>(pairs) * wave / W);
+    const int p1 = static_cast<int>(static_cast<int64_t>(pairs) * (wave + 1) / W);
+    char* const mem = lds + wave * s24_wave_bytes<RB>();
+    const uint32_t mem_at = lds_addr(mem);
 
-    auto load_b = [&](int s, i32x4v* bv) {
+    BTile<4> bt;
+    bt.init(a.B, a.K, a.N, c0, lane);
+    // A: transfer q of row block rb holds its rows 8 q + lane / 8, 16-byte
+    // piece (lane % 8) ^ row of the pair's 128 bytes.
+    const char* const av = static_cast<const char*>(a.vals);
+    const int apiece = (lane & 7) ^ (lane >> 3);
+    // Index words: a window of `wsteps` steps from the aligned dword at or
+    // before its first word (`odd`: the words start 2 bytes after it);
+    // transfer q of row block rb holds its rows 4 q + lane / 16, dword
+    // (lane % 16) ^ 4 q of the window.
+    const char* const am = reinterpret_cast<const char*>(a.meta);
+    const int odd = static_cast<int>(reinterpret_cast<uintptr_t>(am) & 2);
+    const int wpairs = odd ? 3 : 4;
+    const int row_dwords = (a.Kp / 8 + odd + 3) / 4;
+
+    auto issue = [&](int p) {
+        bt.issue(128 * p, mem_at);
+        const bool half = 2 * p + 1 >= steps;  // the pair's second step lies past Kp
 #pragma unroll
-        for (int q = 0; q < PIECES; q++) {
-            const int p = t + kS24Threads * q;
-            const int r = p >> 5, pc = p & 31;
-            const int col = c0 + 8 * pc;
-            const uint32_t off =
-                col < a.N ? static_cast<uint32_t>(64 * s + r) * rowbytes + static_cast<uint32_t>(col) * 2u : kOob;
-            bv[q] = __builtin_bit_cast(i32x4v, __builtin_amdgcn_raw_buffer_load_b128(rB, off, 0, 0));
-        }
-    };
-    auto store_b = [&](int buf, const i32x4v* bv) {
+        for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-        for (int q = 0; q < PIECES; q++) {
-            const int p = t + kS24Threads * q;
-            const int r = p >> 5, pc = p & 31;
-            const int h = r >> 5, rr = r & 31, cb = pc >> 3, lp = pc & 7;
-            uint16_t* dst = &Bs[buf][((h * 4 + cb) * 32 + rr) * kDmaBRow + 8 * (lp ^ bswz64(rr))];
-            *reinterpret_cast<i32x4v*>(dst) = bv[q];
-        }
-    };
-    // compressed A fragments and index words of step s, per row block
-    auto load_a = [&](int s, i32x4v (&af)[4], int (&ix)[4]) {
+            for (int q = 0; q < 2; q++) {
+                const int row = min(row0 + 16 * rb + 8 * q + (lane >> 3), a.M - 1);
+                const char* src = av + static_cast<size_t>(row) * a.Kp + static_cast<size_t>(p) * 128 + 16 * apiece;
+                if (half && apiece >= 4) src = reinterpret_cast<const char*>(&kZeroPiece);
+                dma_x4(src, mem_at + 16384 + 2048 * rb + 1024 * q);
+            }
+        if ((p - p0) % wpairs == 0) {
 #pragma unroll
-        for (int rb = 0; rb < 4; rb++) {
-            const int row = min(row0 + 16 * rb + (lane & 15), a.M - 1);
-            af[rb] = *reinterpret_cast<const i32x4v*>(V + static_cast<size_t>(row) * vcols + 32 * s + 8 * (lane >> 4));
-            const uint32_t m = a.meta[static_cast<size_t>(row) * mcols + 4 * s + (lane >> 4)];
-            ix[rb] = static_cast<int>(m | (m << 16));
+            for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int row = min(row0 + 16 * rb + 4 * q + (lane >> 4), a.M - 1);
+                    const int d = min(4 * p + ((lane & 15) ^ (4 * q)), row_dwords - 1);
+                    const char* src = am - odd + static_cast<size_t>(row) * (a.Kp / 8) + static_cast<size_t>(d) * 4;
+                    dma_x1(src, mem_at + 16384 + 2048 * RB + 1024 * rb + 256 * q);
+                }
         }
     };
 
-    f32x4 acc[4][4];
+    f32x4 acc[RB][4];
 #pragma unroll
-    for (int rb = 0; rb < 4; rb++)
+    for (int rb = 0; rb < RB; rb++)
 #pragma unroll
         for (int c = 0; c < 4; c++) acc[rb][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int li = lane & 15, lh = lane >> 4;
-    const int br = 8 * lh + (li >> 2);
-    const int bx = bswz64(br), bh = (li & 3) >> 1;
-
-    i32x4v bv[PIECES];
-    i32x4v a0[4], a1[4];
-    int x0[4], x1[4];
-    if (steps > 0) {
-        load_b(0, bv);
-        load_a(0, a0, x0);
-        store_b(0, bv);
-    }
-    __syncthreads();
-    auto step = [&](int s, const i32x4v (&ac)[4], const int (&xc)[4], i32x4v (&an)[4], int (&xn)[4]) {
-        const bool more = s + 1 < steps;
-        if (more) {
-            load_b(s + 1, bv);
-            load_a(s + 1, an, xn);
-        }
-        const uint16_t* Bb = &Bs[s & 1][0];
-        // B operand of column block c: halves 0..7 from rows 0..31, 8..15 from rows 32..63
-        i32x4v bq[2][4];
+    const int r = lane & 15, g = lane >> 4;
+    if (p0 < p1) issue(p0);
+    for (int p = p0; p < p1; p++) {
+        wait_vmcnt<0>();
+        typedef int i32x8v __attribute__((ext_vector_type(8)));
+        i32x8v bq[2][4];
+        i32x4v af[2][RB];
+        int ix[2][RB];
+        const int w = (p - p0) % wpairs;
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint16_t* Bfr = Bb + ((h * 4 + wv) * 32 + br) * kDmaBRow + 4 * (li & 1);
+        for (int t = 0; t < 2; t++) {
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const uint16_t* Bp = Bfr + 8 * ((2 * c + bh) ^ bx);
-                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(Bp));
-                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(Bp + 4 * kDmaBRow));
-                bq[h][c] = i32x4v{__builtin_bit_cast(int, __builtin_shufflevector(lo, lo, 0, 1)),
-                                  __builtin_bit_cast(int, __builtin_shufflevector(lo, lo, 2, 3)),
-                                  __builtin_bit_cast(int, __builtin_shufflevector(hi, hi, 0, 1)),
-                                  __builtin_bit_cast(int, __builtin_shufflevector(hi, hi, 2, 3))};
+                const uint16_t* tile = reinterpret_cast<const uint16_t*>(mem + 8192 * t);
+                const i32x4v b0 = b_fragment(tile, c, lane), b1 = b_fragment(tile + 2048, c, lane);
+                bq[t][c] = __builtin_shufflevector(b0, b1, 0, 1, 2, 3, 4, 5, 6, 7);
+            }
+            const int word = 8 * (2 * w + t) + 2 * g + odd;  // byte of the lane's index word in its window
+#pragma unroll
+            for (int rb = 0; rb < RB; rb++) {
+                af[t][rb] = *reinterpret_cast<const i32x4v*>(mem + 16384 + 2048 * rb + 128 * r +
+                                                             16 * ((4 * t + g) ^ (r & 7)));
+                const int m = *reinterpret_cast<const int*>(mem + 16384 + 2048 * RB + 1024 * rb + 64 * r +
+                                                            4 * ((word >> 2) ^ (4 * (r >> 2))));
+                const uint32_t x = (static_cast<uint32_t>(m) >> (8 * (word & 2))) & 0xffffu;
+                ix[t][rb] = static_cast<int>(x | (x << 16));
             }
         }
+        wait_lds_reads();
+        if (p + 1 < p1) issue(p + 1);
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            typedef int i32x8v __attribute__((ext_vector_type(8)));
-            const i32x8v b8 = __builtin_shufflevector(bq[0][c], bq[1][c], 0, 1, 2, 3, 4, 5, 6, 7);
+        for (int t = 0; t < 2; t++)
 #pragma unroll
-            for (int rb = 0; rb < 4; rb++) {
-                if constexpr (kBf16)
-                    acc[rb][c] = __builtin_amdgcn_smfmac_f32_16x16x64_bf16(
-                        __builtin_bit_cast(bf16x8, ac[rb]), __builtin_bit_cast(bf16x16, b8), acc[rb][c], xc[rb], 0, 0);
-                else
-                    acc[rb][c] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(
-                        __builtin_bit_cast(f16x8, ac[rb]), __builtin_bit_cast(f16x16, b8), acc[rb][c], xc[rb], 0, 0);
-            }
-        }
-        if (more) store_b((s + 1) & 1, bv);
-        __syncthreads();
-    };
-    int s = 0;
-    for (; s + 1 < steps; s += 2) {
-        step(s, a0, x0, a1, x1);
-        step(s + 1, a1, x1, a0, x0);
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int rb = 0; rb < RB; rb++) {
+                    if constexpr (kBf16)
+                        acc[rb][c] = __builtin_amdgcn_smfmac_f32_16x16x64_bf16(__builtin_bit_cast(bf16x8, af[t][rb]),
+                                                                               __builtin_bit_cast(bf16x16, bq[t][c]),
+                                                                               acc[rb][c], ix[t][rb], 0, 0);
+                    else
+                        acc[rb][c] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(__builtin_bit_cast(f16x8, af[t][rb]),
+                                                                              __builtin_bit_cast(f16x16, bq[t][c]),
+                                                                              acc[rb][c], ix[t][rb], 0, 0);
+                }
     }
-    if (s < steps) step(s, a0, x0, a1, x1);
-
-#pragma unroll
-    for (int rb = 0; rb < 4; rb++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int col = c0 + 64 * wv + 16 * c + (lane & 15);
-            if (col >= a.N) continue;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = row0 + 16 * rb + 4 * (lane >> 4) + r;
-                if (row < a.M) __builtin_nontemporal_store(acc[rb][c][r], a.C + static_cast<size_t>(row) * a.N + col);
-            }
-        }
+    reduce_store<RB, 4, W>(acc, lds, wave, lane, row0, c0, a.M, a.N, a.C);
 }
 
 }  // namespace tca

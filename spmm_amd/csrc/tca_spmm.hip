@@ -477,6 +477,36 @@ void launch_sddmm(const SddmmArgs& a, hipStream_t s) {
     else launch_sddmm_e<T, 1>(a, s);
 }
 
+template <bool kBf16, int RB, int W>
+int launch_s24_t(S24Args a, hipStream_t s) {
+    a.row_groups = static_cast<int>((static_cast<int64_t>(a.M) + 16 * RB - 1) / (16 * RB));
+    const int64_t groups = static_cast<int64_t>(a.row_groups) * a.col_groups;
+    if (groups > 0x7fffffff) return fail(TCA_ERR_UNSUPPORTED, "tca_spmm_24: grid too large");
+    static_assert(s24_lds_bytes<RB, W>() <= 160 * 1024, "LDS budget");
+    hipLaunchKernelGGL((sparse24_kernel<kBf16, RB, W>), dim3(static_cast<unsigned>(groups)), dim3(64 * W), 0, s, a);
+    return TCA_OK;
+}
+
+// The tallest tile costs the fewest bytes per output (its B tile serves the
+// most rows) but leaves the chip idle on small outputs: the shortest tile
+// whose workgroups fit the 256 CUs in one round (a workgroup's LDS takes a
+// CU), the tallest when none does.  us per product, bf16, M x K x N
+// (workgroups of the tile in brackets):
+//                        16 rows     32 rows     64 rows     128 rows
+//   287 x 5057 x 16       9.6 [18]    12.2 [9]    17.2 [5]    23.5 [3]
+//   700 x 700 x 512       7.2 [352]    7.2 [176]   7.5 [88]    8.7 [48]
+//   3145 x 5004 x 288    41.5 [985]   28.0 [495]  19.6 [250]  25.3 [125]
+//   5580 x 1872 x 184    24.1 [1047]  20.0 [525]  17.1 [264]  13.6 [132]
+//   4096 x 4096 x 512    62.6 [2048]  40.6 [1024] 28.9 [512]  22.1 [256]
+template <bool kBf16>
+int launch_s24(const S24Args& a, hipStream_t s) {
+    auto fits = [&](int rows) { return (static_cast<int64_t>(a.M) + rows - 1) / rows * a.col_groups <= 256; };
+    if (fits(16)) return launch_s24_t<kBf16, 1, 8>(a, s);
+    if (fits(32)) return launch_s24_t<kBf16, 2, 6>(a, s);
+    if (fits(64)) return launch_s24_t<kBf16, 4, 4>(a, s);
+    return launch_s24_t<kBf16, 8, 4>(a, s);
+}
+
 // Bit 1 << TCA_PHASE_* for each phase in which the plan launches a kernel.
 uint32_t phases_used(const tca_spmm_plan* p) {
     uint32_t m = 0;
@@ -2000,16 +2030,12 @@ int tca_spmm_24(const void* d_vals, const uint16_t* d_meta, int32_t M, int32_t K
     a.C = d_C;
     a.M = M;
     a.N = N;
+    a.K = K;
     a.Kp = (K + 63) / 64 * 64;
     a.col_groups = (N + kS24Cols - 1) / kS24Cols;
-    a.B_bytes = static_cast<uint32_t>(static_cast<uint64_t>(K) * N * 2);
-    const int64_t groups = (static_cast<int64_t>(M) + kS24Rows - 1) / kS24Rows * a.col_groups;
-    if (groups > 0x7fffffff) return fail(TCA_ERR_UNSUPPORTED, "tca_spmm_24: grid too large");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == TCA_BF16)
-        hipLaunchKernelGGL(sparse24_kernel<true>, dim3(static_cast<unsigned>(groups)), dim3(kS24Threads), 0, s, a);
-    else
-        hipLaunchKernelGGL(sparse24_kernel<false>, dim3(static_cast<unsigned>(groups)), dim3(kS24Threads), 0, s, a);
+    const int st = dtype == TCA_BF16 ? launch_s24<true>(a, s) : launch_s24<false>(a, s);
+    if (st) return st;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(TCA_ERR_HIP, "kernel launch: %s", hipGetErrorString(e));
     return TCA_OK;

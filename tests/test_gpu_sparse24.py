@@ -50,3 +50,42 @@ def test_spmm_24_random_values_within_tolerance(torch_cuda):
     b = S.to_storage(rng.uniform(-1, 1, (2048, 512)).astype(np.float32), S.TCA_F16)
     got = _run(torch_cuda, a, b)
     assert_parity(a, b, got, "2:4 2048x2048")
+
+
+@pytest.mark.parametrize("m,n", [(1, 8), (287, 16), (15, 1000), (17, 72), (300, 1000), (600, 1000), (640, 1024),
+                                 (1100, 1000), (1281, 904)])
+@pytest.mark.parametrize("k", [1, 63, 64, 65, 129, 448, 1000])
+def test_spmm_24_every_tile(torch_cuda, m, n, k):
+    """Sizes that take each tile height (16, 32, 64 and 128 rows), with partial
+    row and column tiles, whole and half last step pairs, fewer pairs than
+    wavefronts and index windows that end inside a row."""
+    rng = np.random.default_rng(m * 7 + k)
+    a = _pruned(rng, m, k, 0.2, S.TCA_BF16 if k % 2 else S.TCA_F16)
+    b = S.to_storage(exact_dense(rng, (k, n)), a.dtype)
+    got = _run(torch_cuda, a, b)
+    want = oracle.csr_spmm(a.rowptr, a.colidx, a.values_f32(), S.from_storage(b, a.dtype))
+    assert np.array_equal(got, want), np.abs(got - want).max()
+
+
+@pytest.mark.parametrize("k", [64, 320, 1000])
+@pytest.mark.parametrize("shift", [1, 2])
+def test_spmm_24_index_words_at_any_halfword(torch_cuda, k, shift):
+    """Index words that start 2 or 4 bytes into their buffer; NaN rows of B past
+    K and a NaN row of A after the last one stay out of the product."""
+    torch = torch_cuda
+    rng = np.random.default_rng(k + shift)
+    m, n = 50, 72
+    a = _pruned(rng, m, k, 0.4, S.TCA_F16)
+    vals, meta = S.csr_to_24(a)
+    b = S.to_storage(exact_dense(rng, (k, n)), S.TCA_F16)
+    buf = torch.zeros(meta.size + shift, dtype=torch.int16, device="cuda:0")
+    buf[shift:] = torch.from_numpy(meta.ravel().view(np.int16)).to("cuda:0")
+    nan = np.full((70, n), np.nan, np.float16)
+    bd = _dev(torch, np.concatenate([b, nan]))
+    vd = _dev(torch, np.concatenate([vals, np.full((1, vals.shape[1]), 0x7e00, np.uint16)]))
+    c = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+    print(f"2:4 K={k} shift={shift}", flush=True)
+    S.spmm_24(vd, buf[shift:], m, k, n, S.TCA_F16, bd, c)
+    torch.cuda.synchronize()
+    want = oracle.csr_spmm(a.rowptr, a.colidx, a.values_f32(), S.from_storage(b, S.TCA_F16))
+    assert np.array_equal(c.cpu().numpy(), want)
