@@ -4,27 +4,25 @@
 // Blocked-ELL is the format the reference hands to cusparseSpMM for its
 // block baseline (src/spmm_cusparse.cu:201-342; layout in tca_host.h):
 // every block is a dense BS x BS tile, so the format feeds the matrix cores
-// with no condensing.  A workgroup owns one block row (BS rows) and 256
-// columns of C; wavefront w owns columns 64 w .. 64 w + 63.  Per ELL block e
-// of the block row:
-//   * the BS rows of B it multiplies (block column colind[e] * BS ..) x the
-//     workgroup's 256 columns are staged in LDS, double-buffered: every
-//     thread loads BS / 8 pieces of 16 bytes (coalesced, 512 bytes per row)
-//     one block ahead and writes them after the MFMAs of the current block.
-//     The LDS tile is [32-row step][64-column block][32 rows][64 halves]
-//     with the 16-byte pieces of each 128-byte row XOR-permuted by bswz64,
-//     so the transposing fragment reads (ds_read_b64_tr_b16) are
-//     conflict-free, exactly as in the condensed-tile kernels;
-//   * the A fragments come straight from global memory: lane l of fragment
-//     (row block rf, step ks) needs row 16 rf + l % 16, columns
-//     32 ks + 8 (l / 16) .. + 7 of the block, 16 contiguous bytes of the
-//     row-major ELL values, loaded one block ahead;
-//   * v_mfma_f32_16x16x32_{f16,bf16}: (BS / 16) row blocks x 4 column
-//     blocks x (BS / 32) steps per wavefront.
-// Blocks are added in ELL order, so every output is one MFMA chain in a
-// fixed order (deterministic).  B rows past K and columns past N load as
-// zeros (buffer range checks); rows past M and columns past N are not
-// stored.  Padding blocks (colind -1) end the block row's list.
+// with no condensing.  A workgroup owns one block row (BS rows) and 64 columns
+// of C.  Its W wavefronts split the block row's list, each a contiguous range
+// of it, and meet once at the end (reduce_store), so the loop has no barrier:
+// a wavefront fills LDS of its own with global -> LDS transfers of the next
+// unit as soon as it has read the last one into registers, and multiplies
+// that meanwhile.  A unit is 64 columns of A (one block of 64 or two of 32),
+// so every line of the row-major ELL values is used whole: lines from the L2
+// to the CU, about 4 cycles each, bound the kernel (A 2 BS / 32 KiB, B 8 KiB a
+// unit), and with one block of 32 at a time half of A's would be wasted.
+//
+// 4096 x 4096 fp16 with a quarter of its 32 x 32 blocks at N = 512: 15.1 us
+// (31.5 with a workgroup per block row and 256 columns, B staged one block
+// ahead through registers with a barrier per block).  128 columns per
+// wavefront: 14.5 us there, but up to twice as long on small outputs.
+//
+// Sums run in list order within a wavefront's range, the ranges in order.  The
+// missing half of an odd list's last unit, B rows past K and columns past N
+// come from a zero piece; rows past M are not stored.  Padding blocks (colind
+// -1) end the block row's list.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -34,82 +32,79 @@
 
 namespace tca {
 
-constexpr int kBellThreads = 256;  // 4 wavefronts
-constexpr int kBellCols = 256;     // columns of C per workgroup
+constexpr int kBellCols = 64;  // columns of C per workgroup
 
 struct BellArgs {
     const int* colind;   // [block rows][ell_blocks] block column, -1 = padding
     const void* values;  // [block rows * BS][ell_blocks * BS] row-major
     const void* B;       // K x N row-major
     float* C;            // M x N row-major
-    int M, N, ell_blocks;
-    int col_groups;      // workgroups per block row: blockIdx.x = block row * col_groups + group
-    uint32_t B_bytes;    // K * N * 2
+    int M, N, K, ell_blocks;
+    int row_groups, col_groups;  // block rows, column groups
 };
 
+// LDS of a wavefront: a unit's B tiles and A pieces.
 template <int BS>
-constexpr int bell_lds_bytes() {
-    return 2 * BS * kBellCols * 2;
+constexpr int bell_wave_bytes() {
+    return 8192 + BS * 128;
 }
 
-template <bool kBf16, int BS>
-__global__ __launch_bounds__(kBellThreads) void bell_mfma_kernel(BellArgs a) {
+template <bool kBf16, int BS, int W>
+__global__ __launch_bounds__(64 * W) void bell_mfma_kernel(BellArgs a) {
     static_assert(BS == 32 || BS == 64, "block size");
-    constexpr int KS = BS / 32;               // 32-deep MFMA steps per block
-    constexpr int RF = BS / 16;               // 16-row fragments per block row
-    constexpr int PIECES = BS / 8;            // 16-byte B pieces per thread and block
-    constexpr int kTile = BS * kBellCols;     // halves of one staged B tile
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][kTile];
+    constexpr int RF = BS / 16;   // 16-row fragments per block row
+    constexpr int kBlk = 64 / BS; // blocks of a unit
+    constexpr int kLds = W * (bell_wave_bytes<BS>() > RF * 4096 ? bell_wave_bytes<BS>() : RF * 4096);
+    __shared__ __attribute__((aligned(16))) char lds[kLds];
 
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int brow = blockIdx.x / a.col_groups;
-    const int c0 = (blockIdx.x % a.col_groups) * kBellCols;
-    const int ecols = a.ell_blocks * BS;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int brow, cg;
+    xcd_tile(blockIdx.x, a.row_groups, a.col_groups, brow, cg);
+    const int c0 = cg * kBellCols;
     const int* const cind = a.colind + static_cast<size_t>(brow) * a.ell_blocks;
-    const char* const Av = static_cast<const char*>(a.values);
-    const __amdgpu_buffer_rsrc_t rB = make_rsrc(a.B, a.B_bytes);
-    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * 2u;
 
     // number of blocks in this block row (the list is a prefix, -1 after it)
-    int nblk = 0;
-    while (nblk < a.ell_blocks && cind[nblk] >= 0) nblk++;
+    int nblk = 0, first64 = -1;
+    while (nblk < a.ell_blocks) {
+        const int e = nblk + lane;
+        const int c = cind[min(e, a.ell_blocks - 1)];
+        const uint64_t ends = __ballot(e >= a.ell_blocks || c < 0);
+        if (nblk == 0) first64 = c;
+        nblk += ends ? __builtin_ctzll(ends) : 64;
+        if (ends) break;
+    }
+    // First row of B of block e (the list's first 64 entries stay in registers;
+    // a block column past K reads zeros).
+    const int kblk = (a.K + BS - 1) / BS;
+    auto block_row = [&](int e) {
+        return min(nblk <= 64 ? __builtin_amdgcn_readlane(first64, e) : cind[e], kblk) * BS;
+    };
+    const int units = (nblk + kBlk - 1) / kBlk;
+    const int u0 = static_cast<int>(static_cast<int64_t>(units) * wave / W);
+    const int u1 = static_cast<int>(static_cast<int64_t>(units) * (wave + 1) / W);
+    char* const mem = lds + wave * bell_wave_bytes<BS>();
+    const uint32_t mem_at = lds_addr(mem);
 
-    // B pieces of this thread: piece p = t + 256 q covers row p / 32 of the
-    // block, bytes 16 (p % 32) .. of the workgroup's 512-byte row slice.
-    auto load_b = [&](int e, i32x4v* bv) {
-        const int r0 = cind[e] * BS;
+    BTile<BS / 32> bt;
+    bt.init(a.B, a.K, a.N, c0, lane);
+    // A: transfer q holds rows 8 q + lane / 8 of the block row, 16-byte piece
+    // (lane % 8) ^ row of the unit's 128 bytes.
+    const int apiece = (lane & 7) ^ (lane >> 3);
+    const size_t arow = static_cast<size_t>(a.ell_blocks) * BS * 2;  // bytes
+    const char* const av = static_cast<const char*>(a.values) + (static_cast<size_t>(brow) * BS + (lane >> 3)) * arow +
+                           16 * apiece;
+    auto issue = [&](int u) {
+        const bool half = kBlk == 2 && 2 * u + 1 >= nblk;
 #pragma unroll
-        for (int q = 0; q < PIECES; q++) {
-            const int p = t + kBellThreads * q;
-            const int r = p >> 5, pc = p & 31;
-            const int col = c0 + 8 * pc;
-            const uint32_t off =
-                col < a.N ? static_cast<uint32_t>(r0 + r) * rowbytes + static_cast<uint32_t>(col) * 2u : kOob;
-            bv[q] = __builtin_bit_cast(i32x4v, __builtin_amdgcn_raw_buffer_load_b128(rB, off, 0, 0));
+        for (int b = 0; b < kBlk; b++)
+            bt.issue(b && half ? a.K : block_row(kBlk * u + b), mem_at + 4096 * b);
+#pragma unroll
+        for (int q = 0; q < BS / 8; q++) {
+            const char* src = av + 8 * q * arow + static_cast<size_t>(u) * 128;
+            if (half && apiece >= 4) src = reinterpret_cast<const char*>(&kZeroPiece);
+            dma_x4(src, mem_at + 8192 + 1024 * q);
         }
-    };
-    auto store_b = [&](int buf, const i32x4v* bv) {
-#pragma unroll
-        for (int q = 0; q < PIECES; q++) {
-            const int p = t + kBellThreads * q;
-            const int r = p >> 5, pc = p & 31;
-            const int ks = r >> 5, rr = r & 31, cb = pc >> 3, lp = pc & 7;
-            uint16_t* dst = &Bs[buf][((ks * 4 + cb) * 32 + rr) * kDmaBRow + 8 * (lp ^ bswz64(rr))];
-            *reinterpret_cast<i32x4v*>(dst) = bv[q];
-        }
-    };
-    // A fragments of block e: [row block][step]
-    auto load_a = [&](int e, i32x4v (&af)[RF][KS]) {
-#pragma unroll
-        for (int rf = 0; rf < RF; rf++)
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const size_t row = static_cast<size_t>(brow) * BS + rf * 16 + (lane & 15);
-                const size_t col = static_cast<size_t>(e) * BS + ks * 32 + 8 * (lane >> 4);
-                af[rf][ks] = *reinterpret_cast<const i32x4v*>(Av + (row * ecols + col) * 2);
-            }
     };
 
     f32x4 acc[RF][4];
@@ -118,79 +113,40 @@ __global__ __launch_bounds__(kBellThreads) void bell_mfma_kernel(BellArgs a) {
 #pragma unroll
         for (int c = 0; c < 4; c++) acc[rf][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int li = lane & 15, lh = lane >> 4;
-    const int br = 8 * lh + (li >> 2);
-    const int bx = bswz64(br), bh = (li & 3) >> 1;
-
-    i32x4v bv[PIECES];
-    i32x4v a0[RF][KS], a1[RF][KS];
-    if (nblk > 0) {
-        load_b(0, bv);
-        load_a(0, a0);
-        store_b(0, bv);
-    }
-    __syncthreads();
-    // block e: MFMAs from LDS buffer e & 1 and A registers `ac`; loads of
-    // block e + 1 into registers (B pieces, `an`), B stored after the MFMAs
-    auto block = [&](int e, const i32x4v (&ac)[RF][KS], i32x4v (&an)[RF][KS]) {
-        const bool more = e + 1 < nblk;
-        if (more) {
-            load_b(e + 1, bv);
-            load_a(e + 1, an);
+    const int r = lane & 15, g = lane >> 4;
+    if (u0 < u1) issue(u0);
+    for (int u = u0; u < u1; u++) {
+        wait_vmcnt<0>();
+        i32x4v bq[2][4], af[2][RF];
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) 
+                bq[ks][c] = b_fragment(reinterpret_cast<const uint16_t*>(mem + 4096 * ks), c, lane);
+#pragma unroll
+            for (int rf = 0; rf < RF; rf++)
+                af[ks][rf] =
+                    *reinterpret_cast<const i32x4v*>(mem + 8192 + 2048 * rf + 128 * r + 16 * ((4 * ks + g) ^ (r & 7)));
         }
-        const uint16_t* Bb = &Bs[e & 1][0];
+        wait_lds_reads();
+        if (u + 1 < u1) issue(u + 1);
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++) {
-            const uint16_t* Bfr = Bb + ((ks * 4 + wv) * 32 + br) * kDmaBRow + 4 * (li & 1);
-            i32x4v bq[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const uint16_t* Bp = Bfr + 8 * ((2 * c + bh) ^ bx);
-                const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(Bp));
-                const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(Bp + 4 * kDmaBRow));
-                bq[c] = i32x4v{__builtin_bit_cast(int, __builtin_shufflevector(lo, lo, 0, 1)),
-                               __builtin_bit_cast(int, __builtin_shufflevector(lo, lo, 2, 3)),
-                               __builtin_bit_cast(int, __builtin_shufflevector(hi, hi, 0, 1)),
-                               __builtin_bit_cast(int, __builtin_shufflevector(hi, hi, 2, 3))};
-            }
+        for (int ks = 0; ks < 2; ks++)
 #pragma unroll
             for (int c = 0; c < 4; c++)
 #pragma unroll
                 for (int rf = 0; rf < RF; rf++) {
                     if constexpr (kBf16)
-                        acc[rf][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(bf16x8, ac[rf][ks]), __builtin_bit_cast(bf16x8, bq[c]), acc[rf][c], 0, 0,
-                            0);
+                        acc[rf][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[ks][rf]),
+                                                                             __builtin_bit_cast(bf16x8, bq[ks][c]),
+                                                                             acc[rf][c], 0, 0, 0);
                     else
-                        acc[rf][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            __builtin_bit_cast(f16x8, ac[rf][ks]), __builtin_bit_cast(f16x8, bq[c]), acc[rf][c], 0, 0,
-                            0);
+                        acc[rf][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, af[ks][rf]),
+                                                                            __builtin_bit_cast(f16x8, bq[ks][c]),
+                                                                            acc[rf][c], 0, 0, 0);
                 }
-        }
-        // buffer (e + 1) & 1 was last read in block e - 1, before its barrier
-        if (more) store_b((e + 1) & 1, bv);
-        __syncthreads();
-    };
-    int e = 0;
-    for (; e + 1 < nblk; e += 2) {
-        block(e, a0, a1);
-        block(e + 1, a1, a0);
     }
-    if (e < nblk) block(e, a0, a1);
-
-    // D layout: lane l holds rows 4 (l / 16) + r, column l % 16 of each 16 x 16 block
-#pragma unroll
-    for (int rf = 0; rf < RF; rf++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int col = c0 + 64 * wv + 16 * c + (lane & 15);
-            if (col >= a.N) continue;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = brow * BS + 16 * rf + 4 * (lane >> 4) + r;
-                if (row < a.M) __builtin_nontemporal_store(acc[rf][c][r], a.C + static_cast<size_t>(row) * a.N + col);
-            }
-        }
+    reduce_store<RF, 4, W>(acc, lds, wave, lane, brow * BS, c0, a.M, a.N, a.C);
 }
 
 }  // namespace tca

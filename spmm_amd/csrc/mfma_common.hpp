@@ -126,6 +126,20 @@ __device__ __forceinline__ void wait_vmcnt() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// Workgroup -> tile: workgroup b runs on XCD b % 8; the column groups of one
+// row group follow each other on one XCD, whose L2 then fetches the row
+// group's A once.
+__device__ __forceinline__ void xcd_tile(int b, int row_groups, int col_groups, int& rg, int& cg) {
+    const int q = row_groups / 8 * 8 * col_groups;  // workgroups of whole eights of row groups
+    if (b < q) {
+        rg = b / (8 * col_groups) * 8 + b % 8;
+        cg = b / 8 % col_groups;
+    } else {
+        rg = row_groups / 8 * 8 + (b - q) / col_groups;
+        cg = (b - q) % col_groups;
+    }
+}
+
 // Source of the B rows past K and columns past N of a transfer.
 static __device__ const int4 kZeroPiece = {0, 0, 0, 0};
 

@@ -59,20 +59,6 @@ struct S24Args {
     int row_groups, col_groups;
 };
 
-// Workgroup -> tile: workgroup b runs on XCD b % 8; the column groups of one
-// row group follow each other on one XCD, whose L2 then fetches the row
-// group's A once.
-__device__ __forceinline__ void s24_tile(int b, int row_groups, int col_groups, int& rg, int& cg) {
-    const int q = row_groups / 8 * 8 * col_groups;  // workgroups of whole eights of row groups
-    if (b < q) {
-        rg = b / (8 * col_groups) * 8 + b % 8;
-        cg = b / 8 % col_groups;
-    } else {
-        rg = row_groups / 8 * 8 + (b - q) / col_groups;
-        cg = (b - q) % col_groups;
-    }
-}
-
 // LDS of a wavefront: two steps' B tiles (16 KiB), A pieces (2 KiB per row
 // block) and a window of index words (1 KiB per row block).
 template <int RB>
@@ -91,7 +77,7 @@ __global__ __launch_bounds__(64 * W) void sparse24_kernel(S24Args a) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int rg, cg;
-    s24_tile(blockIdx.x, a.row_groups, a.col_groups, rg, cg);
+    xcd_tile(blockIdx.x, a.row_groups, a.col_groups, rg, cg);
     const int row0 = rg * 16 * RB, c0 = cg * kS24Cols;
     const int steps = a.Kp / 64;
     const int pairs = (steps + 1) / 2;  // the second step of the last pair may be missing

@@ -507,6 +507,28 @@ int launch_s24(const S24Args& a, hipStream_t s) {
     return launch_s24_t<kBf16, 8, 4>(a, s);
 }
 
+// Wavefronts per tile: enough to fill the chip and to shorten a tile's serial
+// chain of units, no more (each holds LDS and adds to the final sums).  us per
+// product, M x K x N, block size, workgroups:     1      2      4      8
+//   287 x 5057 x 16, 32, 9                       18.2   10.8    7.7    7.6
+//   3145 x 5004 x 288, 64, 250                   14.7    9.3    7.6    7.4
+//   5580 x 1872 x 184, 64, 264                   10.8    7.5    7.5    8.3
+//   2000 x 600 x 1000, 32, 1008                   8.7    7.5    8.1   11.9
+//   4096 x 4096 x 512, 32, 1024                  20.2   15.1   17.0   20.0
+template <bool kBf16, int BS>
+void launch_bell_w(const BellArgs& a, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(a.row_groups * a.col_groups));
+    if (grid.x > 512) hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 2>), grid, dim3(128), 0, s, a);
+    else if (grid.x > 256) hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 4>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 8>), grid, dim3(512), 0, s, a);
+}
+
+template <bool kBf16>
+void launch_bell(const BellArgs& a, int bsize, hipStream_t s) {
+    if (bsize == 32) launch_bell_w<kBf16, 32>(a, s);
+    else launch_bell_w<kBf16, 64>(a, s);
+}
+
 // Bit 1 << TCA_PHASE_* for each phase in which the plan launches a kernel.
 uint32_t phases_used(const tca_spmm_plan* p) {
     uint32_t m = 0;
@@ -1992,20 +2014,14 @@ int tca_bell_spmm(const int32_t* d_colind, const void* d_values, int32_t M, int3
     a.M = M;
     a.N = N;
     a.ell_blocks = ell_blocks;
+    a.K = K;
+    a.row_groups = static_cast<int>((static_cast<int64_t>(M) + bsize - 1) / bsize);
     a.col_groups = (N + kBellCols - 1) / kBellCols;
-    a.B_bytes = static_cast<uint32_t>(static_cast<uint64_t>(K) * N * 2);
-    const int64_t brows = (static_cast<int64_t>(M) + bsize - 1) / bsize;
-    if (brows * a.col_groups > 0x7fffffff) return fail(TCA_ERR_UNSUPPORTED, "tca_bell_spmm: grid too large");
-    const dim3 grid(static_cast<unsigned>(brows * a.col_groups));
+    if (static_cast<int64_t>(a.row_groups) * a.col_groups > 0x7fffffff)
+        return fail(TCA_ERR_UNSUPPORTED, "tca_bell_spmm: grid too large");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool bf = dtype == TCA_BF16;
-    if (bsize == 32) {
-        if (bf) hipLaunchKernelGGL((bell_mfma_kernel<true, 32>), grid, dim3(kBellThreads), 0, s, a);
-        else hipLaunchKernelGGL((bell_mfma_kernel<false, 32>), grid, dim3(kBellThreads), 0, s, a);
-    } else {
-        if (bf) hipLaunchKernelGGL((bell_mfma_kernel<true, 64>), grid, dim3(kBellThreads), 0, s, a);
-        else hipLaunchKernelGGL((bell_mfma_kernel<false, 64>), grid, dim3(kBellThreads), 0, s, a);
-    }
+    if (dtype == TCA_BF16) launch_bell<true>(a, bsize, s);
+    else launch_bell<false>(a, bsize, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(TCA_ERR_HIP, "kernel launch: %s", hipGetErrorString(e));
     return TCA_OK;

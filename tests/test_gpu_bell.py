@@ -70,3 +70,48 @@ def test_bell_block_row_without_blocks_is_zero(torch_cuda):
     got = _run(torch_cuda, a, b, 32)
     assert np.all(got[32:64] == 0.0)
     assert np.array_equal(got, oracle.csr_spmm(a.rowptr, a.colidx, a.values_f32(), S.from_storage(b, S.TCA_F16)))
+
+
+def _blocks(rng, lists, k, bs, dtype, pad_nan=False):
+    """Blocked-ELL arrays with the given block columns per block row, and the dense A."""
+    eb = max((len(x) for x in lists), default=0) + (1 if pad_nan else 0)
+    colind = np.full((len(lists), eb), -1, np.int32)
+    vals = np.zeros((len(lists) * bs, eb * bs), np.float32)
+    dense = np.zeros((len(lists) * bs, (k + bs - 1) // bs * bs))
+    if pad_nan:
+        vals[:] = np.nan
+    for i, cols in enumerate(lists):
+        for e, c in enumerate(cols):
+            colind[i, e] = c
+            v = exact_values(rng, bs * bs).reshape(bs, bs) * (rng.random((bs, bs)) < 0.1)
+            vals[i * bs:(i + 1) * bs, e * bs:(e + 1) * bs] = v
+            if c * bs < k:
+                dense[i * bs:(i + 1) * bs, c * bs:(c + 1) * bs] = v
+    return colind, S.to_storage(vals, dtype), dense[:, :k]
+
+
+@pytest.mark.parametrize("bs", [32, 64])
+@pytest.mark.parametrize("n,brows", [(8, 3), (72, 150), (520, 60), (1000, 40)])
+def test_bell_list_lengths(torch_cuda, bs, n, brows):
+    """Every count of wavefronts per tile (by workgroups: up to 256, 512, more)
+    over empty, odd and even lists, shorter and longer than the wavefronts, and
+    lists of more than 64 blocks; NaN in the padding blocks, a block column past
+    K, K that ends inside a block, M inside the last block row."""
+    torch = torch_cuda
+    rng = np.random.default_rng(brows + bs)
+    k = 70 * bs - 5
+    lens = [0, 1, 2, 3, 4, 7, 16, 17]
+    lists = [np.sort(rng.choice(70, lens[i % len(lens)], replace=False)) for i in range(brows)]
+    lists[1], lists[2] = np.arange(70), np.arange(65)
+    lists[0] = np.array([3, 69, 70 + 5, 2 ** 30])
+    colind, vals, dense = _blocks(rng, lists, k, bs, S.TCA_BF16, pad_nan=True)
+    m = brows * bs - 3
+    b = exact_dense(rng, (k, n))
+    c = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda:0")
+    print(f"bell lists bs={bs} n={n} brows={brows}", flush=True)
+    db = _dev(torch, S.to_storage(np.concatenate([b, np.full((64, n), np.nan, np.float32)]), S.TCA_BF16))
+    dc, dv = _dev(torch, colind), _dev(torch, vals)
+    S.bell_spmm(dc, dv, m, k, n, bs, S.TCA_BF16, db, c)
+    torch.cuda.synchronize()
+    want = (dense[:m] @ b.astype(np.float64)).astype(np.float32)
+    assert np.array_equal(c.cpu().numpy(), want)
