@@ -140,9 +140,6 @@ __device__ __forceinline__ void xcd_tile(int b, int row_groups, int col_groups, 
     }
 }
 
-// Source of the B rows past K and columns past N of a transfer.
-static __device__ const int4 kZeroPiece = {0, 0, 0, 0};
-
 // Issues the transfers of 32 * H rows x 64 columns of B (row-major, N columns,
 // rows r0 .., columns c0 ..) into LDS byte address `lds`: H tiles of 32 rows of
 // 128 bytes, 16-byte pieces permuted by bswz64.  4 H transfers of 8 rows.

@@ -37,8 +37,10 @@ int32_t default_slices(int32_t K, int32_t N, int32_t dtype) {
 void plan_geometry(int32_t N, int32_t es, int32_t slices, RowPlan* p) {
     int32_t e = 16 / es;
     while (e > 1 && N % e != 0) e >>= 1;
+    p->ragged = e < 4 && N >= (es == 4 ? kRaggedMinN32 : kRaggedMinN16);
+    if (p->ragged) e = 16 / es;
     p->elems_per_lane = e;
-    const int64_t lanes = N / e;  // 16-byte (or narrower) vectors across one B row
+    const int64_t lanes = (N + e - 1) / e;  // 16-byte (or narrower) vectors across one B row
     int64_t nch = 1;
     if (slices > 0) {
         nch = slices;

@@ -40,6 +40,18 @@ constexpr int32_t kZeroRows = 64;
 constexpr int32_t kMultiPasses = 4;
 inline int32_t multi_group_rows(int32_t slots) { return slots * kMultiPasses < 64 ? slots * kMultiPasses : 64; }
 
+// Widths whose widest dividing vector is one or two elements take whole
+// 16-byte vectors instead, the last one ending at the row's end
+// (RowPlan::ragged); narrower rows keep vectors that divide them.  us per
+// product on the MI355X, dividing against whole vectors, a 3001 x 2049 layer
+// of 8 % / an R-MAT graph of 200,000 nodes and 7M nonzeros: fp32 N = 17
+// 9.7 -> 8.1 / 130 -> 84, N = 26 7.8 -> 8.1 / 110 -> 95, N = 47 graph of
+// 400,000 nodes 356 -> 303; 16-bit N = 17 10.0 -> 10.9 / 127 -> 129, N = 30
+// - / 96.5 -> 97.2, N = 39 13.0 -> 9.9 / 167 -> 136, N = 70 14.0 -> 9.5 /
+// 183 -> 144, bf16 N = 333 72 -> 39 / -.
+constexpr int32_t kRaggedMinN32 = 16;
+constexpr int32_t kRaggedMinN16 = 33;
+
 struct Int4 {
     int32_t x, y, z, w;
 };
@@ -47,6 +59,7 @@ struct Int4 {
 struct RowPlan {
     // lane geometry
     int32_t elems_per_lane = 1;  // B columns per lane per load (16-byte vectors when possible)
+    bool ragged = false;         // elems_per_lane does not divide N: a row's last vector ends at its end
     int32_t log_lanes = 6;       // log2(G): lanes per slot, G >= chunk_lanes
     int32_t chunk_lanes = 64;    // lanes holding data in one column chunk
     int32_t col_chunks = 1;      // column chunks (grid.x = task groups * col_chunks)

@@ -137,10 +137,84 @@ __device__ __forceinline__ void store_line_pieces(float* row, int chunk_col, int
         __builtin_nontemporal_store(p.p1, reinterpret_cast<f32x4*>(row + chunk_col + 4 * (g + cl)));
 }
 
+// Widths that E does not divide (kRagged): lane g of a slot reads columns
+// [min(E g, N - E), + E) of a B row -- the row's last vector ends at the row's
+// end, so no load leaves it -- and left_align moves its sums to E g once per
+// row; C is stored by pieces of four columns, the last one by element.
+// Vectors start at any element: fp32 ones through the buffer (dword aligned),
+// 16-bit ones through plain loads, masked ones from the zero piece.
+static __device__ const int4 kZeroPiece = {0, 0, 0, 0};
+
+template <typename T, int E>
+__device__ __forceinline__ Pack<T, E> load_unaligned(const T* p) {
+    struct __attribute__((packed, aligned(sizeof(T)))) U {
+        T v[E];
+    };
+    return __builtin_bit_cast(Pack<T, E>, *reinterpret_cast<const U*>(p));
+}
+
+// E elements of B at byte offset `off` (zeros unless ok).
+template <typename T, int E, bool kRagged>
+__device__ __forceinline__ Pack<T, E> load_b(__amdgpu_buffer_rsrc_t rB, const void* B, uint32_t off, bool ok) {
+    if constexpr (kRagged && sizeof(T) == 2) {
+        // (global address space spelled out: the select would make it a flat load)
+        typedef int i32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
+        using Global = const __attribute__((address_space(1))) char*;
+        const Global src = ok ? (Global)B + off : (Global)&kZeroPiece;
+        return __builtin_bit_cast(Pack<T, E>, *(const __attribute__((address_space(1))) i32x4a2*)src);
+    } else {
+        return load_pack<T, E>(rB, ok ? off : kOob);
+    }
+}
+
+// v[i] = v[i + by] (0 <= by < E), zeros behind.
+template <int E>
+__device__ __forceinline__ void left_align(float (&v)[E], int by) {
+#pragma unroll
+    for (int s = E / 2; s >= 1; s >>= 1)
+#pragma unroll
+        for (int e = 0; e < E; e++) v[e] = (by & s) ? (e + s < E ? v[e + s] : 0.f) : v[e];
+}
+
+// Columns [col, col + 4) of a row of N, streaming, as far as they lie in it.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void store_piece(float* row, int col, int N, f32x4 v) {
+    if (col + 4 <= N) {
+        __builtin_nontemporal_store(v, reinterpret_cast<f32x4u*>(row + col));
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (col + i < N) __builtin_nontemporal_store(v[i], row + col + i);
+    }
+}
+
 template <typename T, int E>
 __device__ __forceinline__ void fma_pack(float (&acc)[E], float a, const Pack<T, E>& b) {
 #pragma unroll
     for (int e = 0; e < E; e++) acc[e] = __builtin_fmaf(a, to_f32(b.v[e]), acc[e]);
+}
+
+// Stores a slot's sums of one row (lane g holds columns `col` ..; lanes of
+// `mine` write).  Every lane of the slot calls it.
+template <int E, bool kRagged>
+__device__ __forceinline__ void store_sums(float* row, float (&acc)[E], int lane, int g, int col, int chunk_col, int cl,
+                                           int N, bool mine) {
+    if constexpr (kRagged) left_align<E>(acc, max(col + E - N, 0));
+    if constexpr (E == 8) {
+        const LinePieces lp = line_pieces<E>(acc, lane, g, cl);
+        if (mine && g < cl) {
+            if constexpr (kRagged) {
+                store_piece(row, chunk_col + 4 * g, N, lp.p0);
+                store_piece(row, chunk_col + 4 * (g + cl), N, lp.p1);
+            } else {
+                store_line_pieces(row, chunk_col, N, g, cl, lp);
+            }
+        }
+    } else if constexpr (kRagged) {
+        if (mine && g < cl) store_piece(row, col, N, f32x4{acc[0], acc[1], acc[2], acc[3]});
+    } else {
+        if (mine && g < cl && col < N) store_row<E>(row + col, acc);
+    }
 }
 
 struct RowArgs {
@@ -165,13 +239,13 @@ struct RowArgs {
 // columns [col, col + E).  Column indices and values are fetched 64 at a
 // time with one coalesced load and handed to the slots with ds_bpermute (or
 // v_readlane when one slot spans the whole wavefront).
-template <typename T, int E, bool kOneSlot>
+template <typename T, int E, bool kRagged, bool kOneSlot>
 __device__ __forceinline__ void accumulate_span(float (&acc)[E], int beg, int end, const RowArgs& a,
                                                 __amdgpu_buffer_rsrc_t rcol, __amdgpu_buffer_rsrc_t rval,
                                                 __amdgpu_buffer_rsrc_t rB, int col, bool colok, int lane, int slot,
                                                 int logS) {
     const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
-    const uint32_t colbytes = static_cast<uint32_t>(col) * sizeof(T);
+    const uint32_t colbytes = static_cast<uint32_t>(kRagged ? min(col, a.N - E) : col) * sizeof(T);
     // Indices and values of the first chunk of 64; each chunk's loop below
     // first issues the loads of the next chunk, so they travel while the B
     // rows of this one are gathered.
@@ -201,7 +275,7 @@ __device__ __forceinline__ void accumulate_span(float (&acc)[E], int beg, int en
                     av[u] = __shfl(mya, idx & 63);
                     ok = idx < n && colok;
                 }
-                bv[u] = load_pack<T, E>(rB, ok ? static_cast<uint32_t>(c) * rowbytes + colbytes : kOob);
+                bv[u] = load_b<T, E, kRagged>(rB, a.B, static_cast<uint32_t>(c) * rowbytes + colbytes, ok);
             }
 #pragma unroll
             for (int u = 0; u < kRowUnroll; u++) fma_pack<T, E>(acc, av[u], bv[u]);
@@ -211,8 +285,9 @@ __device__ __forceinline__ void accumulate_span(float (&acc)[E], int beg, int en
     }
 }
 
-template <typename T, int E>
+template <typename T, int E, bool kRagged = false>
 __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
+    static_assert(!kRagged || E * sizeof(T) == 16, "ragged rows take whole vectors");
     __shared__ float red[kRowWaves][64 * E];  // wide rows: one partial row chunk per wavefront
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -229,7 +304,8 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
     const int logS = 6 - a.logG;
     const int slot = lane >> a.logG;
     const int g = lane & ((1 << a.logG) - 1);
-    const int col = (chunk * a.chunk_lanes + g) * E;
+    const int chunk_col = chunk * a.chunk_lanes * E;
+    const int col = chunk_col + g * E;
     const bool colok = g < a.chunk_lanes && col < a.N;
     const int4 t = a.tasks[tid];
     float acc[E];
@@ -242,18 +318,32 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
         // differ by its count less one they are consecutive and, with one
         // column chunk, their C rows are one contiguous range: cleared 16
         // bytes per lane, 1 KiB per store instruction.
-        if (a.col_chunks == 1 && (a.N & 3) == 0) {
+        if (a.col_chunks == 1 && (kRagged || (a.N & 3) == 0)) {
             const int r0 = a.perm[t.x];
             if (a.perm[t.x + t.y - 1] - r0 == t.y - 1) {
-                f32x4* const base = reinterpret_cast<f32x4*>(a.C + static_cast<size_t>(r0) * a.N);
-                const int n4 = t.y * (a.N >> 2);
+                float* const base = a.C + static_cast<size_t>(r0) * a.N;
                 const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-                for (int o = lane; o < n4; o += 64) __builtin_nontemporal_store(z, base + o);
+                if constexpr (kRagged) {
+                    const int n = t.y * a.N;
+                    for (int o = 4 * lane; o < n; o += 256) store_piece(base, o, n, z);
+                } else {
+                    const int n4 = t.y * (a.N >> 2);
+                    for (int o = lane; o < n4; o += 64) __builtin_nontemporal_store(z, reinterpret_cast<f32x4*>(base) + o);
+                }
                 return;
             }
         }
         const int step = 1 << logS;
-        if constexpr (E == 8) {
+        if constexpr (kRagged) {
+            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            const int c0 = chunk * a.chunk_lanes * E;
+            if (g < a.chunk_lanes)
+                for (int r = slot; r < t.y; r += step) {
+                    float* dst = a.C + static_cast<size_t>(a.perm[t.x + r]) * a.N;
+#pragma unroll
+                    for (int e = 0; e < E / 4; e++) store_piece(dst, c0 + 4 * (g + e * a.chunk_lanes), a.N, z);
+                }
+        } else if constexpr (E == 8) {
             // 32 bytes per lane: lane g clears 16-byte pieces g and g + chunk
             // lanes of the chunk, so each store instruction covers whole
             // 128-byte lines (store_row's two halves per lane would leave
@@ -285,7 +375,7 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
             len = a.rowptr[row + 1] - beg;
         }
         const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
-        const uint32_t colbytes = static_cast<uint32_t>(col) * sizeof(T);
+        const uint32_t colbytes = static_cast<uint32_t>(kRagged ? min(col, a.N - E) : col) * sizeof(T);
         for (int p0 = 0; p0 < t.y; p0 += S) {
             int nrow = -1, nbeg = 0, nlen = 0;
             if (p0 + S + slot < t.y) {
@@ -306,19 +396,13 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
                 }
 #pragma unroll
                 for (int u = 0; u < kRowUnroll; u++)
-                    bv[u] = load_pack<T, E>(rB, j + u < len && colok ? static_cast<uint32_t>(c[u]) * rowbytes + colbytes
-                                                                     : kOob);
+                    bv[u] = load_b<T, E, kRagged>(rB, a.B, static_cast<uint32_t>(c[u]) * rowbytes + colbytes,
+                                                  j + u < len && colok);
 #pragma unroll
                 for (int u = 0; u < kRowUnroll; u++) fma_pack<T, E>(acc, av[u], bv[u]);
             }
-            if constexpr (E == 8) {
-                const LinePieces lp = line_pieces<E>(acc, lane, g, a.chunk_lanes);
-                if (row >= 0 && g < a.chunk_lanes)
-                    store_line_pieces(a.C + static_cast<size_t>(row) * a.N, chunk * a.chunk_lanes * 8, a.N, g,
-                                      a.chunk_lanes, lp);
-            } else {
-                if (row >= 0 && colok) store_row<E>(a.C + static_cast<size_t>(row) * a.N + col, acc);
-            }
+            store_sums<E, kRagged>(a.C + static_cast<size_t>(max(row, 0)) * a.N, acc, lane, g, col, chunk_col, a.chunk_lanes,
+                                   a.N, row >= 0);
             row = nrow;
             beg = nbeg;
             len = nlen;
@@ -328,9 +412,9 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
 
     // row / seg: all slots on one span
     if (a.logG == 6)
-        accumulate_span<T, E, true>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
+        accumulate_span<T, E, kRagged, true>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
     else
-        accumulate_span<T, E, false>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
+        accumulate_span<T, E, kRagged, false>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
     for (int off = 1 << a.logG; off < 64; off <<= 1)
 #pragma unroll
         for (int e = 0; e < E; e++) acc[e] += __shfl_xor(acc[e], off);
@@ -347,24 +431,13 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
 #pragma unroll
         for (int e = 0; e < E; e++)
             acc[e] = ((red[0][g * E + e] + red[1][g * E + e]) + red[2][g * E + e]) + red[3][g * E + e];
-        if constexpr (E == 8) {
-            const LinePieces lp = line_pieces<E>(acc, lane, g, a.chunk_lanes);
-            if (slot == 0 && g < a.chunk_lanes)
-                store_line_pieces(a.C + static_cast<size_t>(t.x) * a.N, chunk * a.chunk_lanes * 8, a.N, g, a.chunk_lanes,
-                                  lp);
-        } else {
-            if (slot == 0 && colok) store_row<E>(a.C + static_cast<size_t>(t.x) * a.N + col, acc);
-        }
+        store_sums<E, kRagged>(a.C + static_cast<size_t>(t.x) * a.N, acc, lane, g, col, chunk_col, a.chunk_lanes, a.N,
+                               slot == 0);
         return;
     }
     float* const dst_row = t.w == 0 ? a.C + static_cast<size_t>(t.x) * a.N
                                     : a.partials + static_cast<size_t>(t.w >> 2) * a.N;  // seg: partial row of slot t.w >> 2
-    if constexpr (E == 8) {
-        const LinePieces lp = line_pieces<E>(acc, lane, g, a.chunk_lanes);
-        if (slot == 0 && g < a.chunk_lanes) store_line_pieces(dst_row, chunk * a.chunk_lanes * 8, a.N, g, a.chunk_lanes, lp);
-    } else {
-        if (slot == 0 && colok) store_row<E>(dst_row + col, acc);
-    }
+    store_sums<E, kRagged>(dst_row, acc, lane, g, col, chunk_col, a.chunk_lanes, a.N, slot == 0);
 }
 
 // Lanes of seg_finalize_kernel per partial row: four columns each, a power
@@ -407,14 +480,24 @@ __global__ __launch_bounds__(256) void seg_finalize_kernel(const int4* __restric
                 for (int u = 0; u < 8; u++) s += v[u];
             }
             for (; k < k1; k++) s += src[k * stride];
-        } else {  // this thread's columns [col, col + 4) only
+        } else if (col + 4 <= N) {  // rows at any 4 bytes
+            const float* src = partials + static_cast<size_t>(lr.y) * N + col;
+            int k = k0;
+            for (; k + 8 <= k1; k += 8) {
+                f32x4 v[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[u] = *reinterpret_cast<const f32x4u*>(src + static_cast<size_t>(k + u) * N);
+#pragma unroll
+                for (int u = 0; u < 8; u++) s += v[u];
+            }
+            for (; k < k1; k++) s += *reinterpret_cast<const f32x4u*>(src + static_cast<size_t>(k) * N);
+        } else {  // this thread's columns [col, N) only
             const float* src = partials + static_cast<size_t>(lr.y) * N + col;
             for (int k = k0; k < k1; k++) {
                 const float* r = src + static_cast<size_t>(k) * N;
                 s.x += r[0];
                 if (col + 1 < N) s.y += r[1];
                 if (col + 2 < N) s.z += r[2];
-                if (col + 3 < N) s.w += r[3];
             }
         }
     }

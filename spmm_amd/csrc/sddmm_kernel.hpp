@@ -29,16 +29,6 @@ struct SddmmArgs {
     uint32_t batches;  // 64-nonzero batches per wavefront
 };
 
-// E elements of T at element alignment (one load; rows of any width and bases
-// at any element stay on the vector path).
-template <typename T, int E>
-__device__ __forceinline__ Pack<T, E> load_elems(const T* p) {
-    struct __attribute__((packed, aligned(sizeof(T)))) U {
-        T v[E];
-    };
-    return __builtin_bit_cast(Pack<T, E>, *reinterpret_cast<const U*>(p));
-}
-
 // Partner's value within 8 lanes: 7 - lane, lane ^ 2, lane ^ 1.
 template <int kCtrl>
 __device__ __forceinline__ float dpp_swap(float x) {
@@ -135,10 +125,10 @@ __global__ __launch_bounds__(64 * kSddmmWaves, 4) void sddmm_kernel(SddmmArgs a)
             acc[u] += static_cast<double>(E == 8 ? t[0] + t[E / 8] : t[0]);
         };
         auto load_b = [&](int u, int at) {
-            return load_elems<T, E>(reinterpret_cast<const T*>(static_cast<const char*>(a.B) +
+            return load_unaligned<T, E>(reinterpret_cast<const T*>(static_cast<const char*>(a.B) +
                                                                (brow[u] + static_cast<uint32_t>(at) * sizeof(T))));
         };
-        auto load_g = [&](int u, int at) { return load_elems<float, E>(a.G + static_cast<size_t>(grow[u]) * N + at); };
+        auto load_g = [&](int u, int at) { return load_unaligned<float, E>(a.G + static_cast<size_t>(grow[u]) * N + at); };
         auto piece = [&](int at, int skip) {  // columns [at, at + E), the first `skip` of them not counted
             Pack<T, E> b[L];
             const Pack<float, E> g = load_g(0, at);

@@ -242,7 +242,7 @@ thread_local hipEvent_t g_phase_ev[2] = {nullptr, nullptr};
             hipLaunchKernelGGL(kernel, grid, block, shm, stream, __VA_ARGS__);                                  \
     } while (0)
 
-template <typename T, int E>
+template <typename T, int E, bool kRagged = false>
 void launch_rows_t(const tca_spmm_plan* p, const void* val, const void* B, float* C, float* W, hipStream_t s) {
     RowArgs a;
     a.tasks = p->d_tasks;
@@ -263,7 +263,7 @@ void launch_rows_t(const tca_spmm_plan* p, const void* val, const void* B, float
     a.colidx_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * 4);
     a.val_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * sizeof(T));
     a.B_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->K) * p->N * sizeof(T));
-    TCA_PHASE_LAUNCH((row_kernel<T, E>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
+    TCA_PHASE_LAUNCH((row_kernel<T, E, kRagged>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
 }
 
 // Adds the segments of long rows (after the row kernel, same stream).
@@ -275,6 +275,10 @@ void launch_finalize(const tca_spmm_plan* p, float* C, const float* W, hipStream
 
 template <typename T>
 int launch_rows_e(const tca_spmm_plan* p, const void* val, const void* B, float* C, float* W, hipStream_t s) {
+    if (p->rows.ragged) {
+        launch_rows_t<T, 16 / sizeof(T), true>(p, val, B, C, W, s);
+        return TCA_OK;
+    }
     switch (p->rows.elems_per_lane) {
         case 1: launch_rows_t<T, 1>(p, val, B, C, W, s); return TCA_OK;
         case 2: launch_rows_t<T, 2>(p, val, B, C, W, s); return TCA_OK;
@@ -1877,9 +1881,17 @@ int tca_spmm_plan_destroy(tca_spmm_plan* plan) {
 }
 
 // Operand checks of tca_spmm_run (p non-NULL, M > 0).
+// Bytes B must be aligned to: the plan's vector, for ragged rows (which read
+// vectors at any element) the widest that divides N.
+static size_t b_align(const tca_spmm_plan* p) {
+    int e = p->rows.elems_per_lane;
+    while (e > 1 && p->N % e != 0) e >>= 1;
+    return static_cast<size_t>(e) * dtype_size(p->dtype);
+}
+
 static int check_run_operands(const tca_spmm_plan* p, const void* d_val, const void* d_B, const float* d_C) {
     if ((p->nnz > 0 && (!d_val || !d_B)) || !d_C) return fail(TCA_ERR_INVALID, "NULL device pointer");
-    const size_t vb = static_cast<size_t>(p->rows.elems_per_lane) * dtype_size(p->dtype);
+    const size_t vb = b_align(p);
     if (reinterpret_cast<uintptr_t>(d_B) % vb != 0)
         return fail(TCA_ERR_INVALID, "B must be aligned to %zu bytes", vb);
     if (reinterpret_cast<uintptr_t>(d_C) % 16 != 0) return fail(TCA_ERR_INVALID, "C must be aligned to 16 bytes");
@@ -1907,7 +1919,7 @@ int tca_spmm_run_static(const tca_spmm_plan* p, const void* d_val, const void* d
     if (!p) return fail(TCA_ERR_INVALID, "plan is NULL");
     if (p->M == 0) return TCA_OK;
     if ((p->nnz > 0 && (!d_val || !d_B)) || !d_C) return fail(TCA_ERR_INVALID, "NULL device pointer");
-    const size_t vb = static_cast<size_t>(p->rows.elems_per_lane) * dtype_size(p->dtype);
+    const size_t vb = b_align(p);
     if (reinterpret_cast<uintptr_t>(d_B) % vb != 0)
         return fail(TCA_ERR_INVALID, "B must be aligned to %zu bytes", vb);
     if (reinterpret_cast<uintptr_t>(d_C) % 16 != 0) return fail(TCA_ERR_INVALID, "C must be aligned to 16 bytes");
