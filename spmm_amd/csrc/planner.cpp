@@ -54,7 +54,7 @@ void plan_geometry(int32_t N, int32_t es, int32_t slices, RowPlan* p) {
     p->log_lanes = ilog2(next_pow2(p->chunk_lanes));
 }
 
-void plan_row_params(int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan* p) {
+void plan_row_params(int32_t M, int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan* p) {
     plan_geometry(N, es, slices, p);
     const int32_t slots = 64 >> p->log_lanes;
     // Work per wavefront task: about nnz / 32768 nonzeros (four resident
@@ -76,14 +76,27 @@ void plan_row_params(int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan
     const char* w = std::getenv("TCA_WIDE");
     p->wide_len = static_cast<int32_t>((w && std::atoi(w) == 0) ? target : 4 * target);
     p->seg_len = static_cast<int32_t>(target);
-    // Short rows share a wavefront, one slot each, when slots > 1.
+    // Short rows share a wavefront, one slot each, when slots > 1: rows of up
+    // to 2 slots nonzeros.  With 16 slots and more a slot walks its row in
+    // steps of eight nonzeros while most of the chip is idle unless there are
+    // many rows (a wavefront per row takes about 1 us per 2000 rows, four
+    // passes of slots about 0.75 us per nonzero of their longest row), so the
+    // limit follows the number of rows, at most 32.  us per product on the
+    // MI355X at limits of 8 / 16 / 32 / 64 / 128 nonzeros: R-MAT of 10,000
+    // nodes, 110,000 nonzeros, fp16 N = 8 5.9 / 6.1 / 9.0 / 9.9 / 20.2, N = 16
+    // 6.0 / 7.8 / 13.8 / 15.4 / -; 20,000 rows of 9 to 15, fp16 N = 16 18.5 at 8,
+    // 8.8 at 64; R-MAT of 400,000 nodes, 13M, fp16 N = 8 149 / 129 / 118 / 119 /
+    // 164, fp32 N = 8 133 / 119 / 118 / 121 / -; 8192 x 8192 lognormal layer of
+    // 10 %, N = 1: 22.2 / 22.1 / 22.2 / 24.7 / 50.3.
     p->multi_max = slots > 1 ? 2 * slots : -1;
+    if (slots >= 16)
+        p->multi_max = static_cast<int32_t>(std::clamp<int64_t>(std::min<int64_t>(M, nnz / 8) / 600, 4, 32));
     if (const char* s = std::getenv("TCA_MULTI")) p->multi_max = slots > 1 ? std::atoi(s) : -1;
 }
 
 void plan_rows(const int32_t* rowptr, int32_t M, int32_t N, int32_t es, const std::vector<uint8_t>& skip,
                int32_t slices, RowPlan* p) {
-    plan_row_params(rowptr[M], N, es, slices, p);
+    plan_row_params(M, rowptr[M], N, es, slices, p);
     const int32_t slots = 64 >> p->log_lanes;
 
     std::vector<int32_t> rows;

@@ -146,7 +146,7 @@ void plan_geometry(int32_t N, int32_t es, int32_t slices, RowPlan* p);
 
 // Lane geometry and task-length thresholds (row_len, wide_len, seg_len,
 // multi_max) of the row kernel for a matrix of nnz nonzeros.
-void plan_row_params(int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan* p);
+void plan_row_params(int32_t M, int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan* p);
 
 // Row panels with B rows staged in LDS (the panel kernel).  Rows are taken
 // longest first (ties by row id) in panels of R = waves * 4 * rpg rows; the

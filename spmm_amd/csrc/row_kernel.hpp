@@ -285,7 +285,50 @@ __device__ __forceinline__ void accumulate_span(float (&acc)[E], int beg, int en
     }
 }
 
-template <typename T, int E, bool kRagged = false>
+// The same for S = 16, 32 or 64 slots (narrow rows of B): a chunk of 8 S
+// nonzeros, S / 8 index and value registers per lane, so that all eight loads
+// of a lane have a nonzero (chunks of 64 leave all but 64 / S of them idle);
+// with 64 slots every lane keeps its own nonzeros and nothing is shuffled.
+// Slot s takes the same nonzeros in the same order as above.
+template <typename T, int E, bool kRagged, int S>
+__device__ __forceinline__ void accumulate_narrow(float (&acc)[E], int beg, int end, const RowArgs& a,
+                                                  __amdgpu_buffer_rsrc_t rcol, __amdgpu_buffer_rsrc_t rval,
+                                                  __amdgpu_buffer_rsrc_t rB, int col, bool colok, int lane, int slot) {
+    constexpr int R = S * kRowUnroll / 64;
+    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
+    const uint32_t colbytes = static_cast<uint32_t>(kRagged ? min(col, a.N - E) : col) * sizeof(T);
+    int c[R];
+    float v[R];
+    auto fetch = [&](int base) {
+#pragma unroll
+        for (int q = 0; q < R; q++) {
+            const int j = base + 64 * q + lane;
+            c[q] = load_idx(rcol, j, j < end);
+            v[q] = load_val<T>(rval, j, j < end);
+        }
+    };
+    fetch(beg);
+    for (int base = beg; base < end; base += 64 * R) {
+        Pack<T, E> bv[kRowUnroll];
+        float av[kRowUnroll];
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; u++) {
+            const int q = u * S / 64, from = u * S % 64 + slot;  // register and lane of nonzero u S + slot
+            const int cu = S == 64 ? c[q] : __shfl(c[q], from);
+            av[u] = S == 64 ? v[q] : __shfl(v[q], from);
+            bv[u] = load_b<T, E, kRagged>(rB, a.B, static_cast<uint32_t>(cu) * rowbytes + colbytes,
+                                          base + u * S + slot < end && colok);
+        }
+        if (base + 64 * R < end) fetch(base + 64 * R);
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; u++) fma_pack<T, E>(acc, av[u], bv[u]);
+    }
+}
+
+// kNarrow: at least 16 slots (logG <= 2).  An instance of its own: the narrow
+// spans' registers would cost the wide ones occupancy (fp32 65 -> 79, 16-bit
+// 64 -> 94 VGPRs).
+template <typename T, int E, bool kRagged, bool kNarrow>
 __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
     static_assert(!kRagged || E * sizeof(T) == 16, "ragged rows take whole vectors");
     __shared__ float red[kRowWaves][64 * E];  // wide rows: one partial row chunk per wavefront
@@ -411,10 +454,18 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
     }
 
     // row / seg: all slots on one span
-    if (a.logG == 6)
+    if constexpr (kNarrow) {
+        if (a.logG == 0)
+            accumulate_narrow<T, E, kRagged, 64>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
+        else if (a.logG == 1)
+            accumulate_narrow<T, E, kRagged, 32>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
+        else
+            accumulate_narrow<T, E, kRagged, 16>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
+    } else if (a.logG == 6) {
         accumulate_span<T, E, kRagged, true>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
-    else
+    } else {
         accumulate_span<T, E, kRagged, false>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
+    }
     for (int off = 1 << a.logG; off < 64; off <<= 1)
 #pragma unroll
         for (int e = 0; e < E; e++) acc[e] += __shfl_xor(acc[e], off);

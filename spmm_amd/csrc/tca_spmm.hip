@@ -263,7 +263,10 @@ void launch_rows_t(const tca_spmm_plan* p, const void* val, const void* B, float
     a.colidx_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * 4);
     a.val_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * sizeof(T));
     a.B_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->K) * p->N * sizeof(T));
-    TCA_PHASE_LAUNCH((row_kernel<T, E, kRagged>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
+    if (a.logG <= 2)
+        TCA_PHASE_LAUNCH((row_kernel<T, E, kRagged, true>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
+    else
+        TCA_PHASE_LAUNCH((row_kernel<T, E, kRagged, false>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
 }
 
 // Adds the segments of long rows (after the row kernel, same stream).
@@ -1387,7 +1390,7 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         p->device_planned = true;
         p->mfma.row_mfma.clear();
         if (hipGetDevice(&p->device) != hipSuccess) return fail(TCA_ERR_HIP, "no HIP device");
-        plan_row_params(nnz, N, static_cast<int32_t>(dtype_size(dtype)), default_slices(K, N, dtype), &p->rows);
+        plan_row_params(M, nnz, N, static_cast<int32_t>(dtype_size(dtype)), default_slices(K, N, dtype), &p->rows);
         const int group = multi_group_rows(64 >> p->rows.log_lanes);  // rows per multi task
         hipStream_t s = static_cast<hipStream_t>(stream);
 
