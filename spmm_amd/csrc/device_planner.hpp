@@ -33,13 +33,16 @@
 namespace tca {
 
 // CSR checks of tca_csr_validate: rowptr[0] == 0, rowptr[M] == nnz,
-// non-decreasing, columns in [0, K) and strictly ascending within a row.
+// non-decreasing, columns in [0, K) and strictly ascending within a row.  Both
+// copy what they check to the plan (`copy`).
 // err bit 1: row offsets, bit 2: a column.  `start` marks the first entry of
 // every non-empty row (nnz + 1 bytes, zeroed by the caller).
 __global__ void dp_check_rows_kernel(const int* __restrict__ rowptr, int M, int nnz, uint8_t* __restrict__ start,
-                                     int* __restrict__ err) {
+                                     int* __restrict__ err, int* __restrict__ copy) {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < M; r += gridDim.x * blockDim.x) {
         const int b = rowptr[r], e = rowptr[r + 1];
+        copy[r] = b;
+        if (r == M - 1) copy[M] = e;
         if ((r == 0 && b != 0) || (r == M - 1 && e != nnz) || b > e || b < 0 || e > nnz) {
             atomicOr(err, 1);
             continue;
@@ -49,9 +52,10 @@ __global__ void dp_check_rows_kernel(const int* __restrict__ rowptr, int M, int 
 }
 
 __global__ void dp_check_cols_kernel(const int* __restrict__ colidx, int nnz, int K, const uint8_t* __restrict__ start,
-                                     int* __restrict__ err) {
+                                     int* __restrict__ err, int* __restrict__ copy) {
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < nnz; j += gridDim.x * blockDim.x) {
         const int c = colidx[j];
+        copy[j] = c;
         if (c < 0 || c >= K || (j + 1 < nnz && !start[j + 1] && colidx[j + 1] <= c)) atomicOr(err, 2);
     }
 }
@@ -84,6 +88,127 @@ __global__ void dp_bounds_kernel(const uint32_t* __restrict__ len, int M, int wi
         else hi = mid;
     }
     out[k] = lo;
+}
+
+// The row order of up to kSmallSortRows rows in one launch: keys, stable
+// descending sort and bounds (dp_lengths_kernel, a radix sort and
+// dp_bounds_kernel together: 11 launches, 52 us at 20,000 rows and gaps
+// between them; here 38 us).  One workgroup: wavefront w owns the w-th sixteenth of the
+// rows, counts its keys in bins of its own (keys of 511 and more share one),
+// the bins are summed over keys (descending) and wavefronts, and each
+// wavefront then places its rows in order, 64 at a time, equal keys of the 64
+// ranked by ballots.  The rows of the shared bin come first and are ranked by
+// comparing all of them; with more than kSmallSortLong of them *over is set
+// and nothing is written (the caller sorts them the general way).
+constexpr int kSmallSortRows = 65536, kSmallSortBins = 512, kSmallSortLong = 2048;
+
+__global__ __launch_bounds__(1024) void dp_sort_small_kernel(const int* __restrict__ rowptr, int M,
+                                                             const int* __restrict__ wmap,
+                                                             const uint8_t* __restrict__ in_panel, int wide_len,
+                                                             int row_len, int multi_max, uint32_t* __restrict__ keys,
+                                                             int* __restrict__ rows, int* __restrict__ bounds,
+                                                             int* __restrict__ over) {
+    __shared__ int bin[16][kSmallSortBins];
+    __shared__ uint32_t lkey[kSmallSortLong];
+    __shared__ int lrow[kSmallSortLong];
+    __shared__ int nlong, more[4], wsum[16];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int chunk = ((M + 15) / 16 + 63) / 64 * 64;
+    const int r0 = min(M, w * chunk), r1 = min(M, r0 + chunk);
+    auto key_of = [&](int r) {
+        const bool tiles = (wmap && wmap[r / kDmaWinRows] >= 0) || (in_panel && in_panel[r]);
+        return tiles ? 0u : static_cast<uint32_t>(rowptr[r + 1] - rowptr[r]) + 1u;
+    };
+    for (int i = t; i < 16 * kSmallSortBins; i += 1024) (&bin[0][0])[i] = 0;
+    if (t == 0) nlong = 0;
+    if (t < 4) more[t] = 0;
+    __syncthreads();
+    const int th[4] = {wide_len, row_len, max(multi_max, 0), 0};
+    int n[4] = {0, 0, 0, 0};
+    constexpr int kAhead = 8;  // rows loaded at a time
+    for (int rb = r0 + lane; rb < r1; rb += 64 * kAhead) {
+        uint32_t ks[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) ks[u] = rb + 64 * u < r1 ? key_of(rb + 64 * u) : 0u;
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            const int r = rb + 64 * u;
+            if (r >= r1) break;
+            const uint32_t k = ks[u];
+            atomicAdd(&bin[w][min(k, kSmallSortBins - 1u)], 1);
+#pragma unroll
+            for (int q = 0; q < 4; q++) n[q] += static_cast<int64_t>(k) - 1 > th[q];
+            if (k >= kSmallSortBins - 1u) {
+                const int at = atomicAdd(&nlong, 1);
+                if (at < kSmallSortLong) {
+                    lkey[at] = k;
+                    lrow[at] = r;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        if (n[q]) atomicAdd(&more[q], n[q]);
+    __syncthreads();
+    if (nlong > kSmallSortLong) {  // (uniform)
+        if (t == 0) *over = 1;
+        return;
+    }
+    if (t < 4) bounds[t] = more[t];
+    // bins to first positions: thread t has key kSmallSortBins - 1 - t
+    int sum = 0;
+    if (t < kSmallSortBins)
+        for (int v = 0; v < 16; v++) sum += bin[v][kSmallSortBins - 1 - t];
+    int pre = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int x = __shfl_up(pre, d);
+        if (lane >= d) pre += x;
+    }
+    if (lane == 63) wsum[w] = pre;
+    __syncthreads();
+    if (t < kSmallSortBins) {
+        int at = pre - sum;
+        for (int v = 0; v < w; v++) at += wsum[v];
+        for (int v = 0; v < 16; v++) {
+            const int x = bin[v][kSmallSortBins - 1 - t];
+            bin[v][kSmallSortBins - 1 - t] = at;
+            at += x;
+        }
+    }
+    __syncthreads();
+    volatile int* const mine = bin[w];
+    for (int rb = r0; rb < r1; rb += 64 * kAhead) {
+        uint32_t ks[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) ks[u] = rb + 64 * u + lane < r1 ? key_of(rb + 64 * u + lane) : ~0u;
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            const uint32_t k = ks[u];
+            const bool in = k < kSmallSortBins - 1u;
+            uint64_t same = __ballot(in);  // lanes with the same key
+#pragma unroll
+            for (int bit = 1; bit < kSmallSortBins; bit <<= 1) {
+                const uint64_t set = __ballot((k & bit) != 0);
+                same &= k & bit ? set : ~set;
+            }
+            if (in) {
+                const int pos = mine[k] + __popcll(same & ((1ull << lane) - 1));
+                keys[pos] = k;
+                rows[pos] = rb + 64 * u + lane;
+                if ((same >> lane) == 1) mine[k] = pos + 1;  // the last of them
+            }
+        }
+    }
+    for (int e = t; e < nlong; e += 1024) {
+        const uint32_t k = lkey[e];
+        const int r = lrow[e];
+        int pos = 0;
+        for (int f = 0; f < nlong; f++) pos += lkey[f] > k || (lkey[f] == k && lrow[f] < r);
+        keys[pos] = k;
+        rows[pos] = r;
+    }
 }
 
 // segments of each long row (n_long of them, the first in the order)

@@ -86,6 +86,9 @@ struct tca_spmm_plan {
     size_t n_seg_total = 0;   // their segments (rows of d_partials)
     int32_t n_perm = 0;       // rows in multi tasks (entries of d_perm)
     bool device_planned = false;
+    // Planned on the GPU: the structure (d_rowptr, d_colidx) and the row
+    // tables (d_tasks, d_longrows, d_perm) are one allocation each.
+    void *d_struct = nullptr, *d_tables = nullptr;
     float* d_partials = nullptr;
     // row panels (panel kernel)
     PanelPlan panels;
@@ -171,12 +174,17 @@ void free_plan_device(tca_spmm_plan* p) {
     (void)hipFree(p->d_zeros);
     (void)hipFree(p->d_soff);
     (void)hipFree(p->d_wstart);
-    (void)hipFree(p->d_rowptr);
-    (void)hipFree(p->d_colidx);
-    (void)hipFree(p->d_tasks);
+    if (p->device_planned) {
+        (void)hipFree(p->d_struct);
+        (void)hipFree(p->d_tables);
+    } else {
+        (void)hipFree(p->d_rowptr);
+        (void)hipFree(p->d_colidx);
+        (void)hipFree(p->d_tasks);
+        (void)hipFree(p->d_perm);
+        (void)hipFree(p->d_longrows);
+    }
     (void)hipFree(p->d_torder);
-    (void)hipFree(p->d_perm);
-    (void)hipFree(p->d_longrows);
     (void)hipFree(p->d_partials);
     (void)hipFree(p->d_windows);
     (void)hipFree(p->d_ucols);
@@ -1163,6 +1171,8 @@ struct DevPanelPlanner {
         const int32_t es = static_cast<int32_t>(dtype_size(p->dtype));
         E = panel_elems(p->N, es);
         if (!panel_route(p->K, p->N, p->dtype, p->flags, &route) || E == 0 || p->M == 0 || n_nz_rows == 0) return TCA_OK;
+        // all the nonzeros together are too few: no need for the unions
+        if (!route.force && p->nnz < route.min_nnz) return TCA_OK;
         // (the union kernel's column chunks end below c0 + 2^19: K leaves room for them in an int)
         if (p->K > INT_MAX - 32 * kDppChunkWords) return fail(TCA_ERR_UNSUPPORTED, "K too large for panels planned on the GPU");
         P = panel_tile_cols(16 * E * es);
@@ -1394,7 +1404,12 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         const int group = multi_group_rows(64 >> p->rows.log_lanes);  // rows per multi task
         hipStream_t s = static_cast<hipStream_t>(stream);
 
-        // temporaries of the planning, freed on every exit
+        // Temporaries of the planning, freed on every exit.  What every plan
+        // needs is one allocation (`work`), as are the plan's structure and
+        // its row tables: a small structure's planning is allocations,
+        // launches and waits (20,000 rows, 270,000 nonzeros, plan, product and
+        // release 319 -> 122 us).
+        char* work = nullptr;
         uint32_t *keys = nullptr, *keys_s = nullptr, *bm = nullptr, *ekeys = nullptr, *ekeys_s = nullptr;
         int *rows = nullptr, *rows_s = nullptr, *cnt = nullptr, *nseg = nullptr, *segoff = nullptr;
         int *wordpre = nullptr, *scnt = nullptr, *wstat = nullptr, *wmap = nullptr, *wgbase = nullptr, *evals = nullptr,
@@ -1406,41 +1421,67 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         int* dpp_rows = nullptr;  // the panels' row order (phase_b reads it after the second sort)
         auto bail = [&](int st) {
             (void)hipStreamSynchronize(s);
-            for (void* q : {(void*)keys, (void*)keys_s, (void*)rows, (void*)rows_s, (void*)cnt, (void*)nseg, (void*)segoff,
-                            (void*)start, tmp, (void*)bm, (void*)ekeys, (void*)ekeys_s, (void*)wordpre, (void*)scnt,
+            for (void* q : {(void*)work, (void*)nseg, (void*)segoff, tmp, (void*)bm, (void*)ekeys, (void*)ekeys_s, (void*)wordpre, (void*)scnt,
                             (void*)wstat, (void*)wmap, (void*)wgbase, (void*)evals, (void*)evals_s, (void*)skey,
                             (void*)skey_s, (void*)sidx, (void*)sidx_s, (void*)dpp_rows})
                 (void)hipFree(q);
             return st;  // on failure `hold` frees the plan
         };
         int st;
+        auto round_up = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
         // The plan owns its copy of the structure (row kernel and SDDMM read it).
-        if ((st = dev_upload(&p->d_rowptr, nullptr, static_cast<size_t>(M) + 1))) return bail(st);
-        if ((st = dev_upload(&p->d_colidx, nullptr, static_cast<size_t>(nnz)))) return bail(st);
-        if (hipMemcpyAsync(p->d_rowptr, d_rowptr, sizeof(int) * (static_cast<size_t>(M) + 1), hipMemcpyDeviceToDevice, s) !=
-                hipSuccess ||
-            (nnz > 0 && hipMemcpyAsync(p->d_colidx, d_colidx, sizeof(int) * static_cast<size_t>(nnz),
-                                       hipMemcpyDeviceToDevice, s) != hipSuccess))
-            return bail(fail(TCA_ERR_HIP, "structure copy failed"));
+        {
+            const size_t rp = round_up(sizeof(int) * (static_cast<size_t>(M) + 1));
+            char* b = nullptr;
+            if ((st = dev_upload(&b, nullptr, rp + sizeof(int) * static_cast<size_t>(nnz)))) return bail(st);
+            p->d_struct = b;
+            p->d_rowptr = reinterpret_cast<int*>(b);
+            if (nnz > 0) p->d_colidx = reinterpret_cast<int*>(b + rp);
+        }
+        // Rows are sorted by length + 1, at most min(K, nnz) + 1.
+        const unsigned key_bits = 32 - __builtin_clz(static_cast<uint32_t>(std::min(K, nnz)) + 1u);
+        size_t sort_bytes = 0;
+        {
+            if (M > kSmallSortRows && rocprim::radix_sort_pairs_desc(nullptr, sort_bytes, keys, keys_s, rows, rows_s,
+                                                                     static_cast<size_t>(M), 0, key_bits, s) != hipSuccess)
+                return bail(fail(TCA_ERR_HIP, "radix sort sizing failed"));
+            const size_t ks = round_up(sizeof(int) * static_cast<size_t>(M));
+            const size_t head = round_up(8 * sizeof(int) + static_cast<size_t>(nnz) + 1);
+            if ((st = dev_upload(&work, nullptr, head + 4 * ks + sort_bytes))) return bail(st);
+            cnt = reinterpret_cast<int*>(work);  // [0..3] bounds, [4] error bits, [5] compaction check,
+                                                 // [6] the small sort had too many long rows
+            start = reinterpret_cast<uint8_t*>(work) + 8 * sizeof(int);
+            keys = reinterpret_cast<uint32_t*>(work + head);
+            keys_s = reinterpret_cast<uint32_t*>(work + head + ks);
+            rows = reinterpret_cast<int*>(work + head + 2 * ks);
+            rows_s = reinterpret_cast<int*>(work + head + 3 * ks);
+            if (hipMemsetAsync(work, 0, head, s) != hipSuccess) return bail(fail(TCA_ERR_HIP, "hipMemsetAsync failed"));
+        }
+        void* sort_tmp = reinterpret_cast<char*>(rows_s) + round_up(sizeof(int) * static_cast<size_t>(M));
         // CSR checks
-        if ((st = dev_upload(&cnt, nullptr, 4))) return bail(st);  // [0..2] bounds, [3] error bits
-        if ((st = dev_upload(&start, nullptr, static_cast<size_t>(nnz) + 1))) return bail(st);
-        if (hipMemsetAsync(cnt, 0, 4 * sizeof(int), s) != hipSuccess ||
-            hipMemsetAsync(start, 0, static_cast<size_t>(nnz) + 1, s) != hipSuccess)
-            return bail(fail(TCA_ERR_HIP, "hipMemsetAsync failed"));
         const dim3 blk(256);
         auto grid_for = [](int64_t n) { return dim3(static_cast<unsigned>(std::min<int64_t>((n + 255) / 256, 65536))); };
         if (M > 0) {
-            hipLaunchKernelGGL(dp_check_rows_kernel, grid_for(M), blk, 0, s, p->d_rowptr, M, nnz, start, cnt + 3);
-            if (nnz > 0) hipLaunchKernelGGL(dp_check_cols_kernel, grid_for(nnz), blk, 0, s, p->d_colidx, nnz, K, start, cnt + 3);
+            hipLaunchKernelGGL(dp_check_rows_kernel, grid_for(M), blk, 0, s, d_rowptr, M, nnz, start, cnt + 4, p->d_rowptr);
+            if (nnz > 0)
+                hipLaunchKernelGGL(dp_check_cols_kernel, grid_for(nnz), blk, 0, s, d_colidx, nnz, K, start, cnt + 4,
+                                   p->d_colidx);
+        } else if (hipMemcpyAsync(p->d_rowptr, d_rowptr, sizeof(int), hipMemcpyDeviceToDevice, s) != hipSuccess) {
+            return bail(fail(TCA_ERR_HIP, "structure copy failed"));
         }
-        int h_cnt[4] = {0, 0, 0, 0};
-        // the columns index the window bitmaps below: validate first
-        if (hipMemcpyAsync(h_cnt, cnt, sizeof h_cnt, hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            return bail(fail(TCA_ERR_HIP, "CSR checks failed"));
-        if (h_cnt[3] & 1) return bail(fail(TCA_ERR_INVALID, "CSR row offsets are not 0 .. nnz non-decreasing"));
-        if (h_cnt[3] & 2) return bail(fail(TCA_ERR_INVALID, "CSR columns out of range or not strictly ascending in a row"));
+        int h_cnt[7] = {};
+        auto read_cnt = [&]() -> int {  // waits; the checks' verdict first
+            if (hipMemcpyAsync(h_cnt, cnt, sizeof h_cnt, hipMemcpyDeviceToHost, s) != hipSuccess ||
+                hipStreamSynchronize(s) != hipSuccess)
+                return fail(TCA_ERR_HIP, "planning kernels failed");
+            if (h_cnt[4] & 1) return fail(TCA_ERR_INVALID, "CSR row offsets are not 0 .. nnz non-decreasing");
+            if (h_cnt[4] & 2) return fail(TCA_ERR_INVALID, "CSR columns out of range or not strictly ascending in a row");
+            return TCA_OK;
+        };
+        // The columns index the window bitmaps and the short-K tiles: wait for
+        // the checks there.  Sorting row lengths needs no valid structure.
+        const bool maybe_mfma = (flags & TCA_PLAN_NO_MFMA) == 0 && dtype != TCA_F32 && N % 8 == 0;
+        if ((maybe_mfma || M == 0) && (st = read_cnt())) return bail(st);
         if (short_route(M, K, nnz, N, dtype, flags)) {
             // short K: every row on the short-K kernel, which needs only the structure
             p->mfma_short = true;
@@ -1592,15 +1633,15 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
                         const size_t nmask = static_cast<size_t>(steps_all) * 8;
                         if ((st = dev_upload(&p->d_amask, nullptr, nmask))) return bail(st);
                         if (hipMemsetAsync(p->d_amask, 0, nmask * 8, s) != hipSuccess ||
-                            hipMemsetAsync(cnt + 3, 0, sizeof(int), s) != hipSuccess)
+                            hipMemsetAsync(cnt + 5, 0, sizeof(int), s) != hipSuccess)
                             return bail(fail(TCA_ERR_HIP, "hipMemsetAsync failed"));
                         auto* mk = reinterpret_cast<unsigned long long*>(p->d_amask);
                         hipLaunchKernelGGL(dm_cmask_kernel, grid_for(nz_take), blk, 0, s, p->d_dn_pos,
                                            static_cast<int>(nz_take), mk);
                         hipLaunchKernelGGL(dm_cfit_kernel, grid_for(steps_all), blk, 0, s, mk, steps_all, kCpCells,
-                                           cnt + 3);
+                                           cnt + 5);
                         int over = 0;
-                        if (hipMemcpyAsync(&over, cnt + 3, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
+                        if (hipMemcpyAsync(&over, cnt + 5, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
                             hipStreamSynchronize(s) != hipSuccess)
                             return bail(fail(TCA_ERR_HIP, "compaction check failed"));
                         if (over == 0) {
@@ -1636,39 +1677,33 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         // leave too (key 0) and the order is sorted again for the row kernel
         DevPanelPlanner dpp;
         dpp.s = s;
-        size_t sort_bytes = 0;
         auto sort_rows = [&](const uint8_t* in_panel) -> int {
-            hipLaunchKernelGGL(dp_lengths_kernel, grid_for(M), blk, 0, s, p->d_rowptr, M,
-                               p->mfma.windows.empty() ? nullptr : wmap, in_panel, keys, rows);
-            size_t tmp_bytes = 0;
-            if (rocprim::radix_sort_pairs_desc(nullptr, tmp_bytes, keys, keys_s, rows, rows_s, static_cast<size_t>(M), 0, 32,
-                                               s) != hipSuccess)
-                return fail(TCA_ERR_HIP, "radix sort sizing failed");
-            if (tmp_bytes > sort_bytes) {
-                (void)hipStreamSynchronize(s);
-                (void)hipFree(tmp);
-                tmp = nullptr;
-                if (dev_malloc(reinterpret_cast<void**>(&tmp), tmp_bytes) != hipSuccess)
-                    return fail(TCA_ERR_ALLOC, "radix sort workspace");
-                sort_bytes = tmp_bytes;
+            const int* const windows = p->mfma.windows.empty() ? nullptr : wmap;
+            if (M <= kSmallSortRows) {
+                hipLaunchKernelGGL(dp_sort_small_kernel, dim3(1), dim3(1024), 0, s, p->d_rowptr, M, windows, in_panel,
+                                   p->rows.wide_len, p->rows.row_len, p->rows.multi_max, keys_s, rows_s, cnt, cnt + 6);
+                const int e = read_cnt();
+                if (e || !h_cnt[6]) return e;
+                if (!tmp) {
+                    if (rocprim::radix_sort_pairs_desc(nullptr, sort_bytes, keys, keys_s, rows, rows_s,
+                                                       static_cast<size_t>(M), 0, key_bits, s) != hipSuccess ||
+                        dev_malloc(&tmp, sort_bytes) != hipSuccess)
+                        return fail(TCA_ERR_ALLOC, "radix sort workspace");
+                    sort_tmp = tmp;
+                }
             }
-            if (rocprim::radix_sort_pairs_desc(tmp, tmp_bytes, keys, keys_s, rows, rows_s, static_cast<size_t>(M), 0, 32, s) !=
-                hipSuccess)
+            hipLaunchKernelGGL(dp_lengths_kernel, grid_for(M), blk, 0, s, p->d_rowptr, M, windows, in_panel, keys, rows);
+            if (rocprim::radix_sort_pairs_desc(sort_tmp, sort_bytes, keys, keys_s, rows, rows_s, static_cast<size_t>(M), 0,
+                                               key_bits, s) != hipSuccess)
                 return fail(TCA_ERR_HIP, "radix sort failed");
             if (Mp > 0)
                 hipLaunchKernelGGL(dp_bounds_kernel, dim3(1), dim3(64), 0, s, keys_s, Mp, p->rows.wide_len, p->rows.row_len,
                                    p->rows.multi_max, cnt);
-            if (hipMemcpyAsync(h_cnt, cnt, sizeof h_cnt, hipMemcpyDeviceToHost, s) != hipSuccess ||
-                hipStreamSynchronize(s) != hipSuccess)
-                return fail(TCA_ERR_HIP, "planning kernels failed");
-            // (cnt[3] held flags before the bounds kernel wrote it; with Mp == 0 it did not run)
-            if (Mp == 0) h_cnt[0] = h_cnt[1] = h_cnt[2] = h_cnt[3] = 0;
+            if (const int e = read_cnt()) return e;
+            if (Mp == 0) h_cnt[0] = h_cnt[1] = h_cnt[2] = h_cnt[3] = 0;  // (the bounds kernel did not run)
             return TCA_OK;
         };
         if (M > 0) {
-            if ((st = dev_upload(&keys, nullptr, M)) || (st = dev_upload(&keys_s, nullptr, M)) ||
-                (st = dev_upload(&rows, nullptr, M)) || (st = dev_upload(&rows_s, nullptr, M)))
-                return bail(st);
             if ((st = sort_rows(nullptr))) return bail(st);
             // Row panels from the first h_cnt[3] rows of the order (rows with
             // nonzeros outside MFMA windows), as plan_panels takes them.
@@ -1721,10 +1756,17 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         p->n_longrows = n_long + dpp.n_plongrows;  // the panels' long rows follow the row kernel's
         p->n_seg_total = static_cast<size_t>(seg_total) + static_cast<size_t>(dpp.n_segments);
         p->n_perm = n_short;
-        if ((st = dev_upload(&p->d_tasks, nullptr, p->ntasks)) || (st = dev_upload(&p->d_perm, nullptr, n_short)) ||
-            (st = dev_upload(&p->d_longrows, nullptr, p->n_longrows)) ||
-            (!(flags & TCA_PLAN_NO_SCRATCH) && (st = dev_upload(&p->d_partials, nullptr, p->n_seg_total * N))))
-            return bail(st);
+        {
+            const size_t nt = static_cast<size_t>(p->ntasks), nl = static_cast<size_t>(p->n_longrows);
+            char* b = nullptr;
+            if ((st = dev_upload(&b, nullptr, sizeof(int4) * (nt + nl) + sizeof(int) * static_cast<size_t>(n_short))))
+                return bail(st);
+            p->d_tables = b;
+            if (nt > 0) p->d_tasks = reinterpret_cast<int4*>(b);
+            if (nl > 0) p->d_longrows = reinterpret_cast<int4*>(b) + nt;
+            if (n_short > 0) p->d_perm = reinterpret_cast<int*>(reinterpret_cast<int4*>(b) + nt + nl);
+        }
+        if (!(flags & TCA_PLAN_NO_SCRATCH) && (st = dev_upload(&p->d_partials, nullptr, p->n_seg_total * N))) return bail(st);
         if (Mp > 0) {
             DpEmitArgs ea;
             ea.rowptr = p->d_rowptr;
