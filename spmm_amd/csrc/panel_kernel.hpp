@@ -70,6 +70,8 @@ struct PanelArgs {
     const void* B;
     float* C;
     float* partials;
+    const float* G;         // sampled product (panel_sddmm_kernel): M x N
+    float* out;             // and its results [nnz]
     int N;
     int chunks;             // column chunks (grid = units * chunks)
     uint32_t pos_bytes, val_bytes;
@@ -521,6 +523,272 @@ __global__ __launch_bounds__(kPnThreads, 1) void panel_kernel(PanelArgs a) {
             float* dst = u.w < 0 ? a.C + static_cast<size_t>(row) * a.N + col0
                                  : a.partials + static_cast<size_t>(u.w + s * nu) * a.N + col0;
             panel_store<T, E>(dst, g, acc[i]);
+        }
+    };
+    if (a.win[u.x]) consume(PnIndex<1>{});
+    else consume(PnIndex<0>{});
+}
+
+// ---------------- sampled product over the same panels ----------------
+//
+// out[j] = <G[row(j), :], B[col(j), :]> for the nonzeros j of the panels, the
+// plan, staging and walk of panel_kernel with one column chunk (N = 16 E).
+// The gathering kernel (sddmm_kernel.hpp) fetches a row of B per nonzero from
+// behind the L2s; here it is staged once per panel.  A group's lane g holds
+// its E columns of the group's four rows of G in registers; step U of a run
+// multiplies them with nonzero U's staged row, the group's 16 partial sums
+// are added in four DPP steps (every lane then holds the same sum) and lane U
+// keeps it; the run's results are stored side by side.  A step issues about
+// half more than the product's (four DPP adds and a select instead of one
+// broadcast).  11.4M nonzeros of an R-MAT graph of 131,072 nodes, N = 128 fp32:
+// 325 us, and 13 us for the rows outside the panels, against 600 us gathered.
+
+// A wavefront's counts of one tile, and the producers: panel_kernel's own, as
+// functions.  (panel_kernel keeps them inline: with these functions its
+// registers are laid out differently, 77 instructions more, and the 115M-edge
+// graph takes 1,583 to 1,597 instead of 1,573 to 1,584 us.)
+__device__ __forceinline__ void pn_read_counts(const char* p, uint32_t (&c)[kPnCntUsed]) {
+    pn_static_for<0, kPnCntUsed / 4>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        const i32x4v v = *reinterpret_cast<const i32x4v*>(p + 16 * j);
+        c[4 * j] = v.x; c[4 * j + 1] = v.y; c[4 * j + 2] = v.z; c[4 * j + 3] = v.w;
+    });
+    constexpr int b = kPnCntUsed / 4 * 4, rem = kPnCntUsed % 4;
+    if constexpr (rem == 1) {
+        c[b] = *reinterpret_cast<const uint32_t*>(p + 4 * b);
+    } else if constexpr (rem == 2) {
+        typedef int i32x2t __attribute__((ext_vector_type(2)));
+        const i32x2t v = *reinterpret_cast<const i32x2t*>(p + 4 * b);
+        c[b] = v.x; c[b + 1] = v.y;
+    } else if constexpr (rem == 3) {
+        typedef int i32x3t __attribute__((ext_vector_type(3)));
+        const i32x3t v = *reinterpret_cast<const i32x3t*>(p + 4 * b);
+        c[b] = v.x; c[b + 1] = v.y; c[b + 2] = v.z;
+    }
+}
+
+// The producer wavefronts of a workgroup (pid = 0 .. kPnProducers - 1).
+template <typename T, int E>
+__device__ __forceinline__ void pn_produce(const PanelArgs& a, const int4& u, int chunk, int pid, int lane, char* smem) {
+    using G = PanelGeom<T, E>;
+    // ---- producers: tile t + 1 into buffer (t + 1) & 1 while tile t is used;
+    // producer pid issues transfers pid, pid + kPnProducers, ... of a tile (and
+    // producer 0 the counts), so each has at most kInstrs / kPnProducers + 1
+    // transfers in flight (a wavefront's vmcnt counts 63 at most)
+    const int piece = lane % (G::kRowBytes / 16);
+    const int sub = lane / (G::kRowBytes / 16);  // row within one 1 KiB transfer
+    constexpr int kRowsPerInstr = 1024 / G::kRowBytes;
+    // B rows of this column chunk, addressed by 32-bit offsets from one
+    // scalar base held in SGPRs.  readfirstlane returns a signed
+    // int: each half goes through uint32_t before widening, so a low half
+    // with bit 31 set is not sign-extended into the high half.
+    const uint64_t bb = reinterpret_cast<uint64_t>(a.B) + static_cast<uint64_t>(chunk) * G::kRowBytes;
+    const uint32_t bb_hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bb >> 32)));
+    const uint32_t bb_lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(bb)));
+    const char* bbase = reinterpret_cast<const char*>((static_cast<uint64_t>(bb_hi) << 32) | bb_lo);
+    const uint32_t lds0 = pn_lds_addr(smem);
+    // A tile's P offsets come through coalesced vector loads, lane l
+    // holding position j * 64 + l in o[j]; each transfer takes its rows'
+    // offsets by readlane.  Positions past P clamp to P - 1 (never staged).
+    constexpr int kOffRegs = (G::kP + 63) / 64;
+    auto load_offs = [&](int tile, uint32_t (&o)[kOffRegs]) {
+        const uint32_t* bo = a.boff + static_cast<size_t>(tile) * G::kP;
+#pragma unroll
+        for (int j = 0; j < kOffRegs; j++) {
+            const int r = j * 64 + lane;
+            o[j] = bo[r < G::kP ? r : G::kP - 1];
+        }
+    };
+    // counts of tile rel + 1 (clamped to the unit's last tile) into count
+    // slot buf; lanes past the counts re-read the first 16 bytes
+    const uint32_t cnt_lane = 16u * static_cast<uint32_t>(lane < kPnCntTileBytes / 16 ? lane : 0);
+    // Every transfer of the tile, whatever its width: columns past the
+    // width repeat the tile's last B row (plan padding) into rows that no
+    // consumer reads, so each producer issues the same number of memory
+    // operations every tile and its waits below are compile-time counts.
+    auto stage = [&](const uint32_t (&o)[kOffRegs], int buf, int rel) {
+        const int tn = u.y + (rel + 1 < u.z ? rel + 1 : rel);
+        if (pid == 0) pn_dma(a.cnt, static_cast<uint32_t>(tn) * kPnCntTileBytes + cnt_lane, lds0 + pn_cnt_off<T, E>(buf));
+#pragma unroll
+        for (int k = 0; k < G::kInstrs; k++) {
+            if (k % kPnProducers == pid) {
+                const int r0 = k * kRowsPerInstr;
+                uint32_t off = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(o[r0 / 64]), r0 % 64));
+#pragma unroll
+                for (int j = 1; j < kRowsPerInstr; j++) {
+                    const uint32_t oj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(o[r0 / 64]), r0 % 64 + j));
+                    off = sub == j ? oj : off;
+                }
+                pn_dma(bbase, off + 16 * piece, lds0 + pn_zrow_off<T, E>(buf) + G::kRowBytes + k * 1024);
+            }
+        }
+    };
+    // Per tile: the transfers of tile t + 1, then the offsets of tile t + 2
+    // (loaded unconditionally, clamped), then a wait that leaves only
+    // those kOffRegs loads in flight (land): the tile has landed, while
+    // the offsets' latency runs on into the next tile period.  After the
+    // barrier only those loads can be in flight: a full wait there, and
+    // the offsets pass through an empty asm (ready), which ends their load
+    // dependence for the compiler -- it cannot see the transfers (inline
+    // asm), and its own wait before each readlane would otherwise also
+    // wait for the transfers issued before it.
+    auto land = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kOffRegs) : "memory"); };
+    static_assert(kOffRegs <= 15, "vmcnt immediate");
+    uint32_t o[kOffRegs];
+    auto ready = [&]() {
+        pn_wait_all();
+#pragma unroll
+        for (int j = 0; j < kOffRegs; j++) asm volatile("" : "+v"(o[j]));
+    };
+    load_offs(u.y, o);
+    ready();
+    stage(o, 0, 0);
+    load_offs(u.y + (u.z > 1 ? 1 : 0), o);
+    land();
+    for (int t = 0; t < u.z; t++) {
+        pn_barrier();
+        if (t + 1 < u.z) {
+            ready();
+            stage(o, (t + 1) & 1, t + 1);
+            load_offs(u.y + (t + 2 < u.z ? t + 2 : t + 1), o);
+            land();
+        }
+    }
+}
+
+template <int kRor>
+__device__ __forceinline__ float pn_ror_add(float x) {
+    return x + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x120 + kRor, 0xf, 0xf, true));
+}
+
+template <typename T, int E, int U>
+__device__ __forceinline__ void pn_dots(float& res, const float (&gr)[E], uint32_t pa, uint32_t lanepart, int g, int m,
+                                        float (&x)[E], float (&y)[E]) {
+    if constexpr (U < 15) {
+        pn_read_at<T, E>(pn_addr<U + 1, false>(pa, lanepart), y);
+        // keeps the read here (otherwise it sinks into the branch that uses it)
+        asm volatile("" ::: "memory");
+    }
+    // chains of four columns, as the gathering kernel's pieces
+    constexpr int H = E < 4 ? E : 4;
+    float t[E / H];
+#pragma unroll
+    for (int h = 0; h < E / H; h++) {
+        t[h] = gr[H * h] * x[H * h];
+#pragma unroll
+        for (int e = 1; e < H; e++) t[h] = __builtin_fmaf(gr[H * h + e], x[H * h + e], t[h]);
+    }
+    float s = t[0];
+    if constexpr (E / H == 2) s += t[1];
+    s = pn_ror_add<1>(pn_ror_add<2>(pn_ror_add<4>(pn_ror_add<8>(s))));
+    res = g == U ? s : res;
+    if constexpr (U < 15) {
+        if (U + 1 < m) pn_dots<T, E, U + 1>(res, gr, pa, lanepart, g, m, y, x);
+    }
+}
+
+template <typename T, int E>
+__global__ __launch_bounds__(kPnThreads, 1) void panel_sddmm_kernel(PanelArgs a) {
+    using G = PanelGeom<T, E>;
+    constexpr int R = kPnWaves * 4 * kPnRpg;
+    __shared__ __attribute__((aligned(16))) char smem[2 * (G::kBufBytes + G::kRowBytes) + 2 * kPnCntSlot];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int unit = a.order[blockIdx.x];
+    if (unit < 0) return;  // idle: every wavefront leaves before the first barrier
+    const int4 u = a.units[unit];
+    if (wave >= kPnWaves) {
+        pn_produce<T, E>(a, u, 0, wave - kPnWaves, lane, smem);
+        return;
+    }
+    // The consumers of panel_kernel, without values: positions where they lie
+    // or through windows, results stored in place of accumulators.
+    auto consume = [&](auto win_tag) {
+        constexpr bool kWin = decltype(win_tag)::value != 0;
+        const int group = lane >> 4;
+        const int g = lane & 15;
+        const __amdgpu_buffer_rsrc_t rpos = make_rsrc(a.pos, a.pos_bytes);
+        const __amdgpu_buffer_rsrc_t rout = make_rsrc(a.out, a.val_bytes);
+        float gr[kPnRpg][E];
+        int cur[kPnRpg];
+#pragma unroll
+        for (int i = 0; i < kPnRpg; i++) {
+            const int s = (wave * kPnRpg + i) * 4 + group;
+            cur[i] = a.ustart[static_cast<size_t>(unit) * R + s];
+            const int row = a.rows[static_cast<size_t>(u.x) * R + s];
+#pragma unroll
+            for (int e = 0; e < E; e++)
+                gr[i][e] = row >= 0 ? a.G[static_cast<size_t>(row) * a.N + pn_col<T, E>(g, e)] : 0.f;
+        }
+        if (wave == 0)
+            for (int o = 16 * lane; o < G::kRowBytes; o += 1024) {
+                *reinterpret_cast<f32x4*>(smem + pn_zrow_off<T, E>(0) + o) = f32x4{0.f, 0.f, 0.f, 0.f};
+                *reinterpret_cast<f32x4*>(smem + pn_zrow_off<T, E>(1) + o) = f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        const int shift = 8 * group;
+        const uint32_t lds0 = pn_lds_addr(smem);
+        const uint32_t lanepart = static_cast<uint32_t>((G::kLaneBytes == 32 ? 16 : G::kLaneBytes) * g);
+        uint32_t cn[kPnCntUsed], cnx[kPnCntUsed];
+        uint32_t wq[kPnRpg], lq[kPnRpg], rq[kPnRpg];
+        int w0[kPnRpg], nnx[kPnRpg];
+        bool nd[kPnRpg];
+        auto fetch = [&](int i, int nn) {
+            const uint32_t k = static_cast<uint32_t>(cur[i] + g);
+            if constexpr (kWin) {
+                const bool need = nn > 0 && cur[i] + nn > w0[i] + 16;
+                rq[i] = static_cast<uint32_t>(
+                    __builtin_amdgcn_ds_bpermute((lane + cur[i] - w0[i]) << 2, static_cast<int>(wq[i])));
+                lq[i] = __builtin_amdgcn_raw_buffer_load_b8(rpos, need ? k : kOob, 0, 0);
+                w0[i] = need ? cur[i] : w0[i];
+                nd[i] = need;
+            } else {
+                lq[i] = __builtin_amdgcn_raw_buffer_load_b8(rpos, g < nn ? k : kOob, 0, 0);
+            }
+            nnx[i] = nn;
+            asm volatile("" ::: "memory");  // loads in the loop's order
+        };
+        pn_read_counts(reinterpret_cast<const char*>(a.cnt) + (static_cast<size_t>(u.y) * kPnWaves + wave) * (kPnCntRows * 4),
+                       cn);
+#pragma unroll
+        for (int i = 0; i < kPnRpg; i++) {
+            wq[i] = 0u;
+            w0[i] = -64;  // empty: the first run with nonzeros loads a window
+            fetch(i, static_cast<int>((cn[i] >> shift) & 255));
+        }
+        for (int t = 0; t < u.z; t++) {
+            pn_barrier();
+            const bool more = t + 1 < u.z;
+            const uint32_t zb = lds0 + pn_zrow_off<T, E>(t & 1);
+            pn_read_counts(smem + pn_cnt_off<T, E>(t & 1) + wave * (kPnCntRows * 4), cnx);
+            uint32_t mxw[(kPnRpg + 3) / 4];  // entries' longest runs (uniform)
+#pragma unroll
+            for (int w = 0; w < (kPnRpg + 3) / 4; w++)
+                mxw[w] = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(cn[kPnMaxDword + w])));
+            pn_static_for<0, kPnRpg>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                const int nmax = static_cast<int>((mxw[i / 4] >> (8 * (i % 4))) & 255);
+                uint32_t qq;
+                if constexpr (kWin) {
+                    wq[i] = nd[i] ? lq[i] : wq[i];
+                    qq = g < nnx[i] ? (nd[i] ? lq[i] : rq[i]) : 0u;
+                } else {
+                    qq = lq[i];
+                }
+                float res = 0.f;
+                if (nmax > 0) {
+                    const uint32_t pa = qq * static_cast<uint32_t>(G::kRowBytes) + zb;
+                    float b0[E], b1[E];
+                    pn_read_at<T, E>(pn_addr<0, true>(pa, lanepart), b0);
+                    pn_dots<T, E, 0>(res, gr[i], pa, lanepart, g, nmax, b0, b1);
+                }
+                // stored whether or not there is a run: the same memory operations every tile
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, res), rout,
+                                                      g < nnx[i] ? 4u * static_cast<uint32_t>(cur[i] + g) : kOob, 0, 0);
+                cur[i] += static_cast<int>((cn[i] >> shift) & 255);
+                fetch(i, more ? static_cast<int>((cnx[i] >> shift) & 255) : 0);
+            });
+#pragma unroll
+            for (int j = 0; j < kPnCntUsed; j++) cn[j] = cnx[j];
         }
     };
     if (a.win[u.x]) consume(PnIndex<1>{});

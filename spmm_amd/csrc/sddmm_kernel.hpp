@@ -27,6 +27,10 @@ struct SddmmArgs {
     int M, N;
     uint32_t nnz;
     uint32_t batches;  // 64-nonzero batches per wavefront
+    const int4* tasks;  // sddmm_tasks_kernel: the row kernel's task list
+    const int* perm;
+    const int4* longrows;
+    int ntasks;
 };
 
 // Partner's value within 8 lanes: 7 - lane, lane ^ 2, lane ^ 1.
@@ -81,7 +85,104 @@ __device__ __forceinline__ int wave_row_of(const int* __restrict__ rowptr, uint3
 // per nonzero (the previous kernel): 25.2 ms on 11.4M nonzeros of an R-MAT
 // graph of 131,072 nodes at N = 128 fp32, 650 us on a 2048 x 2048 layer of
 // 10 % at N = 1024 bf16; now 0.60 ms and 63 us (9.7 and 13.6 TB/s of gathered
-// rows of B).
+// rows of B).  Rows in panels take panel_sddmm_kernel (panel_kernel.hpp), and
+// the others beside them sddmm_tasks_kernel (the spans above, skipping the
+// panels' nonzeros, took 97 us for them: nearly every span holds a few).
+
+// One batch: the sums of the wavefront's 64 nonzeros (lane i: row `row`, column
+// `col`, a row's nonzeros side by side), lane i's own.
+template <typename T, int E, int L>
+__device__ __forceinline__ float sddmm_batch(const SddmmArgs& a, int row, int col, int lane) {
+    const size_t N = static_cast<size_t>(a.N);
+    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
+    const int l = lane & (L - 1), first = lane - l;
+    const int V = (a.N + E - 1) / E;      // pieces of a row
+    const int full = a.N / (E * L) * L;   // pieces of whole piece columns
+    uint32_t brow[L];  // byte offsets of the rows of B (a plan's B is below 4 GiB)
+    int grow[L];
+#pragma unroll
+    for (int u = 0; u < L; u++) {
+        brow[u] = static_cast<uint32_t>(__shfl(col, first + u)) * rowbytes;
+        grow[u] = __shfl(row, first + u);
+    }
+    const bool one_row = __ballot(grow[0] != grow[L - 1]) == 0;  // a row's nonzeros are side by side
+    double acc[L];
+#pragma unroll
+    for (int u = 0; u < L; u++) acc[u] = 0.;
+    auto add = [&](int u, const Pack<float, E>& g, const Pack<T, E>& b, int skip) {
+        float t[(E + 3) / 4];
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            float s = e % 4 == 0 ? g.v[e] * to_f32(b.v[e]) : __builtin_fmaf(g.v[e], to_f32(b.v[e]), t[e / 4]);
+            if (skip > e) s = 0.f;
+            t[e / 4] = s;
+        }
+        acc[u] += static_cast<double>(E == 8 ? t[0] + t[E / 8] : t[0]);
+    };
+    auto load_b = [&](int u, int at) {
+        return load_unaligned<T, E>(reinterpret_cast<const T*>(static_cast<const char*>(a.B) +
+                                                           (brow[u] + static_cast<uint32_t>(at) * sizeof(T))));
+    };
+    auto load_g = [&](int u, int at) { return load_unaligned<float, E>(a.G + static_cast<size_t>(grow[u]) * N + at); };
+    auto piece = [&](int at, int skip) {  // columns [at, at + E), the first `skip` of them not counted
+        Pack<T, E> b[L];
+        const Pack<float, E> g = load_g(0, at);
+#pragma unroll
+        for (int u = 0; u < L; u++) b[u] = load_b(u, at);
+#pragma unroll
+        for (int u = 0; u < L; u++) add(u, g, b[u], skip);
+    };
+    auto piece_rows = [&](int at, int skip) {  // the same, every nonzero with its own row of G
+        constexpr int H = L > 4 ? 4 : L;       // nonzeros loaded at a time (registers)
+#pragma unroll
+        for (int h = 0; h < L; h += H) {
+            Pack<T, E> b[H];
+            Pack<float, E> g[H];
+#pragma unroll
+            for (int u = 0; u < H; u++) {
+                g[u] = load_g(h + u, at);
+                b[u] = load_b(h + u, at);
+            }
+#pragma unroll
+            for (int u = 0; u < H; u++) add(h + u, g[u], b[u], skip);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    const int tail = full + l;  // the last piece of a row that is no whole number of them ends at the row's end
+    const int at = min(tail * E, a.N - E);
+    if (one_row) {
+#pragma unroll(E == 8 ? 1 : 2)
+        for (int p = 0; p < full; p += L) piece((p + l) * E, 0);
+        if (tail < V) piece(at, tail * E - at);
+    } else {
+#pragma unroll 1
+        for (int p = 0; p < full; p += L) piece_rows((p + l) * E, 0);
+        if (tail < V) piece_rows(at, tail * E - at);
+    }
+    float sum[L];
+#pragma unroll
+    for (int u = 0; u < L; u++) sum[u] = static_cast<float>(acc[u]);
+    if constexpr (L == 8) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const float give = l & 4 ? sum[u] : sum[u + 4], keep = l & 4 ? sum[u + 4] : sum[u];
+            sum[u] = keep + dpp_swap<0x141>(give);  // row_half_mirror
+        }
+    }
+    if constexpr (L >= 4) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const float give = l & 2 ? sum[u] : sum[u + 2], keep = l & 2 ? sum[u + 2] : sum[u];
+            sum[u] = keep + dpp_swap<0x4e>(give);  // quad_perm [2, 3, 0, 1]
+        }
+    }
+    if constexpr (L >= 2) {
+        const float give = l & 1 ? sum[0] : sum[1], keep = l & 1 ? sum[1] : sum[0];
+        sum[0] = keep + dpp_swap<0xb1>(give);  // quad_perm [1, 0, 3, 2]
+    }
+    return sum[0];
+}
+
 template <typename T, int E, int L>
 __global__ __launch_bounds__(64 * kSddmmWaves, 4) void sddmm_kernel(SddmmArgs a) {
     const int lane = threadIdx.x & 63;
@@ -92,100 +193,58 @@ __global__ __launch_bounds__(64 * kSddmmWaves, 4) void sddmm_kernel(SddmmArgs a)
     const uint32_t j1 = min(j0 + span, a.nnz);
     const int r0 = wave_row_of(a.rowptr, j0, a.M, lane);
     const int r1 = wave_row_of(a.rowptr, j1 - 1, a.M, lane);
-    const size_t N = static_cast<size_t>(a.N);
-    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
-    const int l = lane & (L - 1), first = lane - l;
-    const int V = (a.N + E - 1) / E;      // pieces of a row
-    const int full = a.N / (E * L) * L;   // pieces of whole piece columns
     int lo = r0;
     for (uint32_t jb = j0; jb < j1; jb += 64) {
         const uint32_t j = min(jb + lane, j1 - 1);
-        const int mycol = a.colidx[j];
-        const int myrow = row_of(a.rowptr, j, lo, r1);
-        lo = __builtin_amdgcn_readlane(myrow, 63);
-        uint32_t brow[L];  // byte offsets of the rows of B (a plan's B is below 4 GiB)
-        int grow[L];
-#pragma unroll
-        for (int u = 0; u < L; u++) {
-            brow[u] = static_cast<uint32_t>(__shfl(mycol, first + u)) * rowbytes;
-            grow[u] = __shfl(myrow, first + u);
+        const int col = a.colidx[j];
+        const int row = row_of(a.rowptr, j, lo, r1);
+        lo = __builtin_amdgcn_readlane(row, 63);
+        const float sum = sddmm_batch<T, E, L>(a, row, col, lane);
+        if (jb + lane < j1) a.out[j] = sum;
+    }
+}
+
+// The same for the rows of the row kernel's task list (those outside the row
+// panels, whose nonzeros lie scattered through the CSR): a wavefront per task;
+// a group of short rows is walked nonzero by nonzero, 64 at a time.
+template <typename T, int E, int L>
+__global__ __launch_bounds__(64 * kSddmmWaves, 4) void sddmm_tasks_kernel(SddmmArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int tid = blockIdx.x * kSddmmWaves + (threadIdx.x >> 6);
+    if (tid >= a.ntasks) return;
+    const int4 t = a.tasks[tid];
+    if ((t.w & 3) != kTaskMulti) {  // a row, a quarter or a segment of one
+        const int row = (t.w & 3) == kTaskSeg ? a.longrows[t.x].x : t.x;
+        for (int jb = t.y; jb < t.z; jb += 64) {
+            const int j = min(jb + lane, t.z - 1);
+            const float sum = sddmm_batch<T, E, L>(a, row, a.colidx[j], lane);
+            if (jb + lane < t.z) a.out[j] = sum;
         }
-        const bool one_row = __ballot(grow[0] != grow[L - 1]) == 0;  // rows ascend within a slot
-        double acc[L];
+        return;
+    }
+    if (t.z == 0) return;  // empty rows
+    int row = 0, beg = 0, len = 0;
+    if (lane < t.y) {
+        row = a.perm[t.x + lane];
+        beg = a.rowptr[row];
+        len = a.rowptr[row + 1] - beg;
+    }
+    int end = len;  // of the row among the group's nonzeros
 #pragma unroll
-        for (int u = 0; u < L; u++) acc[u] = 0.;
-        auto add = [&](int u, const Pack<float, E>& g, const Pack<T, E>& b, int skip) {
-            float t[(E + 3) / 4];
+    for (int d = 1; d < 64; d <<= 1) {
+        const int x = __shfl_up(end, d);
+        if (lane >= d) end += x;
+    }
+    const int total = __builtin_amdgcn_readlane(end, 63);
+    for (int qb = 0; qb < total; qb += 64) {
+        const int q = min(qb + lane, total - 1);
+        int i = 0;  // the row of nonzero q: the first that ends after it
 #pragma unroll
-            for (int e = 0; e < E; e++) {
-                float s = e % 4 == 0 ? g.v[e] * to_f32(b.v[e]) : __builtin_fmaf(g.v[e], to_f32(b.v[e]), t[e / 4]);
-                if (skip > e) s = 0.f;
-                t[e / 4] = s;
-            }
-            acc[u] += static_cast<double>(E == 8 ? t[0] + t[E / 8] : t[0]);
-        };
-        auto load_b = [&](int u, int at) {
-            return load_unaligned<T, E>(reinterpret_cast<const T*>(static_cast<const char*>(a.B) +
-                                                               (brow[u] + static_cast<uint32_t>(at) * sizeof(T))));
-        };
-        auto load_g = [&](int u, int at) { return load_unaligned<float, E>(a.G + static_cast<size_t>(grow[u]) * N + at); };
-        auto piece = [&](int at, int skip) {  // columns [at, at + E), the first `skip` of them not counted
-            Pack<T, E> b[L];
-            const Pack<float, E> g = load_g(0, at);
-#pragma unroll
-            for (int u = 0; u < L; u++) b[u] = load_b(u, at);
-#pragma unroll
-            for (int u = 0; u < L; u++) add(u, g, b[u], skip);
-        };
-        auto piece_rows = [&](int at, int skip) {  // the same, every nonzero with its own row of G
-            constexpr int H = L > 4 ? 4 : L;       // nonzeros loaded at a time (registers)
-#pragma unroll
-            for (int h = 0; h < L; h += H) {
-                Pack<T, E> b[H];
-                Pack<float, E> g[H];
-#pragma unroll
-                for (int u = 0; u < H; u++) {
-                    g[u] = load_g(h + u, at);
-                    b[u] = load_b(h + u, at);
-                }
-#pragma unroll
-                for (int u = 0; u < H; u++) add(h + u, g[u], b[u], skip);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-        const int tail = full + l;  // the last piece of a row that is no whole number of them ends at the row's end
-        const int at = min(tail * E, a.N - E);
-        if (one_row) {
-#pragma unroll(E == 8 ? 1 : 2)
-            for (int p = 0; p < full; p += L) piece((p + l) * E, 0);
-            if (tail < V) piece(at, tail * E - at);
-        } else {
-#pragma unroll 1
-            for (int p = 0; p < full; p += L) piece_rows((p + l) * E, 0);
-            if (tail < V) piece_rows(at, tail * E - at);
-        }
-        float sum[L];
-#pragma unroll
-        for (int u = 0; u < L; u++) sum[u] = static_cast<float>(acc[u]);
-        if constexpr (L == 8) {
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float give = l & 4 ? sum[u] : sum[u + 4], keep = l & 4 ? sum[u + 4] : sum[u];
-                sum[u] = keep + dpp_swap<0x141>(give);  // row_half_mirror
-            }
-        }
-        if constexpr (L >= 4) {
-#pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const float give = l & 2 ? sum[u] : sum[u + 2], keep = l & 2 ? sum[u + 2] : sum[u];
-                sum[u] = keep + dpp_swap<0x4e>(give);  // quad_perm [2, 3, 0, 1]
-            }
-        }
-        if constexpr (L >= 2) {
-            const float give = l & 1 ? sum[0] : sum[1], keep = l & 1 ? sum[1] : sum[0];
-            sum[0] = keep + dpp_swap<0xb1>(give);  // quad_perm [1, 0, 3, 2]
-        }
-        if (jb + lane < j1) a.out[jb + lane] = sum[0];
+        for (int d = 32; d >= 1; d >>= 1)
+            if (__shfl(end, i + d - 1) <= q) i += d;
+        const int j = __shfl(beg + len - end, i) + q;
+        const float sum = sddmm_batch<T, E, L>(a, __shfl(row, i), a.colidx[j], lane);
+        if (qb + lane < total) a.out[j] = sum;
     }
 }
 

@@ -427,9 +427,8 @@ int launch_rows(const tca_spmm_plan* p, const void* val, const void* B, float* C
     }
 }
 
-template <typename T, int E>
-void launch_panels_t(const tca_spmm_plan* p, const void* val, const void* B, float* C, float* W, hipStream_t s) {
-    PanelArgs a;
+PanelArgs panel_args(const tca_spmm_plan* p) {
+    PanelArgs a{};
     a.units = p->d_units;
     a.order = p->d_porder;
     a.panel_units = p->d_panel_units;
@@ -439,13 +438,19 @@ void launch_panels_t(const tca_spmm_plan* p, const void* val, const void* B, flo
     a.cnt = p->d_pcnt;
     a.pos = p->d_ppos;
     a.ustart = p->d_ustart;
+    a.N = p->N;
+    a.chunks = p->panels.chunks;
+    a.pos_bytes = static_cast<uint32_t>(p->n_pos_bytes);
+    return a;
+}
+
+template <typename T, int E>
+void launch_panels_t(const tca_spmm_plan* p, const void* val, const void* B, float* C, float* W, hipStream_t s) {
+    PanelArgs a = panel_args(p);
     a.val = val;
     a.B = B;
     a.C = C;
     a.partials = W;
-    a.N = p->N;
-    a.chunks = p->panels.chunks;
-    a.pos_bytes = static_cast<uint32_t>(p->n_pos_bytes);
     a.val_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * sizeof(T));
     TCA_PHASE_LAUNCH((panel_kernel<T, E>), dim3(p->n_pblocks * p->panels.chunks), dim3(kPnThreads), 0, s, a);
 }
@@ -479,7 +484,10 @@ void launch_sddmm_e(const SddmmArgs& a, hipStream_t s) {
     const uint64_t span = 64ull * a.batches * kSddmmWaves;
     const dim3 grid(static_cast<unsigned>((a.nnz + span - 1) / span)), block(64 * kSddmmWaves);
     const int V = (a.N + E - 1) / E;
-    if (V > 4) hipLaunchKernelGGL((sddmm_kernel<T, E, 8>), grid, block, 0, s, a);
+    if (a.tasks) {  // beside panels (B rows of at least 64 bytes: 4 pieces and more)
+        const dim3 tgrid((a.ntasks + kSddmmWaves - 1) / kSddmmWaves);
+        if constexpr (E > 1) hipLaunchKernelGGL((sddmm_tasks_kernel<T, E, 8>), tgrid, block, 0, s, a);
+    } else if (V > 4) hipLaunchKernelGGL((sddmm_kernel<T, E, 8>), grid, block, 0, s, a);
     else if (V > 2) hipLaunchKernelGGL((sddmm_kernel<T, E, 4>), grid, block, 0, s, a);
     else if (V > 1) hipLaunchKernelGGL((sddmm_kernel<T, E, 2>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((sddmm_kernel<T, E, 1>), grid, block, 0, s, a);
@@ -542,6 +550,21 @@ template <bool kBf16>
 void launch_bell(const BellArgs& a, int bsize, hipStream_t s) {
     if (bsize == 32) launch_bell_w<kBf16, 32>(a, s);
     else launch_bell_w<kBf16, 64>(a, s);
+}
+
+// The sampled product of the panels' nonzeros (one column chunk).
+template <typename T>
+void launch_sddmm_panels(const tca_spmm_plan* p, const float* G, const void* B, float* out, hipStream_t s) {
+    PanelArgs a = panel_args(p);
+    a.G = G;
+    a.B = B;
+    a.out = out;
+    a.val_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * 4);
+    const dim3 grid(p->n_pblocks), block(kPnThreads);
+    const int e = p->panels.elems;
+    if (e == 8) hipLaunchKernelGGL((panel_sddmm_kernel<T, 8>), grid, block, 0, s, a);
+    else if (e == 4) hipLaunchKernelGGL((panel_sddmm_kernel<T, 4>), grid, block, 0, s, a);
+    else if constexpr (sizeof(T) == 4) hipLaunchKernelGGL((panel_sddmm_kernel<T, 2>), grid, block, 0, s, a);
 }
 
 // Bit 1 << TCA_PHASE_* for each phase in which the plan launches a kernel.
@@ -2037,6 +2060,23 @@ int tca_sddmm(const tca_spmm_plan* p, const float* d_G, const void* d_B, float* 
     a.N = p->N;
     a.nnz = static_cast<uint32_t>(p->nnz);
     a.batches = std::min(std::max(a.nnz / (64 * kSddmmFill), 1u), kSddmmMaxBatches);
+    a.tasks = nullptr;
+    // Rows in panels of one column chunk take the panel kernel (its transfers
+    // need B aligned as a product's), the row kernel's rows the gathering one;
+    // with matrix-core windows, whose rows neither has, everything is gathered.
+    if (p->n_units > 0 && p->panels.chunks == 1 && p->mfma.windows.empty() &&
+        reinterpret_cast<uintptr_t>(d_B) % 16 == 0) {
+        switch (p->dtype) {
+            case TCA_F16: launch_sddmm_panels<_Float16>(p, d_G, d_B, d_out, s); break;
+            case TCA_BF16: launch_sddmm_panels<bf16_t>(p, d_G, d_B, d_out, s); break;
+            default: launch_sddmm_panels<float>(p, d_G, d_B, d_out, s);
+        }
+        a.tasks = p->d_tasks;
+        a.perm = p->d_perm;
+        a.longrows = p->d_longrows;
+        a.ntasks = p->ntasks;
+    }
+    if (!a.tasks || p->panels.nnz < p->nnz)
     switch (p->dtype) {
         case TCA_F16: launch_sddmm<_Float16>(a, s); break;
         case TCA_BF16: launch_sddmm<bf16_t>(a, s); break;

@@ -19,7 +19,7 @@ def _pattern(rng, lens, k):
     return rowptr, colidx.astype(np.int32)
 
 
-def _run(torch, dtype, lens, k, n, rng, shift=0):
+def _run(torch, dtype, lens, k, n, rng, shift=0, flags=S.TCA_PLAN_DEFAULT, info=None):
     """out[j] and its exact value; B, G and out start `shift` elements into their buffers."""
     rowptr, colidx = _pattern(rng, lens, k)
     m, nnz = len(lens), len(colidx)
@@ -34,7 +34,9 @@ def _run(torch, dtype, lens, k, n, rng, shift=0):
 
     out = torch.full((nnz + shift + 1,), -1.0, device="cuda:0")
     gd, bd = dev(g, torch.float32), dev(b, dt)
-    with S.Plan(a, n) as plan:
+    with S.Plan(a, n, flags) as plan:
+        if info is not None:
+            info.update(plan.info())
         S.call("tca_sddmm", plan._p, S._addr(gd), S._addr(bd), S._addr(out[shift:]), None)
         torch.cuda.synchronize()
     got = out.cpu().numpy()
@@ -99,3 +101,107 @@ def test_non_finite_rows_stay_in_their_products(torch_cuda):
     want = (g[rows].double() * b[torch.from_numpy(colidx).long().to("cuda:0")].double()).sum(1).float()
     assert torch.equal(torch.isfinite(out), torch.isfinite(want))
     assert torch.equal(torch.nan_to_num(out, 1.0, 2.0, 3.0), torch.nan_to_num(want, 1.0, 2.0, 3.0))
+
+
+PANEL_SHAPES = [(S.TCA_F32, 32), (S.TCA_F32, 64), (S.TCA_F32, 128), (S.TCA_F16, 64), (S.TCA_F16, 128), (S.TCA_BF16, 64),
+                (S.TCA_BF16, 128)]
+
+
+def _graph_lens(rng):
+    """Rows of a power law, some empty, one in every column."""
+    lens = np.minimum(3000, (4 / rng.random(900) ** 0.8).astype(int))
+    lens[rng.integers(0, 900, 60)] = 0
+    lens[17] = 3000
+    return lens.tolist()
+
+
+@pytest.mark.parametrize("window", ["0", "1"])
+@pytest.mark.parametrize("dtype,n", PANEL_SHAPES)
+def test_panels_exact(torch_cuda, monkeypatch, dtype, n, window):
+    """The panel form (every geometry of one column chunk, run data where they lie
+    or through windows, panels split into several units)."""
+    monkeypatch.setenv("TCA_PANEL_WINDOW", window)
+    monkeypatch.setenv("TCA_PANEL_UNIT", "900")
+    print(f"panel sddmm dtype={dtype} n={n} window={window}", flush=True)
+    rng = np.random.default_rng(n)
+    info = {}
+    got, want = _run(torch_cuda, dtype, _graph_lens(rng), 3000, n, rng, flags=S.TCA_PLAN_FORCE_PANELS | S.TCA_PLAN_NO_MFMA,
+                     info=info)
+    assert info["nnz_panels"] == len(want) and info["n_panel_units"] > info["n_panels"]
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("dtype,n", [(S.TCA_F32, 128), (S.TCA_BF16, 128)])
+def test_panels_and_other_rows(torch_cuda, monkeypatch, dtype, n):
+    """Some rows in panels, the others gathered, each nonzero written once."""
+    monkeypatch.setenv("TCA_PANEL_MIN_REUSE", "1.5")
+    monkeypatch.setenv("TCA_PANEL_MIN_NNZ", "1")
+    rng = np.random.default_rng(n + 7)
+    info = {}
+    got, want = _run(torch_cuda, dtype, _graph_lens(rng) + [2] * 700, 3000, n, rng, flags=S.TCA_PLAN_NO_MFMA, info=info)
+    assert 0 < info["nnz_panels"] < len(want)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("dtype,n", [(S.TCA_F32, 32), (S.TCA_F32, 128), (S.TCA_F16, 64)])
+def test_every_task_beside_panels(torch_cuda, monkeypatch, dtype, n):
+    """Panels keep a band of like rows; short rows in groups, medium rows, quarters
+    and segments of long rows are left to the row kernel's list."""
+    monkeypatch.setenv("TCA_PANEL_MIN_REUSE", "2")
+    monkeypatch.setenv("TCA_PANEL_MIN_NNZ", "1")
+    rng = np.random.default_rng(n + 1)
+    k = 60000
+    lens = [9000, 4000, 1500, 700, 300] + rng.integers(0, 40, 187).tolist() + [0, 1, 2, 3] * 200
+    band = np.arange(40)
+    # the longest rows share little with the 600 rows of 35 that share 40 columns
+    cols = [np.sort(rng.choice(np.arange(40, k), x, replace=False)) for x in lens]
+    lens2 = [35] * 600
+    cols += [np.sort(rng.choice(band, 35, replace=False)) for _ in lens2]
+    lens = lens + lens2
+    rowptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    colidx = np.concatenate(cols).astype(np.int32)
+    a = S.CSR(len(lens), k, rowptr, colidx, S.to_storage(np.ones(len(colidx), np.float32), dtype), dtype)
+    g, b = exact_dense(rng, (len(lens), n)), exact_dense(rng, (k, n))
+    gd = torch_cuda.from_numpy(g).to("cuda:0")
+    bd = torch_cuda.from_numpy(b).to("cuda:0").to(getattr(torch_cuda, TORCH[dtype]))
+    out = torch_cuda.full((len(colidx),), -1.0, device="cuda:0")
+    with S.Plan(a, n, S.TCA_PLAN_NO_MFMA) as plan:
+        info = plan.info()
+        S.call("tca_sddmm", plan._p, S._addr(gd), S._addr(bd), S._addr(out), None)
+        torch_cuda.cuda.synchronize()
+    print(f"tasks beside panels dtype={dtype} n={n}: {info['rows_panels']} of {len(lens)} rows in panels", flush=True)
+    rows = np.repeat(np.arange(len(lens)), lens)
+    want = (g[rows].astype(np.float64) * b[colidx]).sum(1).astype(np.float32)
+    if n == 128:  # (narrower B rows go to panels only when asked)
+        assert 0 < info["rows_panels"] < len(lens) and info["n_long_rows"] > 0 and info["n_wide_tasks"] > 0
+    assert np.array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n,shift", [(256, 0), (128, 1)])
+def test_panels_that_gather(torch_cuda, n, shift):
+    """Plans with two column chunks, and B off 16 bytes, keep to the gathering form."""
+    rng = np.random.default_rng(n)
+    info = {}
+    got, want = _run(torch_cuda, S.TCA_F32, _graph_lens(rng), 3000, n, rng, shift=shift,
+                     flags=S.TCA_PLAN_FORCE_PANELS, info=info)
+    assert info["n_panels"] > 0
+    assert np.array_equal(got, want)
+
+
+def test_panels_keep_non_finite_rows_apart(torch_cuda):
+    """Infinite rows of G and NaN rows of B reach only their own products."""
+    torch = torch_cuda
+    rng = np.random.default_rng(12)
+    lens = _graph_lens(rng)
+    rowptr, colidx = _pattern(rng, lens, 3000)
+    a = S.CSR(len(lens), 3000, rowptr, colidx, np.ones(len(colidx), np.float32), S.TCA_F32)
+    g = torch.from_numpy(exact_dense(rng, (len(lens), 128))).to("cuda:0")
+    b = torch.from_numpy(exact_dense(rng, (3000, 128))).to("cuda:0")
+    g[17], b[8], b[2999] = float("inf"), float("nan"), float("nan")
+    out = torch.empty(len(colidx), device="cuda:0")
+    with S.Plan(a, 128, S.TCA_PLAN_FORCE_PANELS) as plan:
+        S.call("tca_sddmm", plan._p, S._addr(g), S._addr(b), S._addr(out), None)
+        torch.cuda.synchronize()
+    rows = np.repeat(np.arange(len(lens)), lens)
+    bad = torch.from_numpy((rows == 17) | (colidx == 8) | (colidx == 2999)).to("cuda:0")
+    assert torch.equal(~torch.isfinite(out), bad)
