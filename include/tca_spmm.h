@@ -153,7 +153,8 @@ int tca_spmm_plan_create(const int32_t* rowptr, const int32_t* colidx, int32_t M
  * d_B[K*N] (plan dtype) and d_C[M*N] (fp32) are DEVICE pointers; d_B and d_C
  * must be aligned to 16 bytes.  Stream-ordered on `stream` (a hipStream_t,
  * NULL = default stream); does not synchronise.  One plan must not run on two
- * streams at once: long-row partial sums live in plan-owned scratch.  A plan
+ * streams at once: long-row partial sums, and the copy of B that plans of some
+ * widths read at an aligned pitch, live in plan-owned scratch.  A plan
  * whose row phase only clears empty rows (tca_plan_info.rows_beside_panels)
  * runs it on a second stream it owns, beside the panel kernel: that stream
  * waits for the work queued on `stream` before the call, and `stream` waits
@@ -182,7 +183,8 @@ int tca_spmm_run_static(const tca_spmm_plan* plan, const void* d_val, const void
 int tca_spmm_time(const tca_spmm_plan* plan, const void* d_val, const void* d_B, float* d_C,
                   void* stream, int32_t warmup, int32_t iters, float* avg_ms);
 
-/* Phases of one run, in stream order: value pack for the MFMA tiles, MFMA
+/* Phases of one run, in stream order: value pack for the MFMA tiles (or the copy
+ * of B at an aligned pitch, for row kernels of ragged widths), MFMA
  * tile kernel, panel kernel, row kernel, segment sums of split rows (the
  * panel phase has index 4 so the older indices stay as they were). */
 #define TCA_PHASES 5

@@ -54,6 +54,24 @@ void plan_geometry(int32_t N, int32_t es, int32_t slices, RowPlan* p) {
     p->log_lanes = ilog2(next_pow2(p->chunk_lanes));
 }
 
+int32_t padded_pitch(int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t flags, bool on_device,
+                     const RowPlan& p) {
+    if (!p.ragged || (flags & TCA_PLAN_NO_SCRATCH)) return 0;
+    const int64_t e = 16 / es, line = 128 / es;
+    const int64_t whole = (N + e - 1) / e * e, lines = (N + line - 1) / line * line;
+    const bool to_lines = lines * 8 <= static_cast<int64_t>(N) * 9;
+    const int64_t pitch = to_lines ? lines : whole;
+    const int64_t bytes = K * pitch * es;
+    if (bytes > kMallBytes) return 0;  // (also keeps the copy within the 32-bit buffer offsets)
+    // Tuning override (not part of the interface): 0 never, 1 always.
+    if (const char* f = std::getenv("TCA_PAD")) return std::atoi(f) ? static_cast<int32_t>(pitch) : 0;
+    if (!to_lines && !(es == 2 && N % 2 == 1)) return 0;
+    const bool far = static_cast<int64_t>(K) * N * es > kPadFarBytes;
+    const double saved = (far ? kPadFarGain : es == 2 ? kPadNearGain : 0.0) * static_cast<double>(nnz) * N * es;
+    const double cost = kPadFixedUs + 2.0 * static_cast<double>(bytes) / kPadBytesPerUs;
+    return saved > (on_device ? 1.5 : 1.0) * cost ? static_cast<int32_t>(pitch) : 0;
+}
+
 void plan_row_params(int32_t M, int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan* p) {
     plan_geometry(N, es, slices, p);
     const int32_t slots = 64 >> p->log_lanes;

@@ -52,6 +52,24 @@ inline int32_t multi_group_rows(int32_t slots) { return slots * kMultiPasses < 6
 constexpr int32_t kRaggedMinN32 = 16;
 constexpr int32_t kRaggedMinN16 = 33;
 
+// Ragged rows gathered often enough are copied to an aligned pitch first
+// (padded_pitch): to whole 128-byte lines where that adds at most an eighth,
+// else to whole vectors (16-bit types of odd N; the others' vectors start at
+// dwords and gained nothing).  Copied when the time saved, by gathered bytes,
+// passes the copy's; by half as much again for plans made on the device, which
+// may run once.  us per product in place -> copied (copy included) on the
+// MI355X: 3001 x 2049 layer of 8 %, bf16 N = 47 11.0 -> 9.8, N = 333 38.2 ->
+// 29.2, N = 1023 75 -> 48, fp32 N = 333 32 -> 37; R-MAT of 200,000 nodes and
+// 6.7M nonzeros, fp16 N = 47 135 -> 106, N = 70 128 -> 135, N = 127 310 -> 199,
+// fp32 N = 47 127 -> 127, N = 101 296 -> 320, N = 127 504 -> 325; of 20,000
+// nodes and 372k, fp16 N = 255 40 -> 43, fp32 50 -> 55; Zipf rows, 300,000
+// columns, fp16 N = 127 3.7M nonzeros 368 -> 278, N = 47 0.9M 48 -> 58.
+constexpr int64_t kPadFarBytes = int64_t(24) << 20;  // a B past this comes from behind the L2s:
+constexpr double kPadFarGain = 6e-8;     // us saved per gathered byte (measured 4e-8 to 19e-8)
+constexpr double kPadNearGain = 3e-8;    // and within it, 16-bit types (2.5e-8 to 6e-8; fp32 none)
+constexpr double kPadFixedUs = 3.0;      // the copy's launch,
+constexpr double kPadBytesPerUs = 4e6;   // and its rate, each byte read and written
+
 struct Int4 {
     int32_t x, y, z, w;
 };
@@ -143,6 +161,11 @@ int32_t default_slices(int32_t K, int32_t N, int32_t dtype);
 // 8 chunks of at least 128 bytes (one L2 line of B per chunk row), at most
 // 64 lanes each.  `slices` > 0 forces the number of chunks (tuning).
 void plan_geometry(int32_t N, int32_t es, int32_t slices, RowPlan* p);
+
+// Ragged rows (RowPlan::ragged) of B that a plan copies to an aligned pitch
+// before each product: elements per row of the copy, 0 = read B in place
+// (always with TCA_PLAN_NO_SCRATCH, and past the MALL).
+int32_t padded_pitch(int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t flags, bool on_device, const RowPlan& p);
 
 // Lane geometry and task-length thresholds (row_len, wide_len, seg_len,
 // multi_max) of the row kernel for a matrix of nnz nonzeros.

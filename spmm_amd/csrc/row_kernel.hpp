@@ -143,6 +143,14 @@ __device__ __forceinline__ void store_line_pieces(float* row, int chunk_col, int
 // row; C is stored by pieces of four columns, the last one by element.
 // Vectors start at any element: fp32 ones through the buffer (dword aligned),
 // 16-bit ones through plain loads, masked ones from the zero piece.
+//
+// Such vectors cost the memory pipe up to twice an aligned one's time, and
+// column chunks that end inside a 128-byte line share that line between
+// XCDs.  Plans that gather a row of B often enough (padded_pitch, planner.cpp)
+// copy B into rows of `pitch` elements first (pad_rows_kernel) and read whole
+// aligned vectors there (kPadded); the sums and their order are the same.
+// A 3001 x 2049 bf16 layer of 8 % at N = 333: 36.2 -> 27.0 us, copy included.
+enum RowMode : int { kWhole = 0, kRaggedRows = 1, kPadded = 2 };
 static __device__ const int4 kZeroPiece = {0, 0, 0, 0};
 
 template <typename T, int E>
@@ -154,9 +162,9 @@ __device__ __forceinline__ Pack<T, E> load_unaligned(const T* p) {
 }
 
 // E elements of B at byte offset `off` (zeros unless ok).
-template <typename T, int E, bool kRagged>
+template <typename T, int E, int kMode>
 __device__ __forceinline__ Pack<T, E> load_b(__amdgpu_buffer_rsrc_t rB, const void* B, uint32_t off, bool ok) {
-    if constexpr (kRagged && sizeof(T) == 2) {
+    if constexpr (kMode == kRaggedRows && sizeof(T) == 2) {
         // (global address space spelled out: the select would make it a flat load)
         typedef int i32x4a2 __attribute__((ext_vector_type(4), aligned(2)));
         using Global = const __attribute__((address_space(1))) char*;
@@ -196,10 +204,11 @@ __device__ __forceinline__ void fma_pack(float (&acc)[E], float a, const Pack<T,
 
 // Stores a slot's sums of one row (lane g holds columns `col` ..; lanes of
 // `mine` write).  Every lane of the slot calls it.
-template <int E, bool kRagged>
+template <int E, int kMode>
 __device__ __forceinline__ void store_sums(float* row, float (&acc)[E], int lane, int g, int col, int chunk_col, int cl,
                                            int N, bool mine) {
-    if constexpr (kRagged) left_align<E>(acc, max(col + E - N, 0));
+    constexpr bool kRagged = kMode != kWhole;
+    if constexpr (kMode == kRaggedRows) left_align<E>(acc, max(col + E - N, 0));
     if constexpr (E == 8) {
         const LinePieces lp = line_pieces<E>(acc, lane, g, cl);
         if (mine && g < cl) {
@@ -226,6 +235,7 @@ struct RowArgs {
     float* partials;
     float* C;
     int N;
+    int pitch;        // elements from one row of B to the next (kPadded: B is the padded copy)
     int logG;         // log2 of lanes per slot
     int chunk_lanes;  // lanes per slot that hold data
     int col_chunks;   // blockIdx.x = task group * col_chunks + chunk
@@ -239,13 +249,13 @@ struct RowArgs {
 // columns [col, col + E).  Column indices and values are fetched 64 at a
 // time with one coalesced load and handed to the slots with ds_bpermute (or
 // v_readlane when one slot spans the whole wavefront).
-template <typename T, int E, bool kRagged, bool kOneSlot>
+template <typename T, int E, int kMode, bool kOneSlot>
 __device__ __forceinline__ void accumulate_span(float (&acc)[E], int beg, int end, const RowArgs& a,
                                                 __amdgpu_buffer_rsrc_t rcol, __amdgpu_buffer_rsrc_t rval,
                                                 __amdgpu_buffer_rsrc_t rB, int col, bool colok, int lane, int slot,
                                                 int logS) {
-    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
-    const uint32_t colbytes = static_cast<uint32_t>(kRagged ? min(col, a.N - E) : col) * sizeof(T);
+    const uint32_t rowbytes = static_cast<uint32_t>(kMode == kPadded ? a.pitch : a.N) * sizeof(T);
+    const uint32_t colbytes = static_cast<uint32_t>(kMode == kRaggedRows ? min(col, a.N - E) : col) * sizeof(T);
     // Indices and values of the first chunk of 64; each chunk's loop below
     // first issues the loads of the next chunk, so they travel while the B
     // rows of this one are gathered.
@@ -275,7 +285,7 @@ __device__ __forceinline__ void accumulate_span(float (&acc)[E], int beg, int en
                     av[u] = __shfl(mya, idx & 63);
                     ok = idx < n && colok;
                 }
-                bv[u] = load_b<T, E, kRagged>(rB, a.B, static_cast<uint32_t>(c) * rowbytes + colbytes, ok);
+                bv[u] = load_b<T, E, kMode>(rB, a.B, static_cast<uint32_t>(c) * rowbytes + colbytes, ok);
             }
 #pragma unroll
             for (int u = 0; u < kRowUnroll; u++) fma_pack<T, E>(acc, av[u], bv[u]);
@@ -290,13 +300,13 @@ __device__ __forceinline__ void accumulate_span(float (&acc)[E], int beg, int en
 // of a lane have a nonzero (chunks of 64 leave all but 64 / S of them idle);
 // with 64 slots every lane keeps its own nonzeros and nothing is shuffled.
 // Slot s takes the same nonzeros in the same order as above.
-template <typename T, int E, bool kRagged, int S>
+template <typename T, int E, int kMode, int S>
 __device__ __forceinline__ void accumulate_narrow(float (&acc)[E], int beg, int end, const RowArgs& a,
                                                   __amdgpu_buffer_rsrc_t rcol, __amdgpu_buffer_rsrc_t rval,
                                                   __amdgpu_buffer_rsrc_t rB, int col, bool colok, int lane, int slot) {
     constexpr int R = S * kRowUnroll / 64;
-    const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
-    const uint32_t colbytes = static_cast<uint32_t>(kRagged ? min(col, a.N - E) : col) * sizeof(T);
+    const uint32_t rowbytes = static_cast<uint32_t>(kMode == kPadded ? a.pitch : a.N) * sizeof(T);
+    const uint32_t colbytes = static_cast<uint32_t>(kMode == kRaggedRows ? min(col, a.N - E) : col) * sizeof(T);
     int c[R];
     float v[R];
     auto fetch = [&](int base) {
@@ -316,7 +326,7 @@ __device__ __forceinline__ void accumulate_narrow(float (&acc)[E], int beg, int 
             const int q = u * S / 64, from = u * S % 64 + slot;  // register and lane of nonzero u S + slot
             const int cu = S == 64 ? c[q] : __shfl(c[q], from);
             av[u] = S == 64 ? v[q] : __shfl(v[q], from);
-            bv[u] = load_b<T, E, kRagged>(rB, a.B, static_cast<uint32_t>(cu) * rowbytes + colbytes,
+            bv[u] = load_b<T, E, kMode>(rB, a.B, static_cast<uint32_t>(cu) * rowbytes + colbytes,
                                           base + u * S + slot < end && colok);
         }
         if (base + 64 * R < end) fetch(base + 64 * R);
@@ -328,8 +338,9 @@ __device__ __forceinline__ void accumulate_narrow(float (&acc)[E], int beg, int 
 // kNarrow: at least 16 slots (logG <= 2).  An instance of its own: the narrow
 // spans' registers would cost the wide ones occupancy (fp32 65 -> 79, 16-bit
 // 64 -> 94 VGPRs).
-template <typename T, int E, bool kRagged, bool kNarrow>
+template <typename T, int E, int kMode, bool kNarrow>
 __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
+    constexpr bool kRagged = kMode != kWhole;  // N is no whole number of vectors
     static_assert(!kRagged || E * sizeof(T) == 16, "ragged rows take whole vectors");
     __shared__ float red[kRowWaves][64 * E];  // wide rows: one partial row chunk per wavefront
     const int lane = threadIdx.x & 63;
@@ -417,8 +428,8 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
             beg = a.rowptr[row];
             len = a.rowptr[row + 1] - beg;
         }
-        const uint32_t rowbytes = static_cast<uint32_t>(a.N) * sizeof(T);
-        const uint32_t colbytes = static_cast<uint32_t>(kRagged ? min(col, a.N - E) : col) * sizeof(T);
+        const uint32_t rowbytes = static_cast<uint32_t>(kMode == kPadded ? a.pitch : a.N) * sizeof(T);
+        const uint32_t colbytes = static_cast<uint32_t>(kMode == kRaggedRows ? min(col, a.N - E) : col) * sizeof(T);
         for (int p0 = 0; p0 < t.y; p0 += S) {
             int nrow = -1, nbeg = 0, nlen = 0;
             if (p0 + S + slot < t.y) {
@@ -439,12 +450,12 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
                 }
 #pragma unroll
                 for (int u = 0; u < kRowUnroll; u++)
-                    bv[u] = load_b<T, E, kRagged>(rB, a.B, static_cast<uint32_t>(c[u]) * rowbytes + colbytes,
+                    bv[u] = load_b<T, E, kMode>(rB, a.B, static_cast<uint32_t>(c[u]) * rowbytes + colbytes,
                                                   j + u < len && colok);
 #pragma unroll
                 for (int u = 0; u < kRowUnroll; u++) fma_pack<T, E>(acc, av[u], bv[u]);
             }
-            store_sums<E, kRagged>(a.C + static_cast<size_t>(max(row, 0)) * a.N, acc, lane, g, col, chunk_col, a.chunk_lanes,
+            store_sums<E, kMode>(a.C + static_cast<size_t>(max(row, 0)) * a.N, acc, lane, g, col, chunk_col, a.chunk_lanes,
                                    a.N, row >= 0);
             row = nrow;
             beg = nbeg;
@@ -456,15 +467,15 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
     // row / seg: all slots on one span
     if constexpr (kNarrow) {
         if (a.logG == 0)
-            accumulate_narrow<T, E, kRagged, 64>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
+            accumulate_narrow<T, E, kMode, 64>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
         else if (a.logG == 1)
-            accumulate_narrow<T, E, kRagged, 32>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
+            accumulate_narrow<T, E, kMode, 32>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
         else
-            accumulate_narrow<T, E, kRagged, 16>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
+            accumulate_narrow<T, E, kMode, 16>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot);
     } else if (a.logG == 6) {
-        accumulate_span<T, E, kRagged, true>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
+        accumulate_span<T, E, kMode, true>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
     } else {
-        accumulate_span<T, E, kRagged, false>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
+        accumulate_span<T, E, kMode, false>(acc, t.y, t.z, a, rcol, rval, rB, col, colok, lane, slot, logS);
     }
     for (int off = 1 << a.logG; off < 64; off <<= 1)
 #pragma unroll
@@ -482,13 +493,37 @@ __global__ __launch_bounds__(256) void row_kernel(RowArgs a) {
 #pragma unroll
         for (int e = 0; e < E; e++)
             acc[e] = ((red[0][g * E + e] + red[1][g * E + e]) + red[2][g * E + e]) + red[3][g * E + e];
-        store_sums<E, kRagged>(a.C + static_cast<size_t>(t.x) * a.N, acc, lane, g, col, chunk_col, a.chunk_lanes, a.N,
+        store_sums<E, kMode>(a.C + static_cast<size_t>(t.x) * a.N, acc, lane, g, col, chunk_col, a.chunk_lanes, a.N,
                                slot == 0);
         return;
     }
     float* const dst_row = t.w == 0 ? a.C + static_cast<size_t>(t.x) * a.N
                                     : a.partials + static_cast<size_t>(t.w >> 2) * a.N;  // seg: partial row of slot t.w >> 2
-    store_sums<E, kRagged>(dst_row, acc, lane, g, col, chunk_col, a.chunk_lanes, a.N, slot == 0);
+    store_sums<E, kMode>(dst_row, acc, lane, g, col, chunk_col, a.chunk_lanes, a.N, slot == 0);
+}
+
+// Rows of N elements of B into rows of `pitch`, whole vectors with zeros behind
+// column N (what lies past the last vector is never read).  One vector per
+// thread; bound by the memory: B read and written once.
+template <typename T>
+__global__ __launch_bounds__(256) void pad_rows_kernel(const T* __restrict__ B, T* __restrict__ out, int K, int N,
+                                                       int pitch) {
+    constexpr int E = 16 / sizeof(T);
+    const uint32_t V = static_cast<uint32_t>(N + E - 1) / E;  // vectors of a row
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= static_cast<uint64_t>(K) * V) return;
+    const uint32_t r = static_cast<uint32_t>(i) / V;  // (at most 2^28 vectors)
+    const int col = static_cast<int>(static_cast<uint32_t>(i) - r * V) * E;
+    const T* const src = B + static_cast<size_t>(r) * N + col;
+    Pack<T, E> v{};
+    if (col + E <= N) {
+        v = load_unaligned<T, E>(src);
+    } else {
+#pragma unroll
+        for (int e = 0; e < E - 1; e++)
+            if (col + e < N) v.v[e] = src[e];
+    }
+    *reinterpret_cast<Pack<T, E>*>(out + static_cast<size_t>(r) * pitch + col) = v;
 }
 
 // Lanes of seg_finalize_kernel per partial row: four columns each, a power

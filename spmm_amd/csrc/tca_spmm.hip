@@ -62,6 +62,8 @@ struct tca_spmm_plan {
     int32_t n_dn = 0;              // dense kernel: nonzeros the pack writes
     int* d_dn_src = nullptr;       // per nonzero (sorted by position): its CSR index
     uint32_t* d_dn_pos = nullptr;  // and its half index in d_adense
+    void* d_bpad = nullptr;        // row kernel, ragged rows: B's copy at `b_pitch` elements per row (padded_pitch),
+    int32_t b_pitch = 0;           // written by every run
     int32_t mfma_groups = 0; // paired kernel: groups of 64 entries a step may hold (4 or 8)
     size_t mfma_zeros_at = 0;  // word offset of 16 zero bytes in d_packed (LDS-DMA kernel)
     size_t n_packed = 0;       // words of d_packed
@@ -193,6 +195,7 @@ void free_plan_device(tca_spmm_plan* p) {
     (void)hipFree(p->d_pk_src);
     (void)hipFree(p->d_pk_cell);
     (void)hipFree(p->d_packed);
+    (void)hipFree(p->d_bpad);
     (void)hipFree(p->d_adense);
     (void)hipFree(p->d_amask);
     (void)hipFree(p->d_dn_src);
@@ -250,7 +253,7 @@ thread_local hipEvent_t g_phase_ev[2] = {nullptr, nullptr};
             hipLaunchKernelGGL(kernel, grid, block, shm, stream, __VA_ARGS__);                                  \
     } while (0)
 
-template <typename T, int E, bool kRagged = false>
+template <typename T, int E, int kMode = kWhole>
 void launch_rows_t(const tca_spmm_plan* p, const void* val, const void* B, float* C, float* W, hipStream_t s) {
     RowArgs a;
     a.tasks = p->d_tasks;
@@ -266,15 +269,16 @@ void launch_rows_t(const tca_spmm_plan* p, const void* val, const void* B, float
     a.col_chunks = p->rows.col_chunks;
     a.colidx = p->d_colidx;
     a.val = val;
-    a.B = B;
+    a.B = kMode == kPadded ? p->d_bpad : B;
+    a.pitch = kMode == kPadded ? p->b_pitch : p->N;
     // Byte sizes of the buffer ranges (checked < 2^32 - 16 at plan time).
     a.colidx_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * 4);
     a.val_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->nnz) * sizeof(T));
-    a.B_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->K) * p->N * sizeof(T));
+    a.B_bytes = static_cast<uint32_t>(static_cast<uint64_t>(p->K) * a.pitch * sizeof(T));
     if (a.logG <= 2)
-        TCA_PHASE_LAUNCH((row_kernel<T, E, kRagged, true>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
+        TCA_PHASE_LAUNCH((row_kernel<T, E, kMode, true>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
     else
-        TCA_PHASE_LAUNCH((row_kernel<T, E, kRagged, false>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
+        TCA_PHASE_LAUNCH((row_kernel<T, E, kMode, false>), dim3(row_blocks(p)), dim3(64 * kRowWaves), 0, s, a);
 }
 
 // Adds the segments of long rows (after the row kernel, same stream).
@@ -287,7 +291,8 @@ void launch_finalize(const tca_spmm_plan* p, float* C, const float* W, hipStream
 template <typename T>
 int launch_rows_e(const tca_spmm_plan* p, const void* val, const void* B, float* C, float* W, hipStream_t s) {
     if (p->rows.ragged) {
-        launch_rows_t<T, 16 / sizeof(T), true>(p, val, B, C, W, s);
+        if (p->b_pitch) launch_rows_t<T, 16 / sizeof(T), kPadded>(p, val, B, C, W, s);
+        else launch_rows_t<T, 16 / sizeof(T), kRaggedRows>(p, val, B, C, W, s);
         return TCA_OK;
     }
     switch (p->rows.elems_per_lane) {
@@ -304,8 +309,22 @@ int launch_rows_e(const tca_spmm_plan* p, const void* val, const void* B, float*
     }
 }
 
-// Pairs the MFMA entries with this run's values (before the tile kernel).
-void launch_pack(const tca_spmm_plan* p, const void* val, hipStream_t s) {
+template <typename T>
+void launch_pad(const tca_spmm_plan* p, const void* B, hipStream_t s) {
+    constexpr int E = 16 / sizeof(T);
+    const uint64_t vectors = static_cast<uint64_t>(p->K) * ((p->N + E - 1) / E);
+    TCA_PHASE_LAUNCH((pad_rows_kernel<T>), dim3(static_cast<unsigned>((vectors + 255) / 256)), dim3(256), 0, s,
+                     static_cast<const T*>(B), static_cast<T*>(p->d_bpad), p->K, p->N, p->b_pitch);
+}
+
+// What a run lays out before the products: the padded copy of B, or the MFMA
+// entries paired with this run's values (such plans have whole vectors).
+void launch_pack(const tca_spmm_plan* p, const void* val, const void* B, hipStream_t s) {
+    if (p->b_pitch) {
+        if (dtype_size(p->dtype) == 4) launch_pad<float>(p, B, s);
+        else launch_pad<_Float16>(p, B, s);
+        return;
+    }
     if (p->mfma_dense) {
         if (p->n_dn > 0)
             TCA_PHASE_LAUNCH(dense_pack_kernel, dim3((p->n_dn + 255) / 256), dim3(256), 0, s, p->d_dn_src,
@@ -570,7 +589,8 @@ void launch_sddmm_panels(const tca_spmm_plan* p, const float* G, const void* B, 
 // Bit 1 << TCA_PHASE_* for each phase in which the plan launches a kernel.
 uint32_t phases_used(const tca_spmm_plan* p) {
     uint32_t m = 0;
-    if (!p->mfma.windows.empty() && (!p->mfma.entries.empty() || p->n_dn > 0)) m |= 1u << TCA_PHASE_PACK;
+    if (p->b_pitch || (!p->mfma.windows.empty() && (!p->mfma.entries.empty() || p->n_dn > 0)))
+        m |= 1u << TCA_PHASE_PACK;
     if (!p->mfma.windows.empty() || p->mfma_short) m |= 1u << TCA_PHASE_TILES;
     if (p->ntasks > 0) m |= 1u << TCA_PHASE_ROWS;
     if (p->n_longrows > 0) m |= 1u << TCA_PHASE_SEGMENTS;
@@ -578,12 +598,12 @@ uint32_t phases_used(const tca_spmm_plan* p) {
     return m;
 }
 
-// One SpMM in stream order: pack, tile kernel, panel kernel, row kernel, segment sums.
+// One SpMM in stream order: pack (or the padded copy of B), tile kernel, panel kernel, row kernel, segment sums.
 // W: the partial rows of split rows (plan-owned, or the static scratch).
 // mask: the phases to launch (bit 1 << TCA_PHASE_*); all of them for a product.
 int run_phases(const tca_spmm_plan* p, const void* val, const void* B, float* C, float* W, hipStream_t s,
                uint32_t mask = ~0u) {
-    if (mask & (1u << TCA_PHASE_PACK)) launch_pack(p, val, s);
+    if (mask & (1u << TCA_PHASE_PACK)) launch_pack(p, val, B, s);
     int st = TCA_OK;
     if (mask & (1u << TCA_PHASE_TILES)) st = launch_mfma(p, val, B, C, s);
     if (st) return st;
@@ -625,6 +645,21 @@ void setup_side_stream(tca_spmm_plan* p) {
         return;
     }
     p->info.rows_beside_panels = 1;
+}
+
+// The padded copy of B, when the row kernel's plan wants one and the device
+// has room for it (else the plan reads B in place).
+void setup_pad(tca_spmm_plan* p) {
+    const int32_t es = static_cast<int32_t>(dtype_size(p->dtype));
+    if (p->M == 0 || p->nnz == 0) return;
+    const int32_t pitch = padded_pitch(p->K, p->nnz, p->N, es, p->flags, p->device_planned, p->rows);
+    if (pitch == 0) return;
+    if (dev_malloc(&p->d_bpad, static_cast<size_t>(p->K) * pitch * es) != hipSuccess) {
+        p->d_bpad = nullptr;
+        (void)hipGetLastError();  // not the next call's error
+        return;
+    }
+    p->b_pitch = pitch;
 }
 
 // Plan statistics (tca_plan_info) from a built plan.
@@ -700,6 +735,10 @@ void print_launches(const tca_spmm_plan* p) {
     auto line = [](long long blocks, int dim, double lds_bytes, const char* name) {
         std::printf("num_block: %lld blockdim: %d shm: %fKB (%s)\n", blocks, dim, lds_bytes / 1024.0, name);
     };
+    if (p->b_pitch) {
+        const int e = static_cast<int>(16 / dtype_size(p->dtype));
+        line((static_cast<long long>(p->K) * ((p->N + e - 1) / e) + 255) / 256, 256, 0.0, "pad_rows_kernel");
+    }
     if (p->mfma_short) line(in.mfma_blocks, in.mfma_blockdim, in.mfma_lds_bytes, "mfma_short_kernel");
     if (!p->mfma.windows.empty()) {
         if (p->mfma_dense) {
@@ -1108,6 +1147,7 @@ int tca_spmm_plan_create(const int32_t* rowptr, const int32_t* colidx, int32_t M
         }
         if (hipDeviceSynchronize() != hipSuccess) return bail(fail(TCA_ERR_HIP, "hipDeviceSynchronize failed"));
 
+        setup_pad(p);
         fill_info(p);
         setup_side_stream(p);
         p->info.plan_ms = std::chrono::duration<double, std::milli>(t1 - t0).count();
@@ -1844,6 +1884,7 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
             return bail(fail(TCA_ERR_HIP, "task emission failed"));
         st = bail(TCA_OK);  // frees the temporaries only
+        setup_pad(p);
         fill_info(p);
         setup_side_stream(p);
         p->info.plan_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -2253,7 +2294,7 @@ int tca_spmm_time_phases(const tca_spmm_plan* p, const void* d_val, const void* 
     };
     for (int i = 0; i < iters && st == TCA_OK; i++) {
         arm(i, TCA_PHASE_PACK);
-        launch_pack(p, d_val, s);
+        launch_pack(p, d_val, d_B, s);
         arm(i, TCA_PHASE_TILES);
         st = launch_mfma(p, d_val, d_B, d_C, s);
         arm(i, TCA_PHASE_PANELS);
