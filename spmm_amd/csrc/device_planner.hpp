@@ -93,14 +93,17 @@ __global__ void dp_bounds_kernel(const uint32_t* __restrict__ len, int M, int wi
 // The row order of up to kSmallSortRows rows in one launch: keys, stable
 // descending sort and bounds (dp_lengths_kernel, a radix sort and
 // dp_bounds_kernel together: 11 launches, 52 us at 20,000 rows and gaps
-// between them; here 38 us).  One workgroup: wavefront w owns the w-th sixteenth of the
-// rows, counts its keys in bins of its own (keys of 511 and more share one),
-// the bins are summed over keys (descending) and wavefronts, and each
-// wavefront then places its rows in order, 64 at a time, equal keys of the 64
+// between them).  A workgroup places 1024 rows, 64 per wavefront, and
+// counts the keys of all rows itself, so the workgroups need nothing of each
+// other: bins (keys of 511 and more share one) for each of its wavefronts' rows,
+// for the rows before them and for those after.  The bins are summed over keys
+// (descending) and over the rows before; equal keys of a wavefront's 64 rows are
 // ranked by ballots.  The rows of the shared bin come first and are ranked by
 // comparing all of them; with more than kSmallSortLong of them *over is set
-// and nothing is written (the caller sorts them the general way).
+// and nothing is written (the caller sorts them the general way).  20,000 rows:
+// 18 us; with one workgroup placing all of them 38, most of it the ranking.
 constexpr int kSmallSortRows = 65536, kSmallSortBins = 512, kSmallSortLong = 2048;
+constexpr int kSmallSortRowsPerGroup = 1024;  // its threads
 
 __global__ __launch_bounds__(1024) void dp_sort_small_kernel(const int* __restrict__ rowptr, int M,
                                                              const int* __restrict__ wmap,
@@ -108,34 +111,36 @@ __global__ __launch_bounds__(1024) void dp_sort_small_kernel(const int* __restri
                                                              int row_len, int multi_max, uint32_t* __restrict__ keys,
                                                              int* __restrict__ rows, int* __restrict__ bounds,
                                                              int* __restrict__ over) {
-    __shared__ int bin[16][kSmallSortBins];
+    constexpr int kBefore = 16, kAfter = 17;  // bins of the rows before and after this workgroup's
+    __shared__ int bin[18][kSmallSortBins];
     __shared__ uint32_t lkey[kSmallSortLong];
     __shared__ int lrow[kSmallSortLong];
     __shared__ int nlong, more[4], wsum[16];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int chunk = ((M + 15) / 16 + 63) / 64 * 64;
-    const int r0 = min(M, w * chunk), r1 = min(M, r0 + chunk);
+    const int first = blockIdx.x * kSmallSortRowsPerGroup;  // of this workgroup's rows
     auto key_of = [&](int r) {
         const bool tiles = (wmap && wmap[r / kDmaWinRows] >= 0) || (in_panel && in_panel[r]);
         return tiles ? 0u : static_cast<uint32_t>(rowptr[r + 1] - rowptr[r]) + 1u;
     };
-    for (int i = t; i < 16 * kSmallSortBins; i += 1024) (&bin[0][0])[i] = 0;
+    for (int i = t; i < 18 * kSmallSortBins; i += 1024) (&bin[0][0])[i] = 0;
     if (t == 0) nlong = 0;
     if (t < 4) more[t] = 0;
     __syncthreads();
     const int th[4] = {wide_len, row_len, max(multi_max, 0), 0};
     int n[4] = {0, 0, 0, 0};
     constexpr int kAhead = 8;  // rows loaded at a time
-    for (int rb = r0 + lane; rb < r1; rb += 64 * kAhead) {
+    for (int rb = t; rb < M; rb += 1024 * kAhead) {
         uint32_t ks[kAhead];
 #pragma unroll
-        for (int u = 0; u < kAhead; u++) ks[u] = rb + 64 * u < r1 ? key_of(rb + 64 * u) : 0u;
+        for (int u = 0; u < kAhead; u++) ks[u] = rb + 1024 * u < M ? key_of(rb + 1024 * u) : 0u;
 #pragma unroll
         for (int u = 0; u < kAhead; u++) {
-            const int r = rb + 64 * u;
-            if (r >= r1) break;
+            const int r = rb + 1024 * u;
+            if (r >= M) break;
             const uint32_t k = ks[u];
-            atomicAdd(&bin[w][min(k, kSmallSortBins - 1u)], 1);
+            // (t = r mod 1024: the workgroup's own rows fall to the wavefront that places them)
+            const int of = r < first ? kBefore : r < first + kSmallSortRowsPerGroup ? w : kAfter;
+            atomicAdd(&bin[of][min(k, kSmallSortBins - 1u)], 1);
 #pragma unroll
             for (int q = 0; q < 4; q++) n[q] += static_cast<int64_t>(k) - 1 > th[q];
             if (k >= kSmallSortBins - 1u) {
@@ -152,14 +157,14 @@ __global__ __launch_bounds__(1024) void dp_sort_small_kernel(const int* __restri
         if (n[q]) atomicAdd(&more[q], n[q]);
     __syncthreads();
     if (nlong > kSmallSortLong) {  // (uniform)
-        if (t == 0) *over = 1;
+        if (t == 0 && blockIdx.x == 0) *over = 1;
         return;
     }
-    if (t < 4) bounds[t] = more[t];
+    if (t < 4 && blockIdx.x == 0) bounds[t] = more[t];
     // bins to first positions: thread t has key kSmallSortBins - 1 - t
     int sum = 0;
     if (t < kSmallSortBins)
-        for (int v = 0; v < 16; v++) sum += bin[v][kSmallSortBins - 1 - t];
+        for (int v = 0; v < 18; v++) sum += bin[v][kSmallSortBins - 1 - t];
     int pre = sum;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -169,7 +174,7 @@ __global__ __launch_bounds__(1024) void dp_sort_small_kernel(const int* __restri
     if (lane == 63) wsum[w] = pre;
     __syncthreads();
     if (t < kSmallSortBins) {
-        int at = pre - sum;
+        int at = pre - sum + bin[kBefore][kSmallSortBins - 1 - t];
         for (int v = 0; v < w; v++) at += wsum[v];
         for (int v = 0; v < 16; v++) {
             const int x = bin[v][kSmallSortBins - 1 - t];
@@ -178,32 +183,26 @@ __global__ __launch_bounds__(1024) void dp_sort_small_kernel(const int* __restri
         }
     }
     __syncthreads();
-    volatile int* const mine = bin[w];
-    for (int rb = r0; rb < r1; rb += 64 * kAhead) {
-        uint32_t ks[kAhead];
+    {
+        const int r = first + t;
+        const uint32_t k = r < M ? key_of(r) : ~0u;
+        const bool in = k < kSmallSortBins - 1u;
+        uint64_t same = __ballot(in);  // lanes with the same key
 #pragma unroll
-        for (int u = 0; u < kAhead; u++) ks[u] = rb + 64 * u + lane < r1 ? key_of(rb + 64 * u + lane) : ~0u;
-#pragma unroll
-        for (int u = 0; u < kAhead; u++) {
-            const uint32_t k = ks[u];
-            const bool in = k < kSmallSortBins - 1u;
-            uint64_t same = __ballot(in);  // lanes with the same key
-#pragma unroll
-            for (int bit = 1; bit < kSmallSortBins; bit <<= 1) {
-                const uint64_t set = __ballot((k & bit) != 0);
-                same &= k & bit ? set : ~set;
-            }
-            if (in) {
-                const int pos = mine[k] + __popcll(same & ((1ull << lane) - 1));
-                keys[pos] = k;
-                rows[pos] = rb + 64 * u + lane;
-                if ((same >> lane) == 1) mine[k] = pos + 1;  // the last of them
-            }
+        for (int bit = 1; bit < kSmallSortBins; bit <<= 1) {
+            const uint64_t set = __ballot((k & bit) != 0);
+            same &= k & bit ? set : ~set;
+        }
+        if (in) {
+            const int pos = bin[w][k] + __popcll(same & ((1ull << lane) - 1));
+            keys[pos] = k;
+            rows[pos] = r;
         }
     }
     for (int e = t; e < nlong; e += 1024) {
         const uint32_t k = lkey[e];
         const int r = lrow[e];
+        if (r < first || r >= first + kSmallSortRowsPerGroup) continue;  // another workgroup's
         int pos = 0;
         for (int f = 0; f < nlong; f++) pos += lkey[f] > k || (lkey[f] == k && lrow[f] < r);
         keys[pos] = k;

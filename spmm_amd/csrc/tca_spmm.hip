@@ -1471,7 +1471,7 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         // needs is one allocation (`work`), as are the plan's structure and
         // its row tables: a small structure's planning is allocations,
         // launches and waits (20,000 rows, 270,000 nonzeros, plan, product and
-        // release 319 -> 122 us).
+        // release 319 -> 102 us).
         char* work = nullptr;
         uint32_t *keys = nullptr, *keys_s = nullptr, *bm = nullptr, *ekeys = nullptr, *ekeys_s = nullptr;
         int *rows = nullptr, *rows_s = nullptr, *cnt = nullptr, *nseg = nullptr, *segoff = nullptr;
@@ -1743,7 +1743,7 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         auto sort_rows = [&](const uint8_t* in_panel) -> int {
             const int* const windows = p->mfma.windows.empty() ? nullptr : wmap;
             if (M <= kSmallSortRows) {
-                hipLaunchKernelGGL(dp_sort_small_kernel, dim3(1), dim3(1024), 0, s, p->d_rowptr, M, windows, in_panel,
+                hipLaunchKernelGGL(dp_sort_small_kernel, dim3((M + kSmallSortRowsPerGroup - 1) / kSmallSortRowsPerGroup), dim3(1024), 0, s, p->d_rowptr, M, windows, in_panel,
                                    p->rows.wide_len, p->rows.row_len, p->rows.multi_max, keys_s, rows_s, cnt, cnt + 6);
                 const int e = read_cnt();
                 if (e || !h_cnt[6]) return e;
