@@ -503,10 +503,7 @@ void launch_sddmm_e(const SddmmArgs& a, hipStream_t s) {
     const uint64_t span = 64ull * a.batches * kSddmmWaves;
     const dim3 grid(static_cast<unsigned>((a.nnz + span - 1) / span)), block(64 * kSddmmWaves);
     const int V = (a.N + E - 1) / E;
-    if (a.tasks) {  // beside panels (B rows of at least 64 bytes: 4 pieces and more)
-        const dim3 tgrid((a.ntasks + kSddmmWaves - 1) / kSddmmWaves);
-        if constexpr (E > 1) hipLaunchKernelGGL((sddmm_tasks_kernel<T, E, 8>), tgrid, block, 0, s, a);
-    } else if (V > 4) hipLaunchKernelGGL((sddmm_kernel<T, E, 8>), grid, block, 0, s, a);
+    if (V > 4) hipLaunchKernelGGL((sddmm_kernel<T, E, 8>), grid, block, 0, s, a);
     else if (V > 2) hipLaunchKernelGGL((sddmm_kernel<T, E, 4>), grid, block, 0, s, a);
     else if (V > 1) hipLaunchKernelGGL((sddmm_kernel<T, E, 2>), grid, block, 0, s, a);
     else hipLaunchKernelGGL((sddmm_kernel<T, E, 1>), grid, block, 0, s, a);
@@ -517,6 +514,13 @@ void launch_sddmm(const SddmmArgs& a, hipStream_t s) {
     constexpr int E = 16 / sizeof(T);
     if (a.N >= E) launch_sddmm_e<T, E>(a, s);
     else launch_sddmm_e<T, 1>(a, s);
+}
+
+// The rows beside panels (panel_elems: rows of B of at least 128 bytes, 8 pieces).
+template <typename T>
+void launch_sddmm_tasks(const SddmmArgs& a, hipStream_t s) {
+    const dim3 grid((a.ntasks + kSddmmWaves - 1) / kSddmmWaves), block(64 * kSddmmWaves);
+    hipLaunchKernelGGL((sddmm_tasks_kernel<T, 16 / sizeof(T), 8>), grid, block, 0, s, a);
 }
 
 template <bool kBf16, int RB, int W>
@@ -2101,27 +2105,36 @@ int tca_sddmm(const tca_spmm_plan* p, const float* d_G, const void* d_B, float* 
     a.N = p->N;
     a.nnz = static_cast<uint32_t>(p->nnz);
     a.batches = std::min(std::max(a.nnz / (64 * kSddmmFill), 1u), kSddmmMaxBatches);
-    a.tasks = nullptr;
+    a.tasks = p->d_tasks;
+    a.perm = p->d_perm;
+    a.longrows = p->d_longrows;
+    a.ntasks = p->ntasks;
     // Rows in panels of one column chunk take the panel kernel (its transfers
-    // need B aligned as a product's), the row kernel's rows the gathering one;
-    // with matrix-core windows, whose rows neither has, everything is gathered.
+    // need B aligned as a product's), the row kernel's rows, if they hold any
+    // nonzeros, the gathering one over its tasks; with matrix-core windows,
+    // whose rows neither has, everything is gathered.
     if (p->n_units > 0 && p->panels.chunks == 1 && p->mfma.windows.empty() &&
         reinterpret_cast<uintptr_t>(d_B) % 16 == 0) {
+        const bool others = p->panels.nnz < p->nnz;
         switch (p->dtype) {
-            case TCA_F16: launch_sddmm_panels<_Float16>(p, d_G, d_B, d_out, s); break;
-            case TCA_BF16: launch_sddmm_panels<bf16_t>(p, d_G, d_B, d_out, s); break;
-            default: launch_sddmm_panels<float>(p, d_G, d_B, d_out, s);
+            case TCA_F16:
+                launch_sddmm_panels<_Float16>(p, d_G, d_B, d_out, s);
+                if (others) launch_sddmm_tasks<_Float16>(a, s);
+                break;
+            case TCA_BF16:
+                launch_sddmm_panels<bf16_t>(p, d_G, d_B, d_out, s);
+                if (others) launch_sddmm_tasks<bf16_t>(a, s);
+                break;
+            default:
+                launch_sddmm_panels<float>(p, d_G, d_B, d_out, s);
+                if (others) launch_sddmm_tasks<float>(a, s);
         }
-        a.tasks = p->d_tasks;
-        a.perm = p->d_perm;
-        a.longrows = p->d_longrows;
-        a.ntasks = p->ntasks;
-    }
-    if (!a.tasks || p->panels.nnz < p->nnz)
-    switch (p->dtype) {
-        case TCA_F16: launch_sddmm<_Float16>(a, s); break;
-        case TCA_BF16: launch_sddmm<bf16_t>(a, s); break;
-        default: launch_sddmm<float>(a, s);
+    } else {
+        switch (p->dtype) {
+            case TCA_F16: launch_sddmm<_Float16>(a, s); break;
+            case TCA_BF16: launch_sddmm<bf16_t>(a, s); break;
+            default: launch_sddmm<float>(a, s);
+        }
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(TCA_ERR_HIP, "kernel launch: %s", hipGetErrorString(e));

@@ -1,6 +1,8 @@
 """The sampled product of the backward pass (tca_sddmm) at the widths, row
 lengths and alignments where its split of the nonzeros, its piece columns and
 its partial-sum exchange can go wrong."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -175,6 +177,69 @@ def test_every_task_beside_panels(torch_cuda, monkeypatch, dtype, n):
     if n == 128:  # (narrower B rows go to panels only when asked)
         assert 0 < info["rows_panels"] < len(lens) and info["n_long_rows"] > 0 and info["n_wide_tasks"] > 0
     assert np.array_equal(out.cpu().numpy(), want)
+
+
+def _graph_kernels(torch, call):
+    """Kernel nodes of the graph that `call(stream)` is captured into."""
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g, stream=s):
+        call(s.cuda_stream)
+    hip = ctypes.CDLL(None)  # the runtime is loaded for all
+    graph, n = ctypes.c_void_p(g.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    kinds = []
+    for node in nodes:
+        kind = ctypes.c_int(-1)
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0
+        kinds.append(kind.value)
+    return kinds.count(0)  # hipGraphNodeTypeKernel
+
+
+@pytest.mark.parametrize("on_device", [False, True])
+@pytest.mark.parametrize("dtype", [S.TCA_F32, S.TCA_F16, S.TCA_BF16])
+def test_each_nonzero_computed_once(torch_cuda, monkeypatch, dtype, on_device):
+    """One kernel when every nonzero is in panels, with empty rows (the row
+    kernel's list only clears) and without any (it has no list); one when
+    there are no panels; two when rows lie beside them."""
+    torch = torch_cuda
+    monkeypatch.setenv("TCA_PANEL_MIN_REUSE", "1.5")
+    monkeypatch.setenv("TCA_PANEL_MIN_NNZ", "1")
+    n, k = 128, 600
+    band = [120] * 400
+    rng = np.random.default_rng(5)
+    for lens, flags, panels, kernels in ((band, S.TCA_PLAN_FORCE_PANELS, 400, 1),
+                                         (band + [0] * 9, S.TCA_PLAN_FORCE_PANELS, 400, 1),
+                                         (band, S.TCA_PLAN_NO_PANELS, 0, 1),
+                                         (band + [2] * 300, S.TCA_PLAN_DEFAULT, None, 2)):
+        rowptr, colidx = _pattern(rng, lens, k)
+        m, nnz = len(lens), len(colidx)
+        flags |= S.TCA_PLAN_NO_MFMA
+        if on_device:
+            rp, ci = torch.from_numpy(rowptr).to("cuda:0"), torch.from_numpy(colidx).to("cuda:0")
+            plan = S.Plan.from_device(rp, ci, m, k, nnz, n, dtype, flags)
+        else:
+            plan = S.Plan(S.CSR(m, k, rowptr, colidx, S.to_storage(np.ones(nnz, np.float32), dtype), dtype), n, flags)
+        g, b = exact_dense(rng, (m, n)), exact_dense(rng, (k, n))
+        gd = torch.from_numpy(g).to("cuda:0")
+        bd = torch.from_numpy(b).to("cuda:0").to(getattr(torch, TORCH[dtype]))
+        out = torch.full((nnz,), -1.0, device="cuda:0")
+        with plan:
+            info = plan.info()
+            if panels is None:
+                assert 0 < info["nnz_panels"] < nnz
+            else:
+                assert info["rows_panels"] == panels and (info["n_row_tasks"] == 0) == (panels == m)
+            run = lambda s: S.call("tca_sddmm", plan._p, S._addr(gd), S._addr(bd), S._addr(out), s)
+            run(None)
+            torch.cuda.synchronize()
+            got = out.cpu().numpy()
+            count = _graph_kernels(torch, run)
+        rows = np.repeat(np.arange(m), lens)
+        assert np.array_equal(got, (g[rows].astype(np.float64) * b[colidx]).sum(1).astype(np.float32))
+        assert count == kernels, (len(lens), flags)
 
 
 @pytest.mark.parametrize("n,shift", [(256, 0), (128, 1)])
