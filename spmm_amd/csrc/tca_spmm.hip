@@ -89,7 +89,8 @@ struct tca_spmm_plan {
     int32_t n_perm = 0;       // rows in multi tasks (entries of d_perm)
     bool device_planned = false;
     // Planned on the GPU: the structure (d_rowptr, d_colidx) and the row
-    // tables (d_tasks, d_longrows, d_perm) are one allocation each.
+    // tables (d_tasks, d_longrows, d_perm) each lie in one allocation if that
+    // is a small one (dev_group); null: every array is its own.
     void *d_struct = nullptr, *d_tables = nullptr;
     float* d_partials = nullptr;
     // row panels (panel kernel)
@@ -172,16 +173,60 @@ int dev_upload(T** dst, const void* src, size_t count) {
     return TCA_OK;
 }
 
+// n arrays of the given bytes (null where 0): together in one allocation,
+// *whole, while that is below 2 MiB, else each its own and *whole null.  The
+// runtime keeps blocks below 2 MiB in a pool (1.5 us to allocate and free one)
+// and maps larger ones one by one (15 to 60 us; in a pass that allocates and
+// frees more than some 40 MiB of them another 300 us): 70,000 rows of 9
+// nonzeros, fp16, planned, multiplied and released, 742 us with the planning's
+// arrays in one block of 2.3 MiB, 472 with an allocation each.
+constexpr size_t kPooledBytes = size_t(2) << 20;
+
+template <size_t n>
+int dev_group(const size_t (&bytes)[n], void** whole, void* (&part)[n]) {
+    auto round_up = [](size_t b) { return (b + 255) & ~size_t(255); };
+    size_t total = 0;
+    for (size_t i = 0; i < n; i++) {
+        part[i] = nullptr;
+        total += round_up(bytes[i]);
+    }
+    *whole = nullptr;
+    char* b = nullptr;
+    if (total < kPooledBytes) {
+        if (const int st = dev_upload(&b, nullptr, total)) return st;
+        *whole = b;
+        for (size_t i = 0; i < n; i++) {
+            if (bytes[i] > 0) part[i] = b;
+            b += round_up(bytes[i]);
+        }
+        return TCA_OK;
+    }
+    for (size_t i = 0; i < n; i++) {
+        if (const int st = dev_upload(&b, nullptr, bytes[i])) {
+            for (size_t j = 0; j < i; j++) {
+                (void)hipFree(part[j]);
+                part[j] = nullptr;
+            }
+            return st;
+        }
+        part[i] = b;
+    }
+    return TCA_OK;
+}
+
 void free_plan_device(tca_spmm_plan* p) {
     (void)hipFree(p->d_zeros);
     (void)hipFree(p->d_soff);
     (void)hipFree(p->d_wstart);
-    if (p->device_planned) {
+    if (p->d_struct) {
         (void)hipFree(p->d_struct);
-        (void)hipFree(p->d_tables);
     } else {
         (void)hipFree(p->d_rowptr);
         (void)hipFree(p->d_colidx);
+    }
+    if (p->d_tables) {
+        (void)hipFree(p->d_tables);
+    } else {
         (void)hipFree(p->d_tasks);
         (void)hipFree(p->d_perm);
         (void)hipFree(p->d_longrows);
@@ -1472,11 +1517,11 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         hipStream_t s = static_cast<hipStream_t>(stream);
 
         // Temporaries of the planning, freed on every exit.  What every plan
-        // needs is one allocation (`work`), as are the plan's structure and
-        // its row tables: a small structure's planning is allocations,
-        // launches and waits (20,000 rows, 270,000 nonzeros, plan, product and
-        // release 319 -> 102 us).
-        char* work = nullptr;
+        // needs is one allocation (`work`, dev_group) if that is a small one,
+        // as are the plan's structure and its row tables: a small structure's
+        // planning is allocations, launches and waits (20,000 rows, 270,000
+        // nonzeros, plan, product and release 319 -> 102 us).
+        void *work = nullptr, *wpart[6] = {};
         uint32_t *keys = nullptr, *keys_s = nullptr, *bm = nullptr, *ekeys = nullptr, *ekeys_s = nullptr;
         int *rows = nullptr, *rows_s = nullptr, *cnt = nullptr, *nseg = nullptr, *segoff = nullptr;
         int *wordpre = nullptr, *scnt = nullptr, *wstat = nullptr, *wmap = nullptr, *wgbase = nullptr, *evals = nullptr,
@@ -1488,22 +1533,23 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         int* dpp_rows = nullptr;  // the panels' row order (phase_b reads it after the second sort)
         auto bail = [&](int st) {
             (void)hipStreamSynchronize(s);
-            for (void* q : {(void*)work, (void*)nseg, (void*)segoff, tmp, (void*)bm, (void*)ekeys, (void*)ekeys_s, (void*)wordpre, (void*)scnt,
-                            (void*)wstat, (void*)wmap, (void*)wgbase, (void*)evals, (void*)evals_s, (void*)skey,
+            if (!work)
+                for (void* q : wpart) (void)hipFree(q);
+            for (void* q : {work, (void*)nseg, (void*)segoff, tmp, (void*)bm, (void*)ekeys, (void*)ekeys_s,
+                            (void*)wordpre, (void*)scnt, (void*)wstat, (void*)wmap, (void*)wgbase, (void*)evals, (void*)evals_s, (void*)skey,
                             (void*)skey_s, (void*)sidx, (void*)sidx_s, (void*)dpp_rows})
                 (void)hipFree(q);
             return st;  // on failure `hold` frees the plan
         };
         int st;
-        auto round_up = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
         // The plan owns its copy of the structure (row kernel and SDDMM read it).
         {
-            const size_t rp = round_up(sizeof(int) * (static_cast<size_t>(M) + 1));
-            char* b = nullptr;
-            if ((st = dev_upload(&b, nullptr, rp + sizeof(int) * static_cast<size_t>(nnz)))) return bail(st);
-            p->d_struct = b;
-            p->d_rowptr = reinterpret_cast<int*>(b);
-            if (nnz > 0) p->d_colidx = reinterpret_cast<int*>(b + rp);
+            void* part[2];
+            if ((st = dev_group({sizeof(int) * (static_cast<size_t>(M) + 1), sizeof(int) * static_cast<size_t>(nnz)},
+                                &p->d_struct, part)))
+                return bail(st);
+            p->d_rowptr = static_cast<int*>(part[0]);
+            p->d_colidx = static_cast<int*>(part[1]);
         }
         // Rows are sorted by length + 1, at most min(K, nnz) + 1.
         const unsigned key_bits = 32 - __builtin_clz(static_cast<uint32_t>(std::min(K, nnz)) + 1u);
@@ -1512,19 +1558,20 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
             if (M > kSmallSortRows && rocprim::radix_sort_pairs_desc(nullptr, sort_bytes, keys, keys_s, rows, rows_s,
                                                                      static_cast<size_t>(M), 0, key_bits, s) != hipSuccess)
                 return bail(fail(TCA_ERR_HIP, "radix sort sizing failed"));
-            const size_t ks = round_up(sizeof(int) * static_cast<size_t>(M));
-            const size_t head = round_up(8 * sizeof(int) + static_cast<size_t>(nnz) + 1);
-            if ((st = dev_upload(&work, nullptr, head + 4 * ks + sort_bytes))) return bail(st);
-            cnt = reinterpret_cast<int*>(work);  // [0..3] bounds, [4] error bits, [5] compaction check,
-                                                 // [6] the small sort had too many long rows
-            start = reinterpret_cast<uint8_t*>(work) + 8 * sizeof(int);
-            keys = reinterpret_cast<uint32_t*>(work + head);
-            keys_s = reinterpret_cast<uint32_t*>(work + head + ks);
-            rows = reinterpret_cast<int*>(work + head + 2 * ks);
-            rows_s = reinterpret_cast<int*>(work + head + 3 * ks);
-            if (hipMemsetAsync(work, 0, head, s) != hipSuccess) return bail(fail(TCA_ERR_HIP, "hipMemsetAsync failed"));
+            const size_t ks = sizeof(int) * static_cast<size_t>(M);
+            // (whole words: a fill of odd bytes takes a second kernel, and goes byte by byte)
+            const size_t head = (8 * sizeof(int) + static_cast<size_t>(nnz) + 1 + 255) & ~size_t(255);
+            if ((st = dev_group({head, ks, ks, ks, ks, sort_bytes}, &work, wpart))) return bail(st);
+            cnt = static_cast<int*>(wpart[0]);  // [0..3] bounds, [4] error bits, [5] compaction check,
+                                                // [6] the small sort had too many long rows
+            start = static_cast<uint8_t*>(wpart[0]) + 8 * sizeof(int);
+            keys = static_cast<uint32_t*>(wpart[1]);
+            keys_s = static_cast<uint32_t*>(wpart[2]);
+            rows = static_cast<int*>(wpart[3]);
+            rows_s = static_cast<int*>(wpart[4]);
+            if (hipMemsetAsync(cnt, 0, head, s) != hipSuccess) return bail(fail(TCA_ERR_HIP, "hipMemsetAsync failed"));
         }
-        void* sort_tmp = reinterpret_cast<char*>(rows_s) + round_up(sizeof(int) * static_cast<size_t>(M));
+        void* sort_tmp = wpart[5];
         // CSR checks
         const dim3 blk(256);
         auto grid_for = [](int64_t n) { return dim3(static_cast<unsigned>(std::min<int64_t>((n + 255) / 256, 65536))); };
@@ -1824,14 +1871,15 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         p->n_seg_total = static_cast<size_t>(seg_total) + static_cast<size_t>(dpp.n_segments);
         p->n_perm = n_short;
         {
-            const size_t nt = static_cast<size_t>(p->ntasks), nl = static_cast<size_t>(p->n_longrows);
-            char* b = nullptr;
-            if ((st = dev_upload(&b, nullptr, sizeof(int4) * (nt + nl) + sizeof(int) * static_cast<size_t>(n_short))))
+            void* part[3];
+            if ((st = dev_group({sizeof(int4) * static_cast<size_t>(p->ntasks),
+                                 sizeof(int4) * static_cast<size_t>(p->n_longrows),
+                                 sizeof(int) * static_cast<size_t>(n_short)},
+                                &p->d_tables, part)))
                 return bail(st);
-            p->d_tables = b;
-            if (nt > 0) p->d_tasks = reinterpret_cast<int4*>(b);
-            if (nl > 0) p->d_longrows = reinterpret_cast<int4*>(b) + nt;
-            if (n_short > 0) p->d_perm = reinterpret_cast<int*>(reinterpret_cast<int4*>(b) + nt + nl);
+            p->d_tasks = static_cast<int4*>(part[0]);
+            p->d_longrows = static_cast<int4*>(part[1]);
+            p->d_perm = static_cast<int*>(part[2]);
         }
         if (!(flags & TCA_PLAN_NO_SCRATCH) && (st = dev_upload(&p->d_partials, nullptr, p->n_seg_total * N))) return bail(st);
         if (Mp > 0) {

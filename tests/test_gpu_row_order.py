@@ -57,6 +57,25 @@ def test_many_long_rows(torch_cuda, n_long):
     _same(torch_cuda, _csr(rng, lens, 5100))
 
 
+@pytest.mark.parametrize("m,per_row", [(40000, 12), (40000, 13), (70000, 7), (70000, 20), (300000, 2), (600000, 1)])
+def test_arrays_together_and_apart(torch_cuda, m, per_row):
+    """Structure, temporaries and tables below 2 MiB in one allocation and above
+    it in one each: plans and products equal to the host planner's."""
+    torch = torch_cuda
+    rng = np.random.default_rng(m + per_row)
+    a = _csr(rng, rng.integers(max(per_row - 2, 0), per_row + 3, m), 5000)
+    _same(torch, a)
+    val = torch.from_numpy(rng.choice(np.float32([-1, 1]), a.nnz)).to("cuda:0")
+    b = torch.from_numpy(rng.integers(-9, 9, (5000, 32)).astype(np.float32)).to("cuda:0")
+    rp, ci = torch.from_numpy(a.rowptr).to("cuda:0"), torch.from_numpy(a.colidx).to("cuda:0")
+    c = torch.full((2, m, 32), -1.0, device="cuda:0")
+    with S.Plan(a, 32, FLAGS) as host, S.Plan.from_device(rp, ci, m, 5000, a.nnz, 32, S.TCA_F32, FLAGS) as dev:
+        host.run(val, b, c[0])
+        dev.run(val, b, c[1])
+        torch.cuda.synchronize()
+    assert torch.equal(c[0], c[1])
+
+
 @pytest.mark.parametrize("where", ["rows", "columns", "range"])
 def test_invalid_structures_are_refused(torch_cuda, where):
     torch = torch_cuda
