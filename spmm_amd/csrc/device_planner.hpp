@@ -6,7 +6,7 @@
 //   [0, 4 W)              the 4 quarters of the W wide rows,
 //   [4 W, 4 W + S)        the segments of the long rows (S in all),
 //   [4 W + S, .. + R)     one task per medium row,
-//   then                  groups of multi_group_rows(slots) consecutive short
+//   then                  groups of multi_group_rows() consecutive short
 //                         rows, and groups of kZeroRows empty rows.
 // Long rows come first in the order, then wide, medium and short rows, so
 // the category boundaries are three positions in the sorted lengths.  The

@@ -10,6 +10,7 @@
 // workgroups with an ordered two-kernel sum.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 #include <utility>
 #include <vector>
@@ -22,7 +23,7 @@ constexpr int kXcds = 8;  // XCDs of the MI355X: the hardware deals workgroup b 
 constexpr int64_t kMallBytes = int64_t(256) << 20;  // MI355X Infinity Cache (MALL), shared by the XCDs
 
 // Task kinds of the row kernel (int4 {x, y, z, w}).  Multi tasks hold at most
-// multi_group_rows(slots) rows, walked `slots` at a time, except zero tasks
+// multi_group_rows() rows, walked `slots` at a time, except zero tasks
 // (z == 0), which hold up to kZeroRows empty rows whose C rows the wavefront
 // only clears.
 enum TaskKind : int32_t {
@@ -33,12 +34,27 @@ enum TaskKind : int32_t {
 };
 
 constexpr int32_t kZeroRows = 64;
-// Short rows per multi task: kMultiPasses passes of `slots` rows (one row per
-// slot and pass), at most 64.  Measured on MI355X against one pass per task
-// (config 3's row phase): 2 passes 0.282 ms, 4 passes 0.279, 1 pass 0.297;
-// config 4 191.1 against 192.2 us at 4 passes, 203 us at 8.
+// Short rows per multi task: passes of `slots` rows (one row per slot and
+// pass), at most kMultiPasses of them and 64 rows.  A pass waits for three
+// loads in a row or more, so several only pay where the tasks are enough for
+// the chip all the same: at least kMultiTasks of them, or so many others
+// (row, wide and segment tasks) beside few short rows that these end long
+// before.  us per product at one / four passes on the MI355X: a 300 x 200
+// layer of 2 %, fp32 N = 47 3.1 / 5.4, bf16 4.2 / 9.8; 12,000 x 1000 of 2 %,
+// fp32 N = 17 6.8 / 10.4, fp16 N = 48 8.8 / 12.6; R-MAT of 10,000 nodes and
+// 110,000 nonzeros, fp32 N = 18 8.2 / 11.0; of 200,000 and 3.4M, N = 20 48.4 /
+// 52.1; 60,000 rows of 5, N = 32 8.6 / 9.3; of 1.5M and 17M, N = 20 346 / 339; of
+// 2.4M and 64M, N = 47 2101 / 2084; 2^20 rows, 20M nonzeros in 15,000 of them,
+// fp16 N = 64 (23,000 other tasks, 1600 of short rows) 171.0 / 169.2; 100,000
+// rows of the kind, N = 48 (4200 and 270) 17.6 / 24.2.
 constexpr int32_t kMultiPasses = 4;
-inline int32_t multi_group_rows(int32_t slots) { return slots * kMultiPasses < 64 ? slots * kMultiPasses : 64; }
+constexpr int64_t kMultiTasks = 16384;
+inline int32_t multi_group_rows(int32_t slots, int64_t n_short, int64_t n_other) {
+    const int64_t tasks = n_short / slots;  // of one pass
+    const bool hidden = n_other >= kMultiTasks && n_other >= 8 * tasks;
+    const int64_t passes = hidden ? kMultiPasses : std::clamp<int64_t>(tasks / kMultiTasks, 1, kMultiPasses);
+    return static_cast<int32_t>(std::min<int64_t>(64, slots * passes));
+}
 
 // Widths whose widest dividing vector is one or two elements take whole
 // 16-byte vectors instead, the last one ending at the row's end

@@ -1513,7 +1513,6 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         p->mfma.row_mfma.clear();
         if (hipGetDevice(&p->device) != hipSuccess) return fail(TCA_ERR_HIP, "no HIP device");
         plan_row_params(M, nnz, N, static_cast<int32_t>(dtype_size(dtype)), default_slices(K, N, dtype), &p->rows);
-        const int group = multi_group_rows(64 >> p->rows.log_lanes);  // rows per multi task
         hipStream_t s = static_cast<hipStream_t>(stream);
 
         // Temporaries of the planning, freed on every exit.  What every plan
@@ -1861,6 +1860,8 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
                 return bail(fail(TCA_ERR_HIP, "segment scan failed"));
         }
         const int n_wide = end_wide - n_long, n_row = end_row - end_wide, n_short = Mp - end_row;
+        const int group = multi_group_rows(64 >> p->rows.log_lanes, end_nz - end_row,
+                                           4ll * n_wide + seg_total + n_row);  // rows per multi task
         const int n_multi = (end_nz - end_row + group - 1) / group + (Mp - end_nz + kZeroRows - 1) / kZeroRows;
         p->ntasks = 4 * n_wide + seg_total + n_row + n_multi;
         p->rows.n_wide = 4 * n_wide;
