@@ -67,13 +67,21 @@ int32_t padded_pitch(int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t fla
     if (const char* f = std::getenv("TCA_PAD")) return std::atoi(f) ? static_cast<int32_t>(pitch) : 0;
     if (!to_lines && !(es == 2 && N % 2 == 1)) return 0;
     const bool far = static_cast<int64_t>(K) * N * es > kPadFarBytes;
-    const double saved = (far ? kPadFarGain : es == 2 ? kPadNearGain : 0.0) * static_cast<double>(nnz) * N * es;
+    const int64_t row = static_cast<int64_t>(N) * es;
+    const double saved = static_cast<double>(nnz) * (far       ? kPadFarGain * std::min(row, kPadFarRow)
+                                                     : es == 2 ? kPadNearGain * row
+                                                               : 0.0);
     const double cost = kPadFixedUs + 2.0 * static_cast<double>(bytes) / kPadBytesPerUs;
     return saved > (on_device ? 1.5 : 1.0) * cost ? static_cast<int32_t>(pitch) : 0;
 }
 
-void plan_row_params(int32_t M, int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan* p) {
+void plan_row_params(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t flags, int32_t slices,
+                     RowPlan* p) {
     plan_geometry(N, es, slices, p);
+    // (the stricter rule for the copy on both sides: plans made on the device equal the host's)
+    if (p->ragged && slices == 0 && nnz < kRaggedChunkReuse * K &&
+        padded_pitch(K, nnz, N, es, flags, true, *p) == 0)
+        plan_geometry(N, es, N * es > 512 && static_cast<int64_t>(K) * N * es <= kRaggedTwoChunkBytes ? 2 : 1, p);
     const int32_t slots = 64 >> p->log_lanes;
     // Work per wavefront task: about nnz / 32768 nonzeros (four resident
     // wavefronts on each of 256 CUs x 4 SIMDs x 8 slots, so long rows do
@@ -112,9 +120,9 @@ void plan_row_params(int32_t M, int64_t nnz, int32_t N, int32_t es, int32_t slic
     if (const char* s = std::getenv("TCA_MULTI")) p->multi_max = slots > 1 ? std::atoi(s) : -1;
 }
 
-void plan_rows(const int32_t* rowptr, int32_t M, int32_t N, int32_t es, const std::vector<uint8_t>& skip,
-               int32_t slices, RowPlan* p) {
-    plan_row_params(M, rowptr[M], N, es, slices, p);
+void plan_rows(const int32_t* rowptr, int32_t M, int32_t K, int32_t N, int32_t es, uint32_t flags,
+               const std::vector<uint8_t>& skip, int32_t slices, RowPlan* p) {
+    plan_row_params(M, K, rowptr[M], N, es, flags, slices, p);
     const int32_t slots = 64 >> p->log_lanes;
 
     std::vector<int32_t> rows;
@@ -736,7 +744,8 @@ extern "C" int tca_plan_row_tasks(const int32_t* rowptr, int32_t M, int32_t K, i
         if (!rowptr || M < 0 || K < 1 || N < 1 || !dtype_ok(dtype) || !n_tasks || !n_perm || !n_long)
             return fail(TCA_ERR_INVALID, "tca_plan_row_tasks: bad argument");
         RowPlan p;
-        plan_rows(rowptr, M, N, static_cast<int32_t>(dtype_size(dtype)), {}, default_slices(K, N, dtype), &p);
+        plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), TCA_PLAN_DEFAULT, {},
+                  default_slices(K, N, dtype), &p);
         if (tasks) {
             if (*n_tasks < static_cast<int32_t>(p.tasks.size()) || *n_perm < static_cast<int32_t>(p.perm.size()) ||
                 *n_long < static_cast<int32_t>(p.longrows.size()) || !perm || !longrows)
@@ -807,7 +816,8 @@ extern "C" int tca_plan_launch_orders(const int32_t* rowptr, const int32_t* coli
         std::vector<uint8_t> skip(M, 0);
         for (int32_t r = 0; r < M; r++) skip[r] = (!mp.row_mfma.empty() && mp.row_mfma[r]) || pp.row_panel[r];
         RowPlan rp;
-        plan_rows(rowptr, M, N, static_cast<int32_t>(dtype_size(dtype)), skip, default_slices(K, N, dtype), &rp);
+        plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), flags, skip, default_slices(K, N, dtype),
+                  &rp);
         order_row_tasks(colidx, &rp);
         if (panel_order) {
             if (*n_blocks < static_cast<int32_t>(pp.order.size()) || *n_tasks < static_cast<int32_t>(rp.tasks.size()) ||

@@ -74,17 +74,34 @@ constexpr int32_t kRaggedMinN16 = 33;
 // dwords and gained nothing).  Copied when the time saved, by gathered bytes,
 // passes the copy's; by half as much again for plans made on the device, which
 // may run once.  us per product in place -> copied (copy included) on the
-// MI355X: 3001 x 2049 layer of 8 %, bf16 N = 47 11.0 -> 9.8, N = 333 38.2 ->
-// 29.2, N = 1023 75 -> 48, fp32 N = 333 32 -> 37; R-MAT of 200,000 nodes and
-// 6.7M nonzeros, fp16 N = 47 135 -> 106, N = 70 128 -> 135, N = 127 310 -> 199,
-// fp32 N = 47 127 -> 127, N = 101 296 -> 320, N = 127 504 -> 325; of 20,000
-// nodes and 372k, fp16 N = 255 40 -> 43, fp32 50 -> 55; Zipf rows, 300,000
-// columns, fp16 N = 127 3.7M nonzeros 368 -> 278, N = 47 0.9M 48 -> 58.
+// MI355X: 3001 x 2049 layer of 8 %, bf16 N = 47 11.2 -> 9.8, N = 333 36 -> 27,
+// N = 1023 76 -> 47, fp32 N = 333 32 -> 36; R-MAT of 300,000 nodes and 10M
+// nonzeros, fp16 N = 47 179 -> 140, N = 127 439 -> 294, N = 255 757 -> 613, fp32
+// N = 62 235 -> 251, N = 127 771 -> 544; of 100,000 and 3.4M, fp16 N = 127 88 ->
+// 97, fp32 N = 127 182 -> 155, N = 255 351 -> 309; of 30,000 and 1M, fp32 N = 255
+// 63 -> 91; Zipf rows, 300,000 columns, 3M, fp16 N = 47 84 -> 79, N = 127 139 ->
+// 253.
 constexpr int64_t kPadFarBytes = int64_t(24) << 20;  // a B past this comes from behind the L2s:
-constexpr double kPadFarGain = 6e-8;     // us saved per gathered byte (measured 4e-8 to 19e-8)
-constexpr double kPadNearGain = 3e-8;    // and within it, 16-bit types (2.5e-8 to 6e-8; fp32 none)
+constexpr double kPadFarGain = 4e-8;     // us saved per gathered byte (measured 1e-8 to 6.5e-8),
+constexpr int64_t kPadFarRow = 640;      // of rows of at most so many bytes (a wider one too saves one line),
+constexpr double kPadNearGain = 3e-8;    // and within them, 16-bit types (2.5e-8 to 6e-8; fp32 none)
 constexpr double kPadFixedUs = 3.0;      // the copy's launch,
 constexpr double kPadBytesPerUs = 4e6;   // and its rate, each byte read and written
+
+// Column chunks of ragged rows read in place end inside lines, and with the
+// 128-byte chunks of a wide B a row then costs up to twice its lines: they
+// take one chunk (two of a small B whose rows fill a wavefront, for the
+// parallelism) unless every row of B is gathered so often that the XCDs'
+// slices of B pay.  us per product with the chunks of aligned rows / with one
+// on the MI355X (before, with vectors that divide N, in brackets): Zipf rows of
+// 100,000 columns, 1M nonzeros, fp32 N = 63 80 / 30 (34), N = 127 153 / 54 (116),
+// fp16 N = 126 92 / 37 (38); 300,000 columns, 3M, fp32 N = 255 991 / 375 (723);
+// R-MAT of 300,000 nodes and 3.5M, fp32 N = 62 158 / 113 (133), N = 127 404 / 326
+// (384); of 10,000 and 110,000, N = 255 19.4, 23.5 with one and 17.2 with two (21);
+// an 8000 x 8000 layer of 5 % (B's rows 400 times), fp32 N = 333 230 / 259, N =
+// 1023 689 / 1063, bf16 N = 333 200 / 200.
+constexpr int64_t kRaggedChunkReuse = 128;
+constexpr int64_t kRaggedTwoChunkBytes = int64_t(16) << 20;
 
 struct Int4 {
     int32_t x, y, z, w;
@@ -185,7 +202,8 @@ int32_t padded_pitch(int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t fla
 
 // Lane geometry and task-length thresholds (row_len, wide_len, seg_len,
 // multi_max) of the row kernel for a matrix of nnz nonzeros.
-void plan_row_params(int32_t M, int64_t nnz, int32_t N, int32_t es, int32_t slices, RowPlan* p);
+void plan_row_params(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t flags, int32_t slices,
+                     RowPlan* p);
 
 // Row panels with B rows staged in LDS (the panel kernel).  Rows are taken
 // longest first (ties by row id) in panels of R = waves * 4 * rpg rows; the
@@ -332,8 +350,8 @@ struct WinStat {
 void route_windows(const std::vector<WinStat>& st, int32_t M, int64_t nnz_total, int32_t N, bool force,
                    double min_density, const MfmaShape& shape, std::vector<uint8_t>* take);
 
-void plan_rows(const int32_t* rowptr, int32_t M, int32_t N, int32_t es, const std::vector<uint8_t>& skip,
-               int32_t slices, RowPlan* p);
+void plan_rows(const int32_t* rowptr, int32_t M, int32_t K, int32_t N, int32_t es, uint32_t flags,
+               const std::vector<uint8_t>& skip, int32_t slices, RowPlan* p);
 
 // Sorted column union of every window of `win` rows and each nonzero's
 // position in it (the indexing exported by tca_condense_windows).

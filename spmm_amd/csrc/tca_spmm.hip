@@ -975,8 +975,8 @@ int tca_spmm_plan_create(const int32_t* rowptr, const int32_t* colidx, int32_t M
         std::vector<uint8_t> skip_rows(M, p->mfma_short ? 1 : 0);
         for (int32_t r = 0; r < M && !p->mfma_short; r++)
             skip_rows[r] = (!p->mfma.row_mfma.empty() && p->mfma.row_mfma[r]) || p->panels.row_panel[r];
-        plan_rows(rowptr, M, N, static_cast<int32_t>(dtype_size(dtype)), skip_rows, default_slices(K, N, dtype),
-                  &p->rows);
+        plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), flags, skip_rows,
+                  default_slices(K, N, dtype), &p->rows);
         order_row_tasks(colidx, &p->rows);
         p->ntasks = static_cast<int32_t>(p->rows.tasks.size());
         const size_t n_seg_rows =
@@ -1512,7 +1512,8 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         p->device_planned = true;
         p->mfma.row_mfma.clear();
         if (hipGetDevice(&p->device) != hipSuccess) return fail(TCA_ERR_HIP, "no HIP device");
-        plan_row_params(M, nnz, N, static_cast<int32_t>(dtype_size(dtype)), default_slices(K, N, dtype), &p->rows);
+        plan_row_params(M, K, nnz, N, static_cast<int32_t>(dtype_size(dtype)), flags, default_slices(K, N, dtype),
+                        &p->rows);
         hipStream_t s = static_cast<hipStream_t>(stream);
 
         // Temporaries of the planning, freed on every exit.  What every plan
