@@ -34,11 +34,12 @@ namespace tca {
 
 // CSR checks of tca_csr_validate: rowptr[0] == 0, rowptr[M] == nnz,
 // non-decreasing, columns in [0, K) and strictly ascending within a row.  Both
-// copy what they check to the plan (`copy`).
+// copy what they check to the plan (`copy`); *longest (if given): the longest row.
 // err bit 1: row offsets, bit 2: a column.  `start` marks the first entry of
 // every non-empty row (nnz + 1 bytes, zeroed by the caller).
 __global__ void dp_check_rows_kernel(const int* __restrict__ rowptr, int M, int nnz, uint8_t* __restrict__ start,
-                                     int* __restrict__ err, int* __restrict__ copy) {
+                                     int* __restrict__ err, int* __restrict__ copy, int* __restrict__ longest) {
+    int len = 0;
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < M; r += gridDim.x * blockDim.x) {
         const int b = rowptr[r], e = rowptr[r + 1];
         copy[r] = b;
@@ -48,6 +49,12 @@ __global__ void dp_check_rows_kernel(const int* __restrict__ rowptr, int M, int 
             continue;
         }
         if (b < e) start[b] = 1;
+        len = max(len, e - b);
+    }
+    if (longest) {
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) len = max(len, __shfl_xor(len, d));
+        if ((threadIdx.x & 63) == 0) atomicMax(longest, len);
     }
 }
 

@@ -34,10 +34,10 @@ int32_t default_slices(int32_t K, int32_t N, int32_t dtype) {
     return b_bytes > (8ull << 20) ? 0 : 1;
 }
 
-void plan_geometry(int32_t N, int32_t es, int32_t slices, RowPlan* p) {
+void plan_geometry(int32_t N, int32_t es, int32_t slices, bool short_rows, RowPlan* p) {
     int32_t e = 16 / es;
     while (e > 1 && N % e != 0) e >>= 1;
-    p->ragged = e < 4 && N >= (es == 4 ? kRaggedMinN32 : kRaggedMinN16);
+    p->ragged = e < 4 && N >= (es == 4 ? kRaggedMinN32 : kRaggedMinN16) && !short_rows;
     if (p->ragged) e = 16 / es;
     p->elems_per_lane = e;
     const int64_t lanes = (N + e - 1) / e;  // 16-byte (or narrower) vectors across one B row
@@ -75,13 +75,21 @@ int32_t padded_pitch(int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t fla
     return saved > (on_device ? 1.5 : 1.0) * cost ? static_cast<int32_t>(pitch) : 0;
 }
 
+bool short_rows_matter(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es) {
+    const int32_t e = N % 2 == 0 ? 2 : 1;  // the dividing vector
+    return es == 2 && N % 4 != 0 && N >= kRaggedMinN16 && N <= 64 * e && K <= kShortRowCols && nnz <= kShortRowNnz * M;
+}
+
 void plan_row_params(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t flags, int32_t slices,
-                     RowPlan* p) {
-    plan_geometry(N, es, slices, p);
+                     int32_t longest, RowPlan* p) {
+    const bool short_rows =
+        short_rows_matter(M, K, nnz, N, es) && static_cast<int64_t>(longest) * M <= 2 * nnz + kShortRowMore * M;
+    plan_geometry(N, es, slices, short_rows, p);
     // (the stricter rule for the copy on both sides: plans made on the device equal the host's)
     if (p->ragged && slices == 0 && nnz < kRaggedChunkReuse * K &&
         padded_pitch(K, nnz, N, es, flags, true, *p) == 0)
-        plan_geometry(N, es, N * es > 512 && static_cast<int64_t>(K) * N * es <= kRaggedTwoChunkBytes ? 2 : 1, p);
+        plan_geometry(N, es, N * es > 512 && static_cast<int64_t>(K) * N * es <= kRaggedTwoChunkBytes ? 2 : 1,
+                      short_rows, p);
     const int32_t slots = 64 >> p->log_lanes;
     // Work per wavefront task: about nnz / 32768 nonzeros (four resident
     // wavefronts on each of 256 CUs x 4 SIMDs x 8 slots, so long rows do
@@ -122,7 +130,10 @@ void plan_row_params(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es, u
 
 void plan_rows(const int32_t* rowptr, int32_t M, int32_t K, int32_t N, int32_t es, uint32_t flags,
                const std::vector<uint8_t>& skip, int32_t slices, RowPlan* p) {
-    plan_row_params(M, K, rowptr[M], N, es, flags, slices, p);
+    int32_t longest = 0;
+    if (short_rows_matter(M, K, rowptr[M], N, es))
+        for (int32_t r = 0; r < M; r++) longest = std::max(longest, rowptr[r + 1] - rowptr[r]);
+    plan_row_params(M, K, rowptr[M], N, es, flags, slices, longest, p);
     const int32_t slots = 64 >> p->log_lanes;
 
     std::vector<int32_t> rows;

@@ -68,6 +68,24 @@ inline int32_t multi_group_rows(int32_t slots, int64_t n_short, int64_t n_other)
 constexpr int32_t kRaggedMinN32 = 16;
 constexpr int32_t kRaggedMinN16 = 33;
 
+// Where every row is short and B is small, a wavefront of the dividing vectors
+// of 16-bit types (N <= 64 of them) reads its row in a few steps, with nothing
+// to add across slots, and they stay.  us per product on the MI355X, dividing
+// against whole vectors, uniform layers: 300 x 200 of 2 % (4 a row), N = 33 2.8 /
+// 3.8, N = 70 2.8 / 3.5; 5000 x 500 of 2 % (10), N = 47 4.1 / 5.1, N = 81 (two
+// wavefronts' widths) 5.5 / 5.7; 12,000 x 1000 of 2 % (20), N = 34 6.9 / 9.1, N = 47
+// 7.7 / 10.7, N = 70 8.0 / 9.6; of 4 % (40), N = 47 11.3 / 12.7, N = 70 11.9 / 11.6;
+// 3000 x 2000 of 4 % (80), N = 34 6.4 / 6.0, N = 47 7.7 / 7.8; with rows of up to
+// some 300 among 20, N = 47 14.2 / 9.4, of up to 60 among 4, 7.7 / 4.1.  60,000
+// sampled rows of 5 of 240,000, N = 47 18.6 / 15.2.  fp32 gains from whole vectors
+// there too (12,000 x 300 of 2 %, N = 47 7.2 / 4.9), but for the smallest (300 x
+// 200 of 2 % 2.8 / 3.1).
+constexpr int32_t kShortRowCols = 2048;
+constexpr int64_t kShortRowNnz = 48;   // nonzeros a row on average,
+constexpr int64_t kShortRowMore = 12;  // and at most twice as many and these
+// Whether the longest row decides the vectors (K, the average and N fit).
+bool short_rows_matter(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es);
+
 // Ragged rows gathered often enough are copied to an aligned pitch first
 // (padded_pitch): to whole 128-byte lines where that adds at most an eighth,
 // else to whole vectors (16-bit types of odd N; the others' vectors start at
@@ -193,7 +211,8 @@ int32_t default_slices(int32_t K, int32_t N, int32_t dtype);
 // (<= 16 bytes) whose element count divides N, and the column chunks: up to
 // 8 chunks of at least 128 bytes (one L2 line of B per chunk row), at most
 // 64 lanes each.  `slices` > 0 forces the number of chunks (tuning).
-void plan_geometry(int32_t N, int32_t es, int32_t slices, RowPlan* p);
+// short_rows: ragged widths keep the vectors that divide them.
+void plan_geometry(int32_t N, int32_t es, int32_t slices, bool short_rows, RowPlan* p);
 
 // Ragged rows (RowPlan::ragged) of B that a plan copies to an aligned pitch
 // before each product: elements per row of the copy, 0 = read B in place
@@ -202,8 +221,9 @@ int32_t padded_pitch(int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t fla
 
 // Lane geometry and task-length thresholds (row_len, wide_len, seg_len,
 // multi_max) of the row kernel for a matrix of nnz nonzeros.
+// longest: the longest row's nonzeros, read where short_rows_matter.
 void plan_row_params(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es, uint32_t flags, int32_t slices,
-                     RowPlan* p);
+                     int32_t longest, RowPlan* p);
 
 // Row panels with B rows staged in LDS (the panel kernel).  Rows are taken
 // longest first (ties by row id) in panels of R = waves * 4 * rpg rows; the

@@ -1512,8 +1512,8 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         p->device_planned = true;
         p->mfma.row_mfma.clear();
         if (hipGetDevice(&p->device) != hipSuccess) return fail(TCA_ERR_HIP, "no HIP device");
-        plan_row_params(M, K, nnz, N, static_cast<int32_t>(dtype_size(dtype)), flags, default_slices(K, N, dtype),
-                        &p->rows);
+        const int32_t es = static_cast<int32_t>(dtype_size(dtype));
+        const bool need_longest = short_rows_matter(M, K, nnz, N, es);
         hipStream_t s = static_cast<hipStream_t>(stream);
 
         // Temporaries of the planning, freed on every exit.  What every plan
@@ -1563,7 +1563,7 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
             const size_t head = (8 * sizeof(int) + static_cast<size_t>(nnz) + 1 + 255) & ~size_t(255);
             if ((st = dev_group({head, ks, ks, ks, ks, sort_bytes}, &work, wpart))) return bail(st);
             cnt = static_cast<int*>(wpart[0]);  // [0..3] bounds, [4] error bits, [5] compaction check,
-                                                // [6] the small sort had too many long rows
+                                                // [6] the small sort had too many long rows, [7] longest row
             start = static_cast<uint8_t*>(wpart[0]) + 8 * sizeof(int);
             keys = static_cast<uint32_t*>(wpart[1]);
             keys_s = static_cast<uint32_t*>(wpart[2]);
@@ -1576,14 +1576,15 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         const dim3 blk(256);
         auto grid_for = [](int64_t n) { return dim3(static_cast<unsigned>(std::min<int64_t>((n + 255) / 256, 65536))); };
         if (M > 0) {
-            hipLaunchKernelGGL(dp_check_rows_kernel, grid_for(M), blk, 0, s, d_rowptr, M, nnz, start, cnt + 4, p->d_rowptr);
+            hipLaunchKernelGGL(dp_check_rows_kernel, grid_for(M), blk, 0, s, d_rowptr, M, nnz, start, cnt + 4, p->d_rowptr,
+                               need_longest ? cnt + 7 : nullptr);
             if (nnz > 0)
                 hipLaunchKernelGGL(dp_check_cols_kernel, grid_for(nnz), blk, 0, s, d_colidx, nnz, K, start, cnt + 4,
                                    p->d_colidx);
         } else if (hipMemcpyAsync(p->d_rowptr, d_rowptr, sizeof(int), hipMemcpyDeviceToDevice, s) != hipSuccess) {
             return bail(fail(TCA_ERR_HIP, "structure copy failed"));
         }
-        int h_cnt[7] = {};
+        int h_cnt[8] = {};
         auto read_cnt = [&]() -> int {  // waits; the checks' verdict first
             if (hipMemcpyAsync(h_cnt, cnt, sizeof h_cnt, hipMemcpyDeviceToHost, s) != hipSuccess ||
                 hipStreamSynchronize(s) != hipSuccess)
@@ -1595,7 +1596,8 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         // The columns index the window bitmaps and the short-K tiles: wait for
         // the checks there.  Sorting row lengths needs no valid structure.
         const bool maybe_mfma = (flags & TCA_PLAN_NO_MFMA) == 0 && dtype != TCA_F32 && N % 8 == 0;
-        if ((maybe_mfma || M == 0) && (st = read_cnt())) return bail(st);
+        if ((maybe_mfma || need_longest || M == 0) && (st = read_cnt())) return bail(st);
+        plan_row_params(M, K, nnz, N, es, flags, default_slices(K, N, dtype), h_cnt[7], &p->rows);
         if (short_route(M, K, nnz, N, dtype, flags)) {
             // short K: every row on the short-K kernel, which needs only the structure
             p->mfma_short = true;

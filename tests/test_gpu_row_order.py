@@ -12,11 +12,12 @@ pytestmark = pytest.mark.gpu
 FLAGS = S.TCA_PLAN_NO_MFMA | S.TCA_PLAN_NO_PANELS
 
 
-def _csr(rng, lens, k):
+def _csr(rng, lens, k, dtype=S.TCA_F32):
     rowptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     starts = rng.integers(0, k - np.asarray(lens) + 1)
     colidx = np.concatenate([np.arange(s, s + n) for s, n in zip(starts, lens)] + [np.zeros(0)]).astype(np.int32)
-    return S.CSR(len(lens), k, rowptr, colidx, np.zeros(len(colidx), np.float32), S.TCA_F32)
+    return S.CSR(len(lens), k, rowptr, colidx, S.to_storage(np.zeros(len(colidx), np.float32), dtype),
+                 dtype)
 
 
 def _same(torch, a, n=32):
@@ -24,7 +25,7 @@ def _same(torch, a, n=32):
         want, order = host.export_rows(), host.export_order()
     rp = torch.from_numpy(a.rowptr).to("cuda:0")
     ci = torch.from_numpy(a.colidx if a.nnz else np.zeros(1, np.int32)).to("cuda:0")
-    with S.Plan.from_device(rp, ci, a.nrow, a.ncol, a.nnz, n, S.TCA_F32, FLAGS) as dev:
+    with S.Plan.from_device(rp, ci, a.nrow, a.ncol, a.nnz, n, a.dtype, FLAGS) as dev:
         got, got_order = dev.export_rows(), dev.export_order()
     for x, y in zip(want, got):
         assert np.array_equal(x, y)
@@ -55,6 +56,21 @@ def test_many_long_rows(torch_cuda, n_long):
     rng.shuffle(lens)
     lens[lens == 510] = 511
     _same(torch_cuda, _csr(rng, lens, 5100))
+
+
+@pytest.mark.parametrize("longest,elems", [(20, 1), (26, 8)])
+def test_vectors_by_the_longest_row(torch_cuda, longest, elems):
+    """The longest row, which decides the vectors of short-row plans, is found on
+    the GPU as on the host, in the first rows and in the last."""
+    rng = np.random.default_rng(longest)
+    for m, at in ((3, 2), (70, 0), (5000, 4999), (70000, 66000)):
+        lens = rng.integers(4, 7, m)
+        lens[at] = longest
+        a = _csr(rng, lens, 1000, S.TCA_F16)
+        if m > 3:
+            with S.Plan(a, 47, FLAGS) as plan:
+                assert plan.info()["elems_per_lane"] == elems
+        _same(torch_cuda, a, 47)
 
 
 @pytest.mark.parametrize("m,per_row", [(40000, 12), (40000, 13), (70000, 7), (70000, 20), (300000, 2), (600000, 1)])
