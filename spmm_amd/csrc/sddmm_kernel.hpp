@@ -204,6 +204,49 @@ __global__ __launch_bounds__(64 * kSddmmWaves, 4) void sddmm_kernel(SddmmArgs a)
     }
 }
 
+// The same for few nonzeros and wide rows, where batches of 64 leave the chip
+// idle: a wavefront per nonzero, lane l on pieces l, l + 64, ... of its rows.
+// A piece's products in fp32 (chains of four), everything else in fp64.  us at
+// N columns, batches / a wavefront each (one wavefront per row, before both, in
+// brackets), fp32: 1200 nonzeros in 300 rows, N = 64 4.4 / 3.8 (4.0), N = 256 8.6 /
+// 3.9 (5.1), N = 1024 24.8 / 4.5 (11.5), N = 4096 151 / 4.6 (42); 8000 in 1000, N = 64
+// 3.8 / 4.8 (6.1), N = 256 5.6 / 4.8 (8.1), N = 1024 17.0 / 6.3 (24); 40,000 in 4000, N
+// = 256 14.3 / 14.6 (13.2), N = 512 26.4 / 18.9 (31), N = 1024 48 / 28 (60); 80,000 in
+// 2000, N = 512 14.8 / 32; bf16: 40,000, N = 512 11.8 / 17.2 (27), N = 1024 20.1 / 22.8
+// (60).  A batch takes about 0.085 us a piece of its rows and a wavefront per
+// nonzero 0.2 us per 1000 of them.
+inline bool sddmm_wide(uint32_t nnz, int pieces) {
+    return pieces >= 16 && nnz <= 65536u && nnz <= 256u * static_cast<uint32_t>(pieces);
+}
+
+template <typename T, int E>
+__global__ __launch_bounds__(64 * kSddmmWaves) void sddmm_wide_kernel(SddmmArgs a) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t j = blockIdx.x * kSddmmWaves + (threadIdx.x >> 6);
+    if (j >= a.nnz) return;
+    const float* const g = a.G + static_cast<size_t>(wave_row_of(a.rowptr, j, a.M, lane)) * a.N;
+    const T* const b = static_cast<const T*>(a.B) + static_cast<size_t>(a.colidx[j]) * a.N;
+    const int V = (a.N + E - 1) / E;
+    double acc = 0.;
+#pragma unroll 4
+    for (int p = lane; p < V; p += 64) {
+        const int at = min(p * E, a.N - E), skip = p * E - at;  // the last piece ends at the row's end
+        const Pack<float, E> x = load_unaligned<float, E>(g + at);
+        const Pack<T, E> y = load_unaligned<T, E>(b + at);
+        float t[(E + 3) / 4];
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            float s = e % 4 == 0 ? x.v[e] * to_f32(y.v[e]) : __builtin_fmaf(x.v[e], to_f32(y.v[e]), t[e / 4]);
+            if (skip > e) s = 0.f;
+            t[e / 4] = s;
+        }
+        acc += static_cast<double>(E == 8 ? t[0] + t[E / 8] : t[0]);
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d);
+    if (lane == 0) a.out[j] = static_cast<float>(acc);
+}
+
 // The same for the rows of the row kernel's task list (those outside the row
 // panels, whose nonzeros lie scattered through the CSR): a wavefront per task;
 // a group of short rows is walked nonzero by nonzero, 64 at a time.

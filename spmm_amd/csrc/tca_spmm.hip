@@ -548,6 +548,13 @@ void launch_sddmm_e(const SddmmArgs& a, hipStream_t s) {
     const uint64_t span = 64ull * a.batches * kSddmmWaves;
     const dim3 grid(static_cast<unsigned>((a.nnz + span - 1) / span)), block(64 * kSddmmWaves);
     const int V = (a.N + E - 1) / E;
+    if constexpr (E > 1) {
+        if (sddmm_wide(a.nnz, V)) {
+            const dim3 wgrid((a.nnz + kSddmmWaves - 1) / kSddmmWaves);
+            hipLaunchKernelGGL((sddmm_wide_kernel<T, E>), wgrid, block, 0, s, a);
+            return;
+        }
+    }
     if (V > 4) hipLaunchKernelGGL((sddmm_kernel<T, E, 8>), grid, block, 0, s, a);
     else if (V > 2) hipLaunchKernelGGL((sddmm_kernel<T, E, 4>), grid, block, 0, s, a);
     else if (V > 1) hipLaunchKernelGGL((sddmm_kernel<T, E, 2>), grid, block, 0, s, a);

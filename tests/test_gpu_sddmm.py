@@ -105,6 +105,41 @@ def test_non_finite_rows_stay_in_their_products(torch_cuda):
     assert torch.equal(torch.nan_to_num(out, 1.0, 2.0, 3.0), torch.nan_to_num(want, 1.0, 2.0, 3.0))
 
 
+@pytest.mark.parametrize("dtype,n", [(S.TCA_F32, 60), (S.TCA_F32, 61), (S.TCA_F32, 64), (S.TCA_F32, 255), (S.TCA_F32, 257),
+                                     (S.TCA_F16, 121), (S.TCA_F16, 128), (S.TCA_BF16, 333), (S.TCA_BF16, 520)])
+def test_wavefront_per_nonzero_and_batches(torch_cuda, dtype, n):
+    """The most nonzeros that take a wavefront each (16 pieces of 16 bytes a row
+    and more: 256 per piece) and one more, which go in batches."""
+    pieces = -(-n // (4 if dtype == S.TCA_F32 else 8))
+    for nnz in (256 * pieces, 256 * pieces + 1):
+        print(f"sddmm dtype={dtype} n={n} nnz={nnz}", flush=True)
+        rng = np.random.default_rng(nnz)
+        lens = [0, 1, 0, 3, 64, 0, 200] * 8
+        lens += [500] * ((nnz - sum(lens)) // 500)
+        lens += [nnz - sum(lens), 0]
+        got, want = _run(torch_cuda, dtype, lens, 700, n, rng, shift=n % 2)
+        assert len(want) == nnz and np.array_equal(got, want)
+
+
+def test_wavefront_per_nonzero_keeps_non_finite_rows_apart(torch_cuda):
+    """Its last piece overlaps the one before: an infinity there counts once."""
+    torch = torch_cuda
+    rng = np.random.default_rng(8)
+    rowptr, colidx = _pattern(rng, [20, 9, 33], 40)
+    a = S.CSR(3, 40, rowptr, colidx, np.ones(62, np.float32), S.TCA_F32)
+    g = torch.from_numpy(exact_dense(rng, (3, 1025)) + 2).to("cuda:0")
+    b = torch.from_numpy(exact_dense(rng, (40, 1025))).to("cuda:0")
+    b[7, 1023], b[8] = float("inf"), float("nan")
+    out = torch.empty(62, device="cuda:0")
+    with S.Plan(a, 1025) as plan:
+        S.call("tca_sddmm", plan._p, S._addr(g), S._addr(b), S._addr(out), None)
+        torch.cuda.synchronize()
+    rows = torch.from_numpy(np.repeat(np.arange(3), np.diff(rowptr))).to("cuda:0")
+    want = (g[rows].double() * b[torch.from_numpy(colidx).long().to("cuda:0")].double()).sum(1).float()
+    assert torch.equal(torch.isfinite(out), torch.isfinite(want))
+    assert torch.equal(torch.nan_to_num(out, 1.0, 2.0, 3.0), torch.nan_to_num(want, 1.0, 2.0, 3.0))
+
+
 PANEL_SHAPES = [(S.TCA_F32, 32), (S.TCA_F32, 64), (S.TCA_F32, 128), (S.TCA_F16, 64), (S.TCA_F16, 128), (S.TCA_BF16, 64),
                 (S.TCA_BF16, 128)]
 
