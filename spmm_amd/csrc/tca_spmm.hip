@@ -596,13 +596,23 @@ int launch_s24_t(S24Args a, hipStream_t s) {
 //   3145 x 5004 x 288    41.5 [985]   28.0 [495]  19.6 [250]  25.3 [125]
 //   5580 x 1872 x 184    24.1 [1047]  20.0 [525]  17.1 [264]  13.6 [132]
 //   4096 x 4096 x 512    62.6 [2048]  40.6 [1024] 28.9 [512]  22.1 [256]
+// More tallest tiles than CUs: as many wavefronts each, of four, as still let
+// two or four tiles share a CU, and for a K of few steps the next shorter tile
+// with one (6000 x 256 x 512 7.7 us, 6000 x 128 x 512 7.3).  us with one / two / four:
+//   6000 x 256 x 1024 [752]  13.5 / 16.9 / 19.9    6000 x 4000 x 1024 52 / 70 / 64
+//   6000 x 256 x 512 [376]   11.6 /  9.0 / 13.3    3000 x 512 x 1024 [384] 13.8 / 10.6 / 13.7
+//   4096 x 4096 x 512 [256]  45.7 / 28.0 / 21.1
 template <bool kBf16>
 int launch_s24(const S24Args& a, hipStream_t s) {
-    auto fits = [&](int rows) { return (static_cast<int64_t>(a.M) + rows - 1) / rows * a.col_groups <= 256; };
-    if (fits(16)) return launch_s24_t<kBf16, 1, 8>(a, s);
-    if (fits(32)) return launch_s24_t<kBf16, 2, 6>(a, s);
-    if (fits(64)) return launch_s24_t<kBf16, 4, 4>(a, s);
-    return launch_s24_t<kBf16, 8, 4>(a, s);
+    auto fits = [&](int rows, int tiles) {
+        return (static_cast<int64_t>(a.M) + rows - 1) / rows * a.col_groups <= tiles;
+    };
+    if (fits(16, 256)) return launch_s24_t<kBf16, 1, 8>(a, s);
+    if (fits(32, 256)) return launch_s24_t<kBf16, 2, 6>(a, s);
+    if (fits(64, 256)) return launch_s24_t<kBf16, 4, 4>(a, s);
+    if (fits(128, 256) && a.Kp > 128) return launch_s24_t<kBf16, 8, 4>(a, s);
+    if (fits(128, 512)) return a.Kp > 256 ? launch_s24_t<kBf16, 8, 2>(a, s) : launch_s24_t<kBf16, 4, 1>(a, s);
+    return launch_s24_t<kBf16, 8, 1>(a, s);
 }
 
 // Wavefronts per tile: enough to fill the chip and to shorten a tile's serial

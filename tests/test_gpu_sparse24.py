@@ -89,3 +89,17 @@ def test_spmm_24_index_words_at_any_halfword(torch_cuda, k, shift):
     torch.cuda.synchronize()
     want = oracle.csr_spmm(a.rowptr, a.colidx, a.values_f32(), S.from_storage(b, S.TCA_F16))
     assert np.array_equal(c.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("m,k,n", [(5901, 60, 512), (5901, 256, 504),           # one wavefront, 64 rows
+                                   (5901, 257, 512), (2950, 700, 1000),         # two, 128 rows
+                                   (5901, 250, 1016), (8321, 61, 520), (4200, 900, 1024),  # one, 128 rows
+                                   (4096, 129, 512), (4097, 193, 512)])         # tallest tiles on 256 CUs, one more
+def test_spmm_24_more_tiles_than_cus(torch_cuda, m, k, n):
+    rng = np.random.default_rng(m + k)
+    a = _pruned(rng, m, k, 0.4, S.TCA_BF16 if k % 2 else S.TCA_F16)
+    b = S.to_storage(exact_dense(rng, (k, n)), a.dtype)
+    print(f"2:4 {m} x {k} x {n}", flush=True)
+    got = _run(torch_cuda, a, b)
+    want = oracle.csr_spmm(a.rowptr, a.colidx, a.values_f32(), S.from_storage(b, a.dtype))
+    assert np.array_equal(got, want)
