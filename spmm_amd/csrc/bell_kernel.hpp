@@ -121,7 +121,7 @@ __global__ __launch_bounds__(64 * W) void bell_mfma_kernel(BellArgs a) {
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
 #pragma unroll
-            for (int c = 0; c < 4; c++) 
+            for (int c = 0; c < 4; c++)
                 bq[ks][c] = b_fragment(reinterpret_cast<const uint16_t*>(mem + 4096 * ks), c, lane);
 #pragma unroll
             for (int rf = 0; rf < RF; rf++)

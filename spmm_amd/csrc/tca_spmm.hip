@@ -623,10 +623,15 @@ int launch_s24(const S24Args& a, hipStream_t s) {
 //   5580 x 1872 x 184, 64, 264                   10.8    7.5    7.5    8.3
 //   2000 x 600 x 1000, 32, 1008                   8.7    7.5    8.1   11.9
 //   4096 x 4096 x 512, 32, 1024                  20.2   15.1   17.0   20.0
+//   6000 x 6000 x 1024, half the blocks, 32, 3008 94.7  113.2  113.5
+//   6000 x 6000 x 512, half, 32, 1504            63.2   49.8   46.6
+//   6000 x 256 x 1024, half, 32, 3008            11.5   10.2   10.2
 template <bool kBf16, int BS>
 void launch_bell_w(const BellArgs& a, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(a.row_groups * a.col_groups));
-    if (grid.x > 512) hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 2>), grid, dim3(128), 0, s, a);
+    if (grid.x > 2048 && a.ell_blocks > 1024 / BS)
+        hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 1>), grid, dim3(64), 0, s, a);
+    else if (grid.x > 512) hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 2>), grid, dim3(128), 0, s, a);
     else if (grid.x > 256) hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 4>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((bell_mfma_kernel<kBf16, BS, 8>), grid, dim3(512), 0, s, a);
 }

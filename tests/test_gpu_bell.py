@@ -115,3 +115,9 @@ def test_bell_list_lengths(torch_cuda, bs, n, brows):
     torch.cuda.synchronize()
     want = (dense[:m] @ b.astype(np.float64)).astype(np.float32)
     assert np.array_equal(c.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("bs,n,brows", [(32, 1000, 130), (64, 520, 230), (32, 1000, 128)])
+def test_bell_one_wavefront_per_tile(torch_cuda, bs, n, brows):
+    """The same over more than 2048 workgroups (and just 2048) with long lists."""
+    test_bell_list_lengths(torch_cuda, bs, n, brows)
