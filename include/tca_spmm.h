@@ -67,7 +67,8 @@ typedef enum tca_status {
  * rows of at least 256 bytes and at least 2^21 nonzeros in panels. */
 #define TCA_PLAN_NO_PANELS 256u    /* no panels: rows outside MFMA windows go to the row kernel */
 #define TCA_PLAN_FORCE_PANELS 512u /* every eligible row in panels, whatever their reuse */
-#define TCA_PLAN_NO_SCRATCH 1024u  /* the plan keeps no partial-row scratch: run it with tca_spmm_run_static */
+/* The plan keeps no partial-row scratch and no copy of B: run it with tca_spmm_run_static. */
+#define TCA_PLAN_NO_SCRATCH 1024u
 /* Short-K matrix-core kernel (TCA_TILES_SHORT): fp16 / bf16, N % 8 == 0 and
  * K <= 640: every row, in windows of 64 rows x 64 columns built in LDS from
  * the CSR each run (no plan-time tiles, no pack kernel, one launch).  The
@@ -108,7 +109,8 @@ typedef struct tca_plan_info {
     int32_t mfma_blockdim;
     int32_t mfma_lds_bytes;   /* LDS per MFMA workgroup */
     int32_t seg_len;          /* nonzeros per long-row segment */
-    int64_t scratch_bytes;    /* device scratch owned by the plan */
+    int64_t scratch_bytes;    /* partial rows of split rows: the plan's own, or the static array's with
+                                 TCA_PLAN_NO_SCRATCH (the copy of B: b_copy_bytes) */
     double plan_ms;           /* host planning time */
     int32_t n_wide_tasks;     /* row-kernel tasks that are quarters of workgroup-shared rows */
     int32_t chunk_lanes;      /* lanes holding data in one column chunk */
@@ -128,6 +130,8 @@ typedef struct tca_plan_info {
                                    stream of the plan beside the panel kernel (forked and joined
                                    by events on the run's stream; TCA_ROWS_BESIDE=0 turns it off;
                                    0 also when the runtime could not create that stream) */
+    int64_t b_copy_bytes;     /* device memory the plan keeps for a copy of B at an aligned pitch (at most
+                                 256 MiB, rewritten by every run); 0: B is read in place */
 } tca_plan_info;
 
 /* tca_plan_info.tile_kernel */

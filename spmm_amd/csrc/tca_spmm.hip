@@ -769,6 +769,7 @@ void fill_info(tca_spmm_plan* p) {
     else if (p->mfma_pair)
         in.mfma_lds_bytes = mfma_pair_lds_bytes();
     in.scratch_bytes = static_cast<int64_t>(p->n_seg_total * p->N * sizeof(float));
+    in.b_copy_bytes = static_cast<int64_t>(p->K) * p->b_pitch * static_cast<int64_t>(dtype_size(p->dtype));
     in.n_panels = p->panels.n_panels;
     in.n_panel_units = p->n_units;
     in.rows_panels = p->panels.n_rows;

@@ -92,3 +92,22 @@ def test_graph_replays(torch_cuda, monkeypatch):
             plan.run(val, b, e)
             torch.cuda.synchronize()
             assert torch.equal(c, e)
+
+
+def test_copy_is_reported(torch_cuda, monkeypatch):
+    """b_copy_bytes: rows at the copy's pitch (whole vectors, whole lines where
+    that adds little), none for plans that read B in place or keep no scratch;
+    every plan of a matrix reports its own."""
+    rng = np.random.default_rng(6)
+    a = _matrix(rng, LENS, 4200, S.TCA_F16)
+
+    def copied(n, flags=FLAGS):
+        with S.Plan(a, n, flags) as plan:
+            assert ("pack" in plan.phases()) == (plan.info()["b_copy_bytes"] > 0)
+            return plan.info()["b_copy_bytes"]
+
+    monkeypatch.setenv("TCA_PAD", "1")
+    assert copied(47) == 4200 * 48 * 2 and copied(127) == 4200 * 128 * 2 and copied(48) == 0
+    assert copied(47, FLAGS | S.TCA_PLAN_NO_SCRATCH) == 0
+    monkeypatch.setenv("TCA_PAD", "0")
+    assert copied(47) == 0
