@@ -180,7 +180,7 @@ def test_panels_and_other_rows(torch_cuda, monkeypatch, dtype, n):
     assert np.array_equal(got, want)
 
 
-@pytest.mark.parametrize("dtype,n", [(S.TCA_F32, 32), (S.TCA_F32, 128), (S.TCA_F16, 64)])
+@pytest.mark.parametrize("dtype,n", [(S.TCA_F32, 64), (S.TCA_F32, 128), (S.TCA_F16, 128), (S.TCA_BF16, 128)])
 def test_every_task_beside_panels(torch_cuda, monkeypatch, dtype, n):
     """Panels keep a band of like rows; short rows in groups, medium rows, quarters
     and segments of long rows are left to the row kernel's list."""
@@ -209,8 +209,7 @@ def test_every_task_beside_panels(torch_cuda, monkeypatch, dtype, n):
     print(f"tasks beside panels dtype={dtype} n={n}: {info['rows_panels']} of {len(lens)} rows in panels", flush=True)
     rows = np.repeat(np.arange(len(lens)), lens)
     want = (g[rows].astype(np.float64) * b[colidx]).sum(1).astype(np.float32)
-    if n == 128:  # (narrower B rows go to panels only when asked)
-        assert 0 < info["rows_panels"] < len(lens) and info["n_long_rows"] > 0 and info["n_wide_tasks"] > 0
+    assert 0 < info["rows_panels"] < len(lens) and info["n_long_rows"] > 0 and info["n_wide_tasks"] > 0
     assert np.array_equal(out.cpu().numpy(), want)
 
 
