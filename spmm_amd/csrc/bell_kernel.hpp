@@ -11,13 +11,15 @@
 // unit as soon as it has read the last one into registers, and multiplies
 // that meanwhile.  A unit is 64 columns of A (one block of 64 or two of 32),
 // so every line of the row-major ELL values is used whole: lines from the L2
-// to the CU, about 4 cycles each, bound the kernel (A 2 BS / 32 KiB, B 8 KiB a
-// unit), and with one block of 32 at a time half of A's would be wasted.
+// to the CU bound the kernel (A 2 BS / 32 KiB, B 8 KiB a unit; 1.78M of them on
+// the product below, one per 3.7 cycles and CU, the L1s active in 3.5 of these),
+// and with one block of 32 at a time half of A's would be wasted.
 //
-// 4096 x 4096 fp16 with a quarter of its 32 x 32 blocks at N = 512: 15.1 us
-// (31.5 with a workgroup per block row and 256 columns, B staged one block
+// 4096 x 4096 fp16 with a quarter of its 32 x 32 blocks at N = 512: 15.6 us
+// (31.9 with a workgroup per block row and 256 columns, B staged one block
 // ahead through registers with a barrier per block).  128 columns per
-// wavefront: 14.5 us there, but up to twice as long on small outputs.
+// wavefront take 14.6 there with four wavefronts, but up to twice as long on
+// small outputs.
 //
 // Sums run in list order within a wavefront's range, the ranges in order.  The
 // missing half of an odd list's last unit, B rows past K and columns past N

@@ -280,7 +280,8 @@ __global__ __launch_bounds__(kPnThreads, 1) void panel_kernel(PanelArgs a) {
     const int4 u = a.units[unit];
 
     if (wave >= kPnWaves) {
-        // ---- producers: tile t + 1 into buffer (t + 1) & 1 while tile t is used;
+        // ---- producers (pn_produce below is the same text for the sampled product;
+        // so is pn_read_counts): tile t + 1 into buffer (t + 1) & 1 while tile t is used;
         // producer pid issues transfers pid, pid + kPnProducers, ... of a tile (and
         // producer 0 the counts), so each has at most kInstrs / kPnProducers + 1
         // transfers in flight (a wavefront's vmcnt counts 63 at most)

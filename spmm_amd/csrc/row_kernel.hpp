@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const T* __restrict__ B, 
     const uint32_t V = static_cast<uint32_t>(N + E - 1) / E;  // vectors of a row
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (i >= static_cast<uint64_t>(K) * V) return;
-    const uint32_t r = static_cast<uint32_t>(i) / V;  // (at most 2^28 vectors)
+    const uint32_t r = static_cast<uint32_t>(i) / V;  // (at most 2^24 vectors: kMallBytes)
     const int col = static_cast<int>(static_cast<uint32_t>(i) - r * V) * E;
     const T* const src = B + static_cast<size_t>(r) * N + col;
     Pack<T, E> v{};

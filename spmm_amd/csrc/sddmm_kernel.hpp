@@ -84,8 +84,8 @@ __device__ __forceinline__ int wave_row_of(const int* __restrict__ rowptr, uint3
 // One wavefront per row with one nonzero at a time and a six-step shuffle sum
 // per nonzero (the previous kernel): 25.2 ms on 11.4M nonzeros of an R-MAT
 // graph of 131,072 nodes at N = 128 fp32, 650 us on a 2048 x 2048 layer of
-// 10 % at N = 1024 bf16; now 0.60 ms and 63 us (9.7 and 13.6 TB/s of gathered
-// rows of B).  Rows in panels take panel_sddmm_kernel (panel_kernel.hpp), and
+// 10 % at N = 1024 bf16; gathered this way 0.60 ms and 63 us (9.7 and 13.6 TB/s of
+// rows of B).  Few nonzeros take sddmm_wide_kernel (below).  Rows in panels take panel_sddmm_kernel (panel_kernel.hpp), and
 // the others beside them sddmm_tasks_kernel (the spans above, skipping the
 // panels' nonzeros, took 97 us for them: nearly every span holds a few).
 
@@ -151,7 +151,8 @@ __device__ __forceinline__ float sddmm_batch(const SddmmArgs& a, int row, int co
     const int tail = full + l;  // the last piece of a row that is no whole number of them ends at the row's end
     const int at = min(tail * E, a.N - E);
     if (one_row) {
-#pragma unroll(E == 8 ? 1 : 2)
+        constexpr int kAhead = E == 8 ? 1 : 2;
+#pragma unroll kAhead
         for (int p = 0; p < full; p += L) piece((p + l) * E, 0);
         if (tail < V) piece(at, tail * E - at);
     } else {

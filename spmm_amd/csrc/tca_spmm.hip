@@ -588,8 +588,8 @@ int launch_s24_t(S24Args a, hipStream_t s) {
 // The tallest tile costs the fewest bytes per output (its B tile serves the
 // most rows) but leaves the chip idle on small outputs: the shortest tile
 // whose workgroups fit the 256 CUs in one round (a workgroup's LDS takes a
-// CU), the tallest when none does.  us per product, bf16, M x K x N
-// (workgroups of the tile in brackets):
+// CU), the tallest when none does.  us per product (wall clock over 50 calls,
+// with their host time), bf16, M x K x N (workgroups of the tile in brackets):
 //                        16 rows     32 rows     64 rows     128 rows
 //   287 x 5057 x 16       9.6 [18]    12.2 [9]    17.2 [5]    23.5 [3]
 //   700 x 700 x 512       7.2 [352]    7.2 [176]   7.5 [88]    8.7 [48]
@@ -1819,7 +1819,8 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         auto sort_rows = [&](const uint8_t* in_panel) -> int {
             const int* const windows = p->mfma.windows.empty() ? nullptr : wmap;
             if (M <= kSmallSortRows) {
-                hipLaunchKernelGGL(dp_sort_small_kernel, dim3((M + kSmallSortRowsPerGroup - 1) / kSmallSortRowsPerGroup), dim3(1024), 0, s, p->d_rowptr, M, windows, in_panel,
+                const dim3 groups((M + kSmallSortRowsPerGroup - 1) / kSmallSortRowsPerGroup);
+                hipLaunchKernelGGL(dp_sort_small_kernel, groups, dim3(1024), 0, s, p->d_rowptr, M, windows, in_panel,
                                    p->rows.wide_len, p->rows.row_len, p->rows.multi_max, keys_s, rows_s, cnt, cnt + 6);
                 const int e = read_cnt();
                 if (e || !h_cnt[6]) return e;
@@ -2068,7 +2069,6 @@ int tca_spmm_plan_destroy(tca_spmm_plan* plan) {
     return TCA_OK;
 }
 
-// Operand checks of tca_spmm_run (p non-NULL, M > 0).
 // Bytes B must be aligned to: the plan's vector, for ragged rows (which read
 // vectors at any element) the widest that divides N.
 static size_t b_align(const tca_spmm_plan* p) {
@@ -2077,6 +2077,7 @@ static size_t b_align(const tca_spmm_plan* p) {
     return static_cast<size_t>(e) * dtype_size(p->dtype);
 }
 
+// Operand checks of tca_spmm_run (p non-NULL, M > 0).
 static int check_run_operands(const tca_spmm_plan* p, const void* d_val, const void* d_B, const float* d_C) {
     if ((p->nnz > 0 && (!d_val || !d_B)) || !d_C) return fail(TCA_ERR_INVALID, "NULL device pointer");
     const size_t vb = b_align(p);

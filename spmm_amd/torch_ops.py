@@ -21,7 +21,7 @@ a GCN / GraphSAGE aggregation (C = A * X with A the normalised adjacency)
 calls, forward and backward.
 
 A plan owns device scratch that every run rewrites (packed MFMA entries,
-partial rows of split rows), so one plan cannot serve two streams at once:
+partial rows of split rows, at some widths a copy of B), so one plan cannot serve two streams at once:
 running a SparseMatrix's plan on a stream while its previous run on another
 stream has not completed raises RuntimeError instead of racing.
 
