@@ -129,7 +129,7 @@ void plan_row_params(int32_t M, int32_t K, int64_t nnz, int32_t N, int32_t es, u
 }
 
 void plan_rows(const int32_t* rowptr, int32_t M, int32_t K, int32_t N, int32_t es, uint32_t flags,
-               const std::vector<uint8_t>& skip, int32_t slices, RowPlan* p) {
+               const std::vector<uint8_t>& skip, bool panels, int32_t slices, RowPlan* p) {
     int32_t longest = 0;
     if (short_rows_matter(M, K, rowptr[M], N, es))
         for (int32_t r = 0; r < M; r++) longest = std::max(longest, rowptr[r + 1] - rowptr[r]);
@@ -189,7 +189,7 @@ void plan_rows(const int32_t* rowptr, int32_t M, int32_t K, int32_t N, int32_t e
     size_t end_nz = i;
     while (end_nz < rows.size() && len(rows[end_nz]) > 0) end_nz++;
     const int32_t group =
-        multi_group_rows(slots, static_cast<int64_t>(end_nz - i), static_cast<int64_t>(first_multi));
+        multi_group_rows(slots, static_cast<int64_t>(end_nz - i), static_cast<int64_t>(first_multi), panels);
     for (size_t k = i; k < rows.size();) {
         const size_t lim = k < end_nz ? std::min<size_t>(k + group, end_nz)
                                       : std::min<size_t>(k + kZeroRows, rows.size());
@@ -755,7 +755,7 @@ extern "C" int tca_plan_row_tasks(const int32_t* rowptr, int32_t M, int32_t K, i
         if (!rowptr || M < 0 || K < 1 || N < 1 || !dtype_ok(dtype) || !n_tasks || !n_perm || !n_long)
             return fail(TCA_ERR_INVALID, "tca_plan_row_tasks: bad argument");
         RowPlan p;
-        plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), TCA_PLAN_DEFAULT, {},
+        plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), TCA_PLAN_DEFAULT, {}, false,
                   default_slices(K, N, dtype), &p);
         if (tasks) {
             if (*n_tasks < static_cast<int32_t>(p.tasks.size()) || *n_perm < static_cast<int32_t>(p.perm.size()) ||
@@ -827,8 +827,8 @@ extern "C" int tca_plan_launch_orders(const int32_t* rowptr, const int32_t* coli
         std::vector<uint8_t> skip(M, 0);
         for (int32_t r = 0; r < M; r++) skip[r] = (!mp.row_mfma.empty() && mp.row_mfma[r]) || pp.row_panel[r];
         RowPlan rp;
-        plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), flags, skip, default_slices(K, N, dtype),
-                  &rp);
+        plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), flags, skip, pp.n_panels > 0,
+                  default_slices(K, N, dtype), &rp);
         order_row_tasks(colidx, &rp);
         if (panel_order) {
             if (*n_blocks < static_cast<int32_t>(pp.order.size()) || *n_tasks < static_cast<int32_t>(rp.tasks.size()) ||

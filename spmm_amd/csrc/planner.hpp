@@ -46,13 +46,19 @@ constexpr int32_t kZeroRows = 64;
 // 52.1; 60,000 rows of 5, N = 32 8.6 / 9.3; of 1.5M and 17M, N = 20 346 / 339; of
 // 2.4M and 64M, N = 47 2101 / 2084; 2^20 rows, 20M nonzeros in 15,000 of them,
 // fp16 N = 64 (23,000 other tasks, 1600 of short rows) 171.0 / 169.2; 100,000
-// rows of the kind, N = 48 (4200 and 270) 17.6 / 24.2.
+// rows of the kind, N = 48 (4200 and 270) 17.6 / 24.2.  With four slots and two a
+// pass has less to do and enough is a quarter and a sixteenth: R-MAT of 63,000
+// nodes and 490,000 nonzeros, bf16 N = 25 (two) 23.2 / 20.8; 12,000 x 300 of 2 %,
+// fp32 N = 47 (four) 4.9 / 6.4.  Rows beside panels keep four: the sampled
+// product's kernel of their tasks wants full batches of 64 nonzeros (131,000
+// nodes, fp32 N = 128 18.5 / 15.0).
 constexpr int32_t kMultiPasses = 4;
 constexpr int64_t kMultiTasks = 16384;
-inline int32_t multi_group_rows(int32_t slots, int64_t n_short, int64_t n_other) {
+inline int32_t multi_group_rows(int32_t slots, int64_t n_short, int64_t n_other, bool beside_panels) {
     const int64_t tasks = n_short / slots;  // of one pass
     const bool hidden = n_other >= kMultiTasks && n_other >= 8 * tasks;
-    const int64_t passes = hidden ? kMultiPasses : std::clamp<int64_t>(tasks / kMultiTasks, 1, kMultiPasses);
+    const int64_t enough = slots < 8 ? kMultiTasks * slots * slots / 64 : kMultiTasks;
+    const int64_t passes = hidden || beside_panels ? kMultiPasses : std::clamp<int64_t>(tasks / enough, 1, kMultiPasses);
     return static_cast<int32_t>(std::min<int64_t>(64, slots * passes));
 }
 
@@ -371,7 +377,7 @@ void route_windows(const std::vector<WinStat>& st, int32_t M, int64_t nnz_total,
                    double min_density, const MfmaShape& shape, std::vector<uint8_t>* take);
 
 void plan_rows(const int32_t* rowptr, int32_t M, int32_t K, int32_t N, int32_t es, uint32_t flags,
-               const std::vector<uint8_t>& skip, int32_t slices, RowPlan* p);
+               const std::vector<uint8_t>& skip, bool panels, int32_t slices, RowPlan* p);
 
 // Sorted column union of every window of `win` rows and each nonzero's
 // position in it (the indexing exported by tca_condense_windows).

@@ -999,7 +999,7 @@ int tca_spmm_plan_create(const int32_t* rowptr, const int32_t* colidx, int32_t M
         for (int32_t r = 0; r < M && !p->mfma_short; r++)
             skip_rows[r] = (!p->mfma.row_mfma.empty() && p->mfma.row_mfma[r]) || p->panels.row_panel[r];
         plan_rows(rowptr, M, K, N, static_cast<int32_t>(dtype_size(dtype)), flags, skip_rows,
-                  default_slices(K, N, dtype), &p->rows);
+                  p->panels.n_panels > 0, default_slices(K, N, dtype), &p->rows);
         order_row_tasks(colidx, &p->rows);
         p->ntasks = static_cast<int32_t>(p->rows.tasks.size());
         const size_t n_seg_rows =
@@ -1888,7 +1888,7 @@ int tca_spmm_plan_create_device(const int32_t* d_rowptr, const int32_t* d_colidx
         }
         const int n_wide = end_wide - n_long, n_row = end_row - end_wide, n_short = Mp - end_row;
         const int group = multi_group_rows(64 >> p->rows.log_lanes, end_nz - end_row,
-                                           4ll * n_wide + seg_total + n_row);  // rows per multi task
+                                           4ll * n_wide + seg_total + n_row, dpp.n_take > 0);  // rows per multi task
         const int n_multi = (end_nz - end_row + group - 1) / group + (Mp - end_nz + kZeroRows - 1) / kZeroRows;
         p->ntasks = 4 * n_wide + seg_total + n_row + n_multi;
         p->rows.n_wide = 4 * n_wide;
